@@ -446,7 +446,8 @@ bool recognise_orbit(nqs_log_amp_fn_t fn, void* user, OrbitSource& o) {
 struct Workspace {
   DBuf spins, t_re, t_im, q_re, q_im, la, ar, e_re, e_im, O, Oi, colwork, u1, u2, vecs, T, diag,
       y, scal, cg, fail, ham, sublat, hostla, hostar, linv, T2, Sd, elw, fwd, xr, heun, bond_ham,
-      bond_sub, orb_rows, orb_lp, orb_ar, orb_O, orb_Oi, orb_w, orb_cfg, o32, x3part, x3max;
+      bond_sub, orb_rows, orb_lp, orb_ar, orb_O, orb_Oi, orb_w, orb_cfg, o32, x3part, x3max,
+      fr_t, fr_bits, fr_lanes, fr_work;
 };
 
 // FP32 arithmetic for amplitudes, local energies, moves and O (the FP32 and
@@ -1788,6 +1789,9 @@ struct StepTimer {
 };
 
 // CG solve of (A + eps I) x = F on the device; A applied through `apply`.
+// Eight iterations are queued at a time and the scalars of the eight before
+// are looked at meanwhile, so the queue never drains; iterations past the
+// end do nothing.
 template <typename Apply>
 int cg_device(long P, const double* F, double* x, int max_iters, double tol, Apply apply,
               int& iters, int& converged, int& breakdown, double& pAp_out, double& rs_ratio) {
@@ -1797,22 +1801,35 @@ int cg_device(long P, const double* F, double* x, int max_iters, double tol, App
   double* r = base + 2 * P;
   double* p = base + 3 * P;
   double* Ap = base + 4 * P;
+  static nqs::CGScalars* seen = nullptr;   // pinned: two snapshots
+  static hipEvent_t ev[2] = {};
+  if (!seen) CK(hipHostMalloc((void**)&seen, 2 * sizeof(nqs::CGScalars), hipHostMallocDefault));
+  for (hipEvent_t& e : ev)
+    if (!e) CK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   CKR(nqs::launch_cg_init(F, P, x, r, p, sc, g_stream));
-  nqs::CGScalars h;
-  int it = 0;
-  for (; it < max_iters; it++) {
-    CKR(apply(p, Ap));
-    CKR(nqs::launch_cg_alpha(sc, p, Ap, P, g_stream));
-    CKR(nqs::launch_cg_update(sc, x, r, p, Ap, P, tol, g_stream));
-    CKR(nqs::launch_cg_direction(sc, p, r, P, g_stream));
-    if ((it & 7) == 7 || it + 1 == max_iters) {
-      CK(hipMemcpyAsync(&h, sc, sizeof(h), hipMemcpyDeviceToHost, g_stream));
-      CK(hipStreamSynchronize(g_stream));
-      if (h.done) break;
+  int groups = 0;
+  for (int it = 0; it < max_iters; it++) {
+    CKR(apply(p, Ap, &sc->done));
+    if (P <= nqs::kCgOneBlock) {
+      CKR(nqs::launch_cg_rest(sc, x, r, p, Ap, P, tol, g_stream));
+    } else {
+      CKR(nqs::launch_cg_alpha(sc, p, Ap, P, g_stream));
+      CKR(nqs::launch_cg_update(sc, x, r, p, Ap, P, tol, g_stream));
+      CKR(nqs::launch_cg_direction(sc, p, r, P, g_stream));
+    }
+    if ((it & 7) == 7) {
+      const int k = groups++ & 1;
+      CK(hipMemcpyAsync(seen + k, sc, sizeof(*sc), hipMemcpyDeviceToHost, g_stream));
+      CK(hipEventRecord(ev[k], g_stream));
+      if (groups > 1) {
+        CK(hipEventSynchronize(ev[k ^ 1]));
+        if (seen[k ^ 1].done) break;
+      }
     }
   }
-  CK(hipMemcpyAsync(&h, sc, sizeof(h), hipMemcpyDeviceToHost, g_stream));
+  CK(hipMemcpyAsync(seen, sc, sizeof(*sc), hipMemcpyDeviceToHost, g_stream));
   CK(hipStreamSynchronize(g_stream));
+  const nqs::CGScalars h = *seen;
   iters = h.iters;
   converged = h.converged;
   breakdown = h.breakdown;
@@ -1820,6 +1837,35 @@ int cg_device(long P, const double* F, double* x, int max_iters, double tol, App
   rs_ratio = h.rs0 > 0.0 ? sqrt(h.rs / h.rs0) : 0.0;
   if (max_iters <= 0) { iters = 0; converged = 0; breakdown = 0; }
   return 0;
+}
+
+// the factors of B samples for the products of k_frows.hip: t = tanh theta
+// as the forward pass left it in the workspace (single: in FP32)
+int frows_view(const nqs_ansatz* a, const int* d_samples, int B, int kind, bool single,
+               nqs::FactorRows& f) {
+  f.B = B;
+  f.N = a->N;
+  f.M = a->M;
+  f.kind = kind;
+  const size_t n = (size_t)B * f.M, np = (size_t)B * nqs::frows_hidden(f.M), planes = kind ? 2 : 1;
+  CKR(g_ws.fr_t.ensure(sizeof(double) * ((n + np) * planes + B)));
+  CKR(g_ws.fr_bits.ensure(sizeof(unsigned) * nqs::frows_bits_elems(B, f.N)));
+  CKR(g_ws.fr_lanes.ensure(sizeof(unsigned long long) * nqs::frows_lane_elems(B, f.N)));
+  CKR(g_ws.fr_work.ensure(sizeof(double) * nqs::frows_work_elems(f)));
+  f.tT = g_ws.fr_t.as<double>();
+  f.tp = f.tT + n;
+  f.ones = f.tp + np;
+  if (kind) {
+    f.tiT = f.ones + B;
+    f.tip = f.tiT + n;
+  }
+  f.bits = g_ws.fr_bits.as<unsigned>();
+  f.lanes = g_ws.fr_lanes.as<unsigned long long>();
+  f.work = g_ws.fr_work.as<double>();
+  return single ? nqs::launch_frows_prep(f, d_samples, nullptr, nullptr, g_ws.t_re.as<float>(),
+                                         g_ws.t_im.as<float>(), g_stream)
+                : nqs::launch_frows_prep(f, d_samples, g_ws.t_re.as<double>(),
+                                         g_ws.t_im.as<double>(), nullptr, nullptr, g_stream);
 }
 
 // MinSR solve (src/nqs/nqs_optimizer.c:1119-1177) on device data, shared by
@@ -2229,13 +2275,28 @@ int sr_step_impl(int method, const nqs_config_t* cfg, int Lx, int Ly, nqs_ansatz
   // sums, so O itself is never written (NQS_HIP_FACTORED_DUAL=0: through O)
   const bool fdual = method == SR_MINSR && dual && prec == NQS_HIP_MIXED && rbm_like && !holo &&
                      factored_dual_on(a);
+  // CG-SR with an RBM's own gradient takes its products with O from the
+  // factors (k_frows.hip: the bits that the stored rows give); gradient
+  // callbacks and mean-field go through O
+  const bool frows = method != SR_MINSR && rbm_like && !hfn && a->M >= 1;
+  nqs::FactorRows fr;
   // ---- 3. O matrix -----------------------------------------------------------
   const size_t ob = sizeof(double) * (size_t)B * (size_t)P;
-  if (!ofree && !fdual) CKR(g_ws.O.ensure(ob));
-  if (holo) CKR(g_ws.Oi.ensure(ob));
-  double* O = (ofree || fdual) ? nullptr : g_ws.O.as<double>();
-  double* Oi = holo ? g_ws.Oi.as<double>() : nullptr;
-  if (ofree) {
+  const bool noO = ofree || fdual || frows;
+  if (!noO) CKR(g_ws.O.ensure(ob));
+  if (holo && !noO) CKR(g_ws.Oi.ensure(ob));
+  double* O = noO ? nullptr : g_ws.O.as<double>();
+  double* Oi = holo && !noO ? g_ws.Oi.as<double>() : nullptr;
+  if (frows) {
+    const bool single = low_prec(prec);
+    if (single)
+      CKR(forward_t<float>(a, d_samples, B, nullptr, nullptr, false, prec == NQS_HIP_MIXED));
+    else
+      CKR(forward_t<double>(a, d_samples, B, nullptr, nullptr));
+    // a real RBM has no imaginary rows
+    CKR(frows_view(a, d_samples, B, a->kind == NQS_ANSATZ_RBM ? 0 : holo ? 2 : 1, single, fr));
+    fr.holo = holo;
+  } else if (ofree) {
     // t in FP64 for the factored Gram and update (the FP64 local energies of
     // this ansatz have just left it in the workspace)
     if (!(e_dev && esrc.a == a && prec == NQS_HIP_FP64))
@@ -2280,7 +2341,7 @@ int sr_step_impl(int method, const nqs_config_t* cfg, int Lx, int Ly, nqs_ansatz
   } else if (fdual) {
     const int nblk = a->kind == NQS_ANSATZ_COMPLEX_RBM ? 2 : 1;
     CKR(g_ws.colwork.ensure(sizeof(double) * nqs::factored_delta_work_elems(B, N, a->M, nblk)));
-  } else {
+  } else if (!frows) {
     CKR(g_ws.colwork.ensure(sizeof(double) * nqs::colsum_work_elems(B, P)));
   }
   CKR(g_ws.u1.ensure(sizeof(double) * B));
@@ -2303,9 +2364,23 @@ int sr_step_impl(int method, const nqs_config_t* cfg, int Lx, int Ly, nqs_ansatz
                                    a->kind == NQS_ANSATZ_COMPLEX_RBM ? g_ws.t_im.as<float>()
                                                                      : nullptr,
                                    nullptr, 1.0 / B, work, Om, g_stream));
-  else if (!ofree)
+  else if (!noO)
     CKR(nqs::launch_colsum(O, B, P, nullptr, 1.0 / B, Om, work, g_stream));
-  if (holo && tvmc) {
+  if (frows) {
+    // the same sums as below, R and I at once
+    CKR(nqs::launch_frows_colsum(fr, nullptr, nullptr, 1.0 / B, 1.0 / B, Om, Im, g_stream));
+    const double* mr = sc + (tvmc ? 2 : excited ? 10 : 0);
+    const double* mi = sc + (tvmc ? 12 : excited ? 11 : 2);
+    CKR(nqs::launch_frows_colsum(fr, tvmc ? Ei : E, tvmc ? E : Ei, 1.0 / B,
+                                 tvmc ? -1.0 / B : 1.0 / B, c1, c2, g_stream));
+    if (tvmc) CKR(nqs::launch_sum(E, B, nullptr, -1.0 / B, sc + 12, g_stream));
+    if (holo && fr.kind != 2) {
+      CKR(nqs::launch_fill(Im, 0.0, P, g_stream));
+      CKR(nqs::launch_fill(c2, 0.0, P, g_stream));
+    }
+    CKR(nqs::launch_qgt_finish(F, c1, Om, mr, holo ? c2 : nullptr, Im, mi, holo ? 2.0 : 1.0, 0.0, c1,
+                               P, g_stream));
+  } else if (holo && tvmc) {
     // F = 2[(R^T E_im - I^T E_re)/Ns - <R><E_im> + <I><E_re>]
     // (nqs_optimizer.c:797-810): second term and mean carry the minus sign
     CKR(nqs::launch_colsum(Oi, B, P, nullptr, 1.0 / B, Im, work, g_stream));
@@ -2351,7 +2426,10 @@ int sr_step_impl(int method, const nqs_config_t* cfg, int Lx, int Ly, nqs_ansatz
   } else {
     double* u1 = g_ws.u1.as<double>();
     double* u2 = g_ws.u2.as<double>();
-    auto apply = [&](const double* v, double* out) -> int {
+    auto apply = [&](const double* v, double* out, const int* done) -> int {
+      if (frows)
+        return nqs::launch_frows_qgt(fr, v, Om, Im, u1, u2, sc + 3, sc + 4, holo ? 2.0 : 1.0, eps,
+                                     out, done, g_stream);
       CKR(nqs::launch_rowdot(O, B, P, v, u1, g_stream));
       CKR(nqs::launch_sum(u1, B, nullptr, 1.0 / B, sc + 3, g_stream));
       CKR(nqs::launch_colsum(O, B, P, u1, 1.0 / B, c1, work, g_stream));

@@ -450,6 +450,41 @@ int launch_qgt_finish(double* out, const double* c1, const double* m1, const dou
                       const double* c2, const double* m2, const double* u2mean,
                       double scale, double eps, const double* v, long P, hipStream_t st);
 
+// ---- products with an RBM's O rows through its factors (k_frows.hip) -----------
+// u = O v and O^T w without O, with the bits that launch_rowdot and
+// launch_colsum give over the stored rows (kind: 0 real RBM, 1 complex RBM
+// real-projected, 2 holomorphic: R and I rows; holo: the step is holomorphic).
+struct FactorRows {
+  int B = 0, N = 0, M = 0, kind = 0, holo = 0;
+  double *tT = nullptr, *tiT = nullptr;     // [M][B] (ti: complex kinds)
+  double *tp = nullptr, *tip = nullptr;     // [B][frows_hidden(M)]
+  double* ones = nullptr;                   // [B]
+  unsigned* bits = nullptr;                 // frows_bits_elems(B, N)
+  unsigned long long* lanes = nullptr;      // frows_lane_elems(B, N)
+  double* work = nullptr;                   // frows_work_elems
+  int Bp = 0;                               // set by launch_frows_prep
+};
+int frows_hidden(int M);
+size_t frows_bits_elems(int B, int N);
+size_t frows_lane_elems(int B, int N);
+size_t frows_work_elems(const FactorRows& f);
+// signs and laid-out factors from t, ti [B][M], or from t32, ti32 in FP32
+int launch_frows_prep(FactorRows& f, const int* spins, const double* t, const double* ti,
+                      const float* t32, const float* ti32, hipStream_t st);
+// out1 = a1 R^T w1 and (kind 2) out2 = a2 I^T w2 (null weights: 1)
+int launch_frows_colsum(const FactorRows& f, const double* w1, const double* w2, double a1,
+                        double a2, double* out1, double* out2, hipStream_t st);
+// the QGT product as launch_qgt_finish ends it; m1 / m2 the column means, u1 /
+// u2 [B] and mean1 / mean2 scratch; nothing is done when *skip is nonzero
+int launch_frows_qgt(const FactorRows& f, const double* v, const double* m1, const double* m2,
+                     double* u1, double* u2, double* mean1, double* mean2, double scale, double eps,
+                     double* out, const int* skip, hipStream_t st);
+// a CG iteration after A p on one workgroup (the launch_cg_* sequence's
+// results) for P <= kCgOneBlock
+constexpr long kCgOneBlock = 16384;
+int launch_cg_rest(CGScalars* sc, double* x, double* r, double* p, const double* Ap, long P,
+                   double tol, hipStream_t st);
+
 // ---- batched independent CG-SR problems (k_multi.hip) -------------------------
 // One real-RBM problem of a batch.  Vectors over the parameters live in a
 // padded (M+1) x (N+1) row-major layout: W[h][i] at (h, i), b[h] at (h, N),
