@@ -197,10 +197,9 @@ def optimise(lib, w, st, budget):
 
 # kernel symbol (as rocprofv3 names it) behind each timing tag
 SYMBOL = {"gemm_potrf": "nqs::k_gemm_big<1>", "gemm_chain": "nqs::k_gemm_lat",
-          "multi_gemm_g": "nqs::(anonymous namespace)::k_mb_gemm_g",
-          "multi_gemm_z": "nqs::(anonymous namespace)::k_mb_gemm_z",
-          "multi_rows": "nqs::(anonymous namespace)::k_mb_rows",
-          "multi_vec": "nqs::(anonymous namespace)::k_mb_finish + k_mb_update + k_mb_dir",
+          "multi_gemm_g": "nqs::(anonymous namespace)::k_mb_phase",
+          "multi_gemm_z": "nqs::(anonymous namespace)::k_mb_phase",
+          "multi_vec": "nqs::(anonymous namespace)::k_mb_phase",
           "gemm": "nqs::k_gemm_big<0>",
           "potrf_panel": "nqs::k_panel2",
           "eloc": "nqs::k_eloc_terms<double, true>", "gen_O": "nqs::k_gen_O<double>",
@@ -222,7 +221,7 @@ def traffic_bytes(workload, tag):
 
 TAGS = ["mh", "ar_mh", "forward", "eloc", "gen_O", "colsum", "gemm", "gemm_small", "gram_x3",
         "gemm_potrf", "gemm_chain", "potrf_panel",
-        "trsv", "trsv_inv", "gram_f", "multi_prep", "multi_gemm_z", "multi_rows", "multi_gemm_g", "multi_vec"]
+        "trsv", "trsv_inv", "gram_f", "multi_prep", "multi_gemm_z", "multi_gemm_g", "multi_vec"]
 
 
 def potrf_widths():
@@ -323,8 +322,6 @@ def kernel_work(tag, w, st, launches, iters):
         return "mfma", 2.0 * (M + 1) * (N + 1) * B, "FLOP"
     if tag == "multi_vec":
         return "hbm", 13 * (M + 1) * (N + 1) * 8, "B"
-    if tag == "multi_rows":
-        return "hbm", 3 * (M + 1) * B * 8, "B"
     if tag == "gen_O":
         return "hbm", B * P * 8 + B * N * 4 + B * M * 8 * (2 if w["kind"] == 6 else 1), "B"
     if tag == "colsum":
@@ -434,7 +431,7 @@ def gpu_run(args, w, move=None, budget=0):
     return res
 
 
-MULTI_TAGS = ["mh", "forward", "eloc", "multi_prep", "multi_gemm_z", "multi_rows", "multi_gemm_g",
+MULTI_TAGS = ["mh", "forward", "eloc", "multi_prep", "multi_gemm_z", "multi_gemm_g",
               "multi_vec"]
 
 
@@ -461,33 +458,11 @@ def multi_gemm_flops(tag, inst, B, iters):
     return tot
 
 
-def multi_nsplit(N, B, target):
-    """Split factor of the batched G product (the rule of the library's
-    autotuned target: tiles x splits <= target, splits <= min(32, B/64))."""
-    M1, N1 = 2 * N + 1, N + 1
-    tiles = -(-M1 // 64) * -(-N1 // 64)
-    max_split = 1
-    while max_split * 2 <= 32 and max_split * 2 * 64 <= B:
-        max_split *= 2
-    ns = 1
-    while ns * 2 <= max_split and tiles * ns * 2 <= target:
-        ns *= 2
-    return ns
-
-
-def multi_bytes(tag, inst, B, target):
-    """Algorithmic HBM bytes of one launch of a batched vector tag over all
-    problems: multi_vec = finish (split partials, Om, p in; Ap out), update
-    (x, p, r, Ap in; x, r out) and direction (r, p in; p out) of one CG
-    iteration; multi_rows = [t, 1], Zt in, weighted [t, 1] out."""
-    tot = 0
-    for N, _ in inst:
-        M1, N1 = 2 * N + 1, N + 1
-        if tag == "multi_vec":
-            tot += (multi_nsplit(N, B, target) + 12) * M1 * N1 * 8
-        else:
-            tot += 3 * M1 * B * 8
-    return tot
+def multi_bytes(inst):
+    """Algorithmic HBM bytes of one CG iteration's vector work over all
+    problems (average of its three launches): A p (O^T u, p, Om, Ap), update
+    (x, p, r, Ap in; x, r out) and direction (r, p in; p out)."""
+    return sum(13 * (2 * N + 1) * (N + 1) * 8 for N, _ in inst) / 3
 
 
 def gpu_run_multi(args, w):
@@ -532,9 +507,9 @@ def gpu_run_multi(args, w):
     ntune = sum(1 for i in range(8) if us[i] > 0)
     log("[bench] autotune (G tiles x splits target: CG product us; 0 = persistent launch): " +
         ", ".join(f"{tg[i]}: {us[i]:.1f}" for i in range(ntune)) + f" -> {chosen}")
-    # one step launch by launch (CG as one launch per phase and iteration,
-    # the timed configuration) for the per-kernel split, then one with the
-    # CG in the persistent cooperative launch for comparison
+    # one step launch by launch (CG as one launch per phase and iteration)
+    # for the per-kernel split, then one with the CG in the cooperative
+    # launch, the timed configuration
     lib.nqs_hip_multi_use_graph(m, 0)
     lib.nqs_hip_multi_use_persistent(m, 0)
     lib.nqs_hip_kernel_timing(",".join(MULTI_TAGS).encode())
@@ -555,12 +530,11 @@ def gpu_run_multi(args, w):
         if lib.nqs_hip_kernel_stats(t.encode(), ctypes.byref(c), ctypes.byref(ms)) == 0 and c.value:
             per_p[t] = (c.value, ms.value)
     lib.nqs_hip_kernel_timing(None)
-    lib.nqs_hip_multi_use_persistent(m, 0)
     lib.nqs_hip_multi_use_graph(m, 1)
     iters_prof = iters_seq
     iters_per = [infos[i].cg_iterations for i in range(n)]
     seq_iter_us = 1e3 * sum(per.get(t, (0, 0.0))[1] for t in
-                            ("multi_gemm_z", "multi_rows", "multi_gemm_g", "multi_vec")) / max(iters_seq)
+                            ("multi_gemm_z", "multi_gemm_g", "multi_vec")) / max(iters_seq)
     cg_iter_us = 1e3 * per_p["multi_cg"][1] / max(iters_per) if "multi_cg" in per_p else None
     log(f"[bench] CG iteration of all problems: launch sequence {seq_iter_us:.1f} us (kernel time), "
         f"persistent launch {cg_iter_us if cg_iter_us is None else round(cg_iter_us, 1)} us")
@@ -608,8 +582,8 @@ def gpu_run_multi(args, w):
     if dom in ("multi_gemm_g", "multi_gemm_z"):
         work = multi_gemm_flops(dom, inst, B, iters_prof) / c
         achieved, peak, runit, bound = work / (avg_ms * 1e-3) / 1e12, PEAK_FP64 / 1e12, "TFLOP/s", "mfma"
-    elif dom in ("multi_vec", "multi_rows"):
-        work = multi_bytes(dom, inst, B, chosen)
+    elif dom == "multi_vec":
+        work = multi_bytes(inst)
         achieved, peak, runit, bound = work / (avg_ms * 1e-3) / 1e9, PEAK_HBM / 1e9, "GB/s", "hbm"
     else:
         # bytes the kernel must move: spins in, samples / energies out

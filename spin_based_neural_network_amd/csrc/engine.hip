@@ -4577,7 +4577,7 @@ struct nqs_hip_multi {
     nqs_sampler* s = nullptr;
     nqs_config_t cfg;
     nqs::HamDev H;
-    DBuf ham, sublat, t, E, S1, S1t, T1t, U, Gp, vec, part, ticket, sc, stats;
+    DBuf ham, sublat, t, tT, tA, E, bits, U, vec, part, ticket, sc, stats;
     int B = 0, rounds = 0, steps = 1, max_split = 1;
   };
   std::vector<Prob> p;
@@ -4620,8 +4620,8 @@ struct nqs_hip_multi {
       if (e) (void)hipEventDestroy(e);
     if (h_out) (void)hipHostFree(h_out);
     for (Prob& q : p) {
-      DBuf* all[] = {&q.ham, &q.sublat, &q.t, &q.E, &q.S1, &q.S1t, &q.T1t, &q.U,
-                     &q.Gp, &q.vec, &q.part, &q.ticket, &q.sc, &q.stats};
+      DBuf* all[] = {&q.ham, &q.sublat, &q.t, &q.tT, &q.tA, &q.E, &q.bits, &q.U,
+                     &q.vec, &q.part, &q.ticket, &q.sc, &q.stats};
       for (DBuf* b : all) b->release();
     }
     d_mp.release();
@@ -4642,7 +4642,7 @@ int multi_set_split(nqs_hip_multi* m, int target) {
     const int tiles = ((M1 + 63) / 64) * ((N1 + 63) / 64);
     int ns = 1;
     while (ns * 2 <= q.max_split && tiles * ns * 2 <= target) ns *= 2;
-    m->mp[i].nsplit = ns;
+    nqs::multi_shape(m->mp[i], ns);
   }
   nqs::multi_layout(m->mp.data(), (int)m->mp.size(), m->mb);
   // the host table is rewritten by the next call (the autotuner sets several
@@ -4758,7 +4758,7 @@ int multi_issue_back(nqs_hip_multi* m) {
     }
   }
   if (!m->persist)
-    for (int it = 0; it < m->max_iters; it++) CKR(nqs::launch_multi_cg_iter(m->mb, 0, g_stream));
+    for (int it = 0; it < m->max_iters; it++) CKR(nqs::launch_multi_cg_iter(m->mb, it, 0, g_stream));
   CKR(nqs::launch_multi_apply(m->mb, g_stream));
   CKR(nqs::launch_multi_gather(m->mb, m->d_out.as<double>(), g_stream));
   CK(hipMemcpyAsync(m->h_out, m->d_out.p, sizeof(double) * nqs::kMultiOut * m->p.size(),
@@ -4778,9 +4778,13 @@ int multi_issue_step(nqs_hip_multi* m) {
   return multi_issue_back(m);
 }
 
-// time the CG product (matvec and alpha, idempotent at the CG start) for
-// each target and keep the fastest
+// time the CG product (idempotent at the CG start) for each target, in the
+// launch shape that the step will use; the largest target (the most slots)
+// unless a smaller one is a quarter faster, so that the summation order does
+// not follow the timer's noise
 int multi_autotune(nqs_hip_multi* m) {
+  // the cooperative launch unless it was switched off or cannot hold the batch
+  if (!m->persist_set) m->persist = m->mb.nblk_cg > 0 ? 1 : 0;
   // NQS_HIP_MULTI_SPLIT=t: split target t without timing, so that the
   // summation order (and with it every result) does not depend on timing
   const char* fixed = getenv("NQS_HIP_MULTI_SPLIT");
@@ -4791,44 +4795,40 @@ int multi_autotune(nqs_hip_multi* m) {
   hipEvent_t e0, e1;
   CK(hipEventCreate(&e0));
   CK(hipEventCreate(&e1));
+  auto timed = [&](double& us) -> int {
+    auto once = [&]() -> int {
+      return m->persist ? nqs::launch_multi_cg_persist(m->mb, 1, g_stream, 1)
+                        : nqs::launch_multi_cg_iter(m->mb, 0, 1, g_stream);
+    };
+    CKR(once());   // warm
+    CK(hipEventRecord(e0, g_stream));
+    const int reps = 2;
+    for (int r = 0; r < reps; r++) CKR(once());
+    CK(hipEventRecord(e1, g_stream));
+    CK(hipEventSynchronize(e1));
+    float ms = 0.f;
+    CK(hipEventElapsedTime(&ms, e0, e1));
+    us = 1e3 * ms / reps;
+    return 0;
+  };
   const int targets[] = {8, 16, 32, 64, 128, 256};
-  double best = 1e300;
-  int best_t = 32;
   m->tuning.clear();
   for (int t : targets) {
     CKR(multi_set_split(m, t));
-    CKR(nqs::launch_multi_cg_iter(m->mb, 1, g_stream));   // warm
-    CK(hipEventRecord(e0, g_stream));
-    const int reps = 5;
-    for (int r = 0; r < reps; r++) CKR(nqs::launch_multi_cg_iter(m->mb, 1, g_stream));
-    CK(hipEventRecord(e1, g_stream));
-    CK(hipEventSynchronize(e1));
-    float ms = 0.f;
-    CK(hipEventElapsedTime(&ms, e0, e1));
-    const double us = 1e3 * ms / reps;
-    m->tuning.push_back({t, us});
-    if (us < best) {
-      best = us;
-      best_t = t;
+    double us = 0.0;
+    if (m->persist && timed(us)) {
+      fprintf(stderr, "nqs_hip_multi_step: the CG runs as a launch sequence\n");
+      m->persist = 0;
     }
+    if (!m->persist) CKR(timed(us));
+    m->tuning.push_back({t, us});
   }
-  CKR(multi_set_split(m, best_t));
-  // launch shape: the persistent cooperative launch against the launch
-  // sequence on the same product at the chosen split (bit-equal results, so
-  // the choice is timing only), unless the caller or NQS_HIP_MULTI_PERSIST
-  // chose; recorded in the tuning list as target 0
-  if (!m->persist_set && nqs::launch_multi_cg_persist(m->mb, 1, g_stream, 1) == 0) {
-    CK(hipEventRecord(e0, g_stream));
-    const int reps = 5;
-    for (int r = 0; r < reps; r++) CKR(nqs::launch_multi_cg_persist(m->mb, 1, g_stream, 1));
-    CK(hipEventRecord(e1, g_stream));
-    CK(hipEventSynchronize(e1));
-    float ms = 0.f;
-    CK(hipEventElapsedTime(&ms, e0, e1));
-    const double us = 1e3 * ms / 5;
-    m->tuning.push_back({0, us});
-    m->persist = us < best ? 1 : 0;
-  }
+  std::pair<int, double> best = m->tuning.back();
+  for (const std::pair<int, double>& c : m->tuning)
+    if (c.second < 0.8 * m->tuning.back().second && c.second < best.second) best = c;
+  CKR(multi_set_split(m, best.first));
+  // target 0: the cooperative launch at the chosen target
+  if (m->persist) m->tuning.push_back({0, best.second});
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   return 0;
@@ -4897,6 +4897,17 @@ int multi_step(nqs_hip_multi* m, nqs_sr_step_info_t* infos) {
   m->step_ms = hipEventElapsedTime(&tms, m->ev_t0, m->ev_t1) == hipSuccess ? tms : -1.0;
   multi_fill_info(m, infos);
   for (nqs_hip_multi::Prob& q : m->p) q.a->m64.valid = 0;
+  bool met = true;
+  for (size_t i = 0; i < m->p.size(); i++)
+    if (m->h_out[i * nqs::kMultiOut + 3] < 0.0) {
+      fprintf(stderr, "nqs_hip_multi_step: problem %zu: the workgroups of the cooperative CG launch "
+                      "did not meet\n", i);
+      met = false;
+    }
+  if (!met) {
+    for (nqs_hip_multi::Prob& q : m->p) CK(hipMemsetAsync(q.ticket.p, 0, 512, g_stream));
+    return -1;
+  }
   // weights beyond the ratio tables' range (flagged by the tables of this
   // step): the step's moves and energies are not trusted
   for (size_t i = 0; i < m->p.size(); i++)
@@ -4961,15 +4972,19 @@ nqs_hip_multi* multi_new(int n, const nqs_config_t* cfgs, const int* size_x, con
     if (ham_upload(hh, s->src, q.ham, q.sublat, q.H)) return fail(i, "device memory");
     q.max_split = 1;
     while (q.max_split * 2 <= 32 && q.max_split * 2 * 64 <= q.B) q.max_split *= 2;
+    nqs::MultiProb& mp = m->mp[i];
+    mp.B = q.B;
+    mp.N = N;
+    mp.M = M;
+    nqs::multi_shape(mp, 1);
     const size_t L = (size_t)M1 * N1, B = (size_t)q.B, d = sizeof(double);
-    if (q.t.ensure(d * 2 * B * M) || q.E.ensure(d * 2 * B) || q.S1.ensure(d * B * N1) ||
-        q.S1t.ensure(d * B * N1) || q.T1t.ensure(d * B * M1) || q.U.ensure(d * B * ((M1 + 63) / 64)) ||
-        q.Gp.ensure(d * 2 * q.max_split * L) ||
-        q.vec.ensure(d * 6 * L) || q.part.ensure(d * nqs::kMultiMaxPart) ||
-        q.ticket.ensure(64) || q.sc.ensure(sizeof(nqs::CGScalars)) || q.stats.ensure(d * 8) ||
+    if (q.t.ensure(d * 2 * B * M) || q.tT.ensure(d * B * M) || q.E.ensure(d * 2 * B) ||
+        q.bits.ensure(sizeof(unsigned) * B * nqs::multi_words(N)) || q.U.ensure(d * B) ||
+        q.tA.ensure(d * nqs::multi_ta_elems(q.B, M)) || q.vec.ensure(d * 6 * L) ||
+        q.part.ensure(d * 4 * nqs::kMultiMaxPart) || q.ticket.ensure(512) || q.sc.ensure(sizeof(nqs::CGScalars)) || q.stats.ensure(d * 8) ||
         s->d_samples.ensure(sizeof(int) * B * N))
       return fail(i, "device memory");
-    if (hipMemsetAsync(q.ticket.p, 0, 64, g_stream) != hipSuccess ||
+    if (hipMemsetAsync(q.ticket.p, 0, 512, g_stream) != hipSuccess ||
         hipMemsetAsync(q.sc.p, 0, sizeof(nqs::CGScalars), g_stream) != hipSuccess)
       return fail(i, "device memory");
     a->dev_fresh = 0;
@@ -4977,12 +4992,7 @@ nqs_hip_multi* multi_new(int n, const nqs_config_t* cfgs, const int* size_x, con
     a->dev_fresh = 1;
     ModelView<double> mv0;
     if (ratio_view<double>(a, mv0)) return fail(i, "amplitude-ratio tables");
-    nqs::MultiProb& mp = m->mp[i];
     mp.range_flag = a->m64.range_flag;
-    mp.B = q.B;
-    mp.N = N;
-    mp.M = M;
-    mp.nsplit = 1;
     mp.max_it = q.cfg.sr_cg_max_iters;
     mp.C = C;
     mp.eps = q.cfg.sr_diag_shift;
@@ -4993,20 +5003,20 @@ nqs_hip_multi* multi_new(int n, const nqs_config_t* cfgs, const int* size_x, con
     mp.spins = s->d_samples.as<int>();
     mp.t = q.t.as<double>();
     mp.E = q.E.as<double>();
-    mp.S1 = q.S1.as<double>();
-    mp.S1t = q.S1t.as<double>();
-    mp.T1t = q.T1t.as<double>();
+    mp.bits = q.bits.as<unsigned>();
+    mp.tT = q.tT.as<double>();
     mp.u = q.U.as<double>();
-    mp.Gp = q.Gp.as<double>();
+    mp.tA = q.tA.as<double>();
     double* v = q.vec.as<double>();
     mp.x = v;
     mp.r = v + L;
     mp.p = v + 2 * L;
     mp.Ap = v + 3 * L;
     mp.Om = v + 4 * L;
-    mp.F = v + 5 * L;
+    mp.g = v + 5 * L;
     mp.part = q.part.as<double>();
-    mp.ticket = q.ticket.as<unsigned>();
+    mp.bar = q.ticket.as<unsigned>();       // two counters in lines of their own, then the ticket
+    mp.ticket = q.ticket.as<unsigned>() + 64;
     mp.sc = q.sc.as<nqs::CGScalars>();
     mp.stats = q.stats.as<double>();
     mp.norm2 = q.stats.as<double>() + 5;

@@ -6,40 +6,67 @@
 // (qgt_apply, :44-80) and cg_solve's stopping rules (:84-139), then
 // theta -= lr delta.
 //
-// MI355X layout: problems of different sizes share every launch; a block
-// finds its problem from the per-launch block offsets.  The O matrix is never
-// formed: in the padded (M+1) x (N+1) parameter layout an O row is
-// [t_b, 1] (x) [s_b, 1], so
+// The O matrix is never formed: in the padded (M+1) x (N+1) parameter layout
+// an O row is [t_b, 1] (x) [s_b, 1], so
 //   (O v)_b     = sum_h [t_b, 1]_h (V [s_b, 1]^T)_h       (Z = V S1^T, row weights u)
-//   (O^T w)_hi  = sum_b w_b [t_b, 1]_h [s_b, 1]_i         (GEMM (T1 w)^T S1)
+//   (O^T w)_hi  = sum_b w_b [t_b, 1]_h [s_b, 1]_i         (G = (T1 w)^T S1)
 // on FP64 MFMA, and the last entry of O^T w is sum_b w_b, the mean that the
-// QGT needs.  Per CG iteration: Z product and row weights u in one pass
-// (Z never leaves the registers), split-K G GEMM with its operand [t_b, 1]
-// scaled by u_b as it is staged, finish (A p, p.Ap, alpha), update (x, r,
-// r.r, beta), direction.
-// Scalar reductions over a problem's blocks use one arrival counter: every
-// block stores its partial, the block that arrives last sums the partials in
-// block order (deterministic) and resets the counter.
-#include <hip/hip_cooperative_groups.h>
-
+// QGT needs.  A spin operand is made in registers from its bit.
+//
+// A CG iteration of a problem is five phases, and the workgroups of the
+// problem meet after each:
+//   Z     u = O p, split over samples
+//   G     O^T u, split over tiles of 16 hidden units; in a workgroup the waves
+//         take slots of the samples (nsplit, in order) and sum them in LDS
+//   A p   and partial p.Ap, split over 256-element slices
+//   x, r  alpha; x, r, partial r.r
+//   p     beta or stop; p
+// k_mb_cg runs every iteration of every problem in one cooperative launch, a
+// workgroup per CU, each problem on workgroups of its own that meet at a
+// counter of its own.  What crosses workgroups (p, u, O^T u, partial sums)
+// goes through relaxed agent-scope atomics, past the L2s that the XCDs do not
+// share, so no cache is flushed at a meeting: 1.7 us for 8 or 32 workgroups,
+// 4.9 us for 256, where a kernel boundary costs about 7 us.  The vectors stay
+// in registers; a small problem (own) has them whole in every workgroup and
+// meets twice an iteration.  k_mb_phase runs one phase as a launch, with the
+// same functions: the same bits.
+//
+// Measured: 32 chains of 16 to 128 sites, 2048 samples each, 240 us an
+// iteration as five launches on 64 x 64 tiles, 110 here (35 us of MFMA time;
+// the rest mostly the latency of t, which 32 problems do not leave in the
+// L2s); one of 16 sites, 1024 samples: 38 us, now 20.
+//
+// Every sum has a fixed order that depends on the problem and nsplit alone:
+// row weights over hidden units by tiles of 64 rows, in each tile eight
+// chains of eight; G over a slot's samples in one fused chain; slots in order;
+// vector sums by 256 elements and then 256 strided partials.
 #include "nqs_kernels.h"
+
+#include <vector>
 
 namespace nqs {
 
 namespace {
 
 typedef double v4d __attribute__((ext_vector_type(4)));
-constexpr int MT = 64, MKS = 16;     // GEMM tile and K step
+constexpr int CT = 512;              // threads of the CG kernels
+constexpr int CW = CT / 64;
+constexpr int kZs = 512;             // samples of a workgroup in hand in Z
+constexpr int kZb = 128;             // samples of a workgroup of the launch of Z
+constexpr int kTiles = 4;            // most site tiles of a wave in G
+constexpr int kPairs = 4;            // pairs of slices of a workgroup in hand
 
-enum { F_PREP = 0, F_Z = 1, F_G = 3, F_G2 = 4, F_VEC = 5 };
+enum { F_PREP = 0, F_Z, F_G, F_VEC, F_APPLY, F_CG };
+enum { PH_G1 = 0, PH_GE, PH_F, PH_Z, PH_G, PH_AP, PH_XR, PH_P };
 
 template <int FIELD>
 __device__ inline int first_blk(const MultiProb& q) {
-  return FIELD == F_PREP ? q.blk_prep
-       : FIELD == F_Z    ? q.blk_z
-       : FIELD == F_G    ? q.blk_g
-       : FIELD == F_G2   ? q.blk_g2
-                         : q.blk_vec;
+  return FIELD == F_PREP    ? q.blk_prep
+       : FIELD == F_Z     ? q.blk_z
+       : FIELD == F_G     ? q.blk_g
+       : FIELD == F_VEC   ? q.blk_vec
+       : FIELD == F_APPLY ? q.blk_apply
+                          : q.blk_cg;
 }
 
 // problem owning block `blk` of a launch (largest q with first block <= blk)
@@ -54,88 +81,735 @@ __device__ inline int find_prob(const MultiBatch& mb, int blk) {
   return lo;
 }
 
-// acc = the 64 x 64 tile [row0.., col0..] of sum_{k0 <= k < k1} A[r][k] w_k
-// Bm[c][k] with w_k = sum_{t < nw} w[t ldw + k] added in t order (w null:
-// 1), 4 waves of 32 x 32, v_mfma_f64_16x16x4f64: lane l
-// supplies A[l%16][l/16] and B[l%16][l/16]; result element j of lane l is
-// D[l/16 + 4j][l%16] (wave rows wr = 32 (wave / 2), columns wc = 32 (wave % 2)).
-// A row times its weight is rounded once as it is staged.
-__device__ inline void tile_acc(int M, int N, int k0, int k1, const double* __restrict__ A,
-                                long lda, const double* __restrict__ w, int nw, long ldw,
-                                const double* __restrict__ Bm, long ldb, int row0, int col0,
-                                v4d (&acc)[2][2]) {
-  __shared__ double As[MT][MKS + 1];
-  __shared__ double Bs[MT][MKS + 1];
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
-  const int lr = lane & 15, lk = lane >> 4;
+// values that workgroups of one launch exchange
+__device__ inline double ld_x(const double* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline void st_x(double* p, double v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// a b rounded: not fused with a sum that it enters
+__device__ inline double mul_only(double a, double b) {
+  double r = a * b;
+  asm volatile("" : "+v"(r));
+  return r;
+}
+
+// +1.0, or -1.0 where bit 0 of m is set
+__device__ inline double spin_of(unsigned m) {
+  return __hiloint2double((int)(0x3FF00000u | (m << 31)), 0);
+}
+
+// LDS of a workgroup: sums (in hand: also the problem's own p), partials,
+// row weights of the samples in hand (finished, and of the tile of 64 rows in
+// hand), their spin words; then the rows of p with partial row weights (Z), or
+// the partial tiles and each wave's samples (G).
+struct Lds {
+  double *red, *part, *u, *cur, *v, *up, *tile, *wu;
+  unsigned *bits, *wbits;
+};
+__device__ __host__ inline size_t lds_head(int nw) {
+  return kPairs * CT + kMultiMaxPart + 2 * kZs + (size_t)kZs * nw / 2;
+}
+__device__ inline Lds carve(const MultiProb& q, double* base) {
+  Lds l;
+  l.red = base;
+  l.part = l.red + kPairs * CT;
+  l.u = l.part + kMultiMaxPart;
+  l.cur = l.u + kZs;
+  l.bits = (unsigned*)(l.cur + kZs);
+  l.v = base + lds_head(q.nw);
+  l.up = l.v + q.hct * 16 * q.si;
+  l.tile = l.v;
+  l.wu = l.tile + CW * kTiles * 256;
+  l.wbits = (unsigned*)(l.wu + CW * 64);
+  return l;
+}
+
+// index of this thread's wave, in a scalar register
+__device__ inline int wave_of() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
+
+// KE steps (four sites) of two tiles of Z; m: the sample's sites, from lane's on
+template <int KE>
+__device__ __forceinline__ void row_steps(const double* pa, const double* pb, unsigned m, v4d& z0,
+                                          v4d& z1) {
 #pragma unroll
-  for (int i = 0; i < 2; i++)
-#pragma unroll
-    for (int j = 0; j < 2; j++) acc[i][j] = (v4d){0.0, 0.0, 0.0, 0.0};
-  for (int kb = k0; kb < k1; kb += MKS) {
-    // a thread stages K index kb + tid % 16 in all four of its rows: its
-    // weight once per step
-    const int gk = kb + (tid & 15);
-    double wk = 1.0;
-    if (w && gk < k1) {
-      wk = w[gk];
-      for (int t = 1; t < nw; t++) wk += w[t * ldw + gk];
-    }
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-      const int e = tid + 256 * q;
-      const int r = e >> 4, kk = e & 15;
-      const int ga = row0 + r, gb = col0 + r;
-      double a = 0.0;
-      if (ga < M && gk < k1) {
-        a = A[(long)ga * lda + gk];
-        if (w) a *= wk;
-      }
-      As[r][kk] = a;
-      Bs[r][kk] = (gb < N && gk < k1) ? Bm[(long)gb * ldb + gk] : 0.0;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int kk = 0; kk < MKS; kk += 4) {
-      const double a0 = As[wr + lr][kk + lk];
-      const double a1 = As[wr + 16 + lr][kk + lk];
-      const double b0 = Bs[wc + lr][kk + lk];
-      const double b1 = Bs[wc + 16 + lr][kk + lk];
-      acc[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b0, acc[0][0], 0, 0, 0);
-      acc[0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b1, acc[0][1], 0, 0, 0);
-      acc[1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b0, acc[1][0], 0, 0, 0);
-      acc[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b1, acc[1][1], 0, 0, 0);
-    }
-    __syncthreads();
+  for (int j = 0; j < KE; j++) {
+    const double sp = spin_of(m >> (4 * j));
+    z0 = __builtin_amdgcn_mfma_f64_16x16x4f64(pa[4 * j], sp, z0, 0, 0, 0);
+    z1 = __builtin_amdgcn_mfma_f64_16x16x4f64(pb[4 * j], sp, z1, 0, 0, 0);
   }
 }
 
-// C[row0.., col0..] = the tile of tile_acc
-__device__ inline void tile_nt(int M, int N, int k0, int k1, const double* __restrict__ A,
-                               long lda, const double* __restrict__ w, int nw, long ldw,
-                               const double* __restrict__ Bm, long ldb, double* C, long ldc,
-                               int row0, int col0) {
-  v4d acc[2][2];
-  tile_acc(M, N, k0, k1, A, lda, w, nw, ldw, Bm, ldb, row0, col0, acc);
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
+// ---- Z: row weights u = O p of the samples of 16-sample tiles t0 .. t1 - 1 -----
+// own: p is l.red.  held: the samples' words are in l.bits from the call before.
+__device__ void cg_rows(const MultiProb& q, const Lds& l, int t0, int t1, bool own, bool held) {
+  const int tid = threadIdx.x, wave = wave_of(), lane = tid & 63;
   const int lr = lane & 15, lk = lane >> 4;
+  const int M = q.M, N1 = q.N + 1, M1 = M + 1, nw = q.nw, si = q.si;
+  const int HT = (M1 + 15) >> 4, KK = (N1 + 3) >> 2;
+  const unsigned magic = 0xFFFFFFFFu / (unsigned)N1 + 1;   // f / N1 for f < 2^17
+  const int end = t1 * 16 < q.B ? t1 * 16 : q.B;
+  for (int g0 = t0 * 16; g0 < end; g0 += kZs) {
+    const int ns = end - g0 < kZs ? end - g0 : kZs;
+    if (!held) {
+      __syncthreads();
+      for (int e = tid; e < ns * nw; e += CT) l.bits[e] = q.bits[(long)g0 * nw + e];
+    }
+    for (int c = 0; c < HT; c += q.hct) {
+      const int nh = HT - c < q.hct ? HT - c : q.hct, pairs = (nh + 1) >> 1;
+      __syncthreads();
+      if (q.hct < HT || g0 == t0 * 16) {
+        // rows past M and columns past N are zero
+        const int r1 = M1 - c * 16 < pairs * 32 ? M1 - c * 16 : pairs * 32;
+        for (int e = tid; e < r1 * (si - N1); e += CT) {
+          const int h = e / (si - N1);
+          l.v[h * si + N1 + e - h * (si - N1)] = 0.0;
+        }
+        for (int e = r1 * si + tid; e < pairs * 32 * si; e += CT) l.v[e] = 0.0;
+        const int f0 = c * 16 * N1, nf = r1 * N1;
+        for (int f = tid; f < nf; f += 16 * CT) {
+          double x[16];
 #pragma unroll
-  for (int i = 0; i < 2; i++)
+          for (int j = 0; j < 16; j++) {
+            const int g = f + j * CT < nf ? f + j * CT : nf - 1;
+            x[j] = own ? l.red[f0 + g] : ld_x(q.p + f0 + g);
+          }
 #pragma unroll
-    for (int j = 0; j < 2; j++)
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int gr = row0 + wr + 16 * i + lk + 4 * r;
-        const int gc = col0 + wc + 16 * j + lr;
-        if (gr < M && gc < N) C[(long)gr * ldc + gc] = acc[i][j][r];
+          for (int j = 0; j < 16; j++) {
+            const int g = f + j * CT;
+            if (g < nf) {
+              const int h = __umulhi((unsigned)g, magic);
+              l.v[h * si + g - h * N1] = x[j];
+            }
+          }
+        }
       }
+      for (int b0 = 0; b0 < ns; b0 += q.zb) {
+        const int nb = ns - b0 < q.zb ? ns - b0 : q.zb, nst = (nb + 15) >> 4;
+        // an item: 32 rows x 16 samples, two tiles of Z = V S1^T (rows hidden
+        // units), weighted by t in a chain of eight as they leave the
+        // accumulators; the next item's t is under way meanwhile
+        double t[8];
+        auto fetch = [&](int it) {
+          const int p = it / nst, s = (it - p * nst) * 16 + lr, sc = s < nb ? s : nb - 1;
+          const double* __restrict__ tT = q.tT + g0 + b0 + sc;
+          const int h0 = (c + 2 * p) * 16 + lk;
+#pragma unroll
+          for (int j = 0; j < 8; j++) {
+            const int h = h0 + 4 * j;
+            t[j] = tT[(long)(h < M ? h : M - 1) * q.B];
+          }
+        };
+        if (wave < nst * pairs) fetch(wave);
+        __syncthreads();
+        for (int it = wave; it < nst * pairs; it += CW) {
+          const int p = it / nst, s = (it - p * nst) * 16 + lr, sc = s < nb ? s : nb - 1;
+          const unsigned* bw = l.bits + (b0 + sc) * nw;
+          const int h0 = (c + 2 * p) * 16 + lk;
+          double w[8];
+#pragma unroll
+          for (int j = 0; j < 8; j++) w[j] = h0 + 4 * j < M ? t[j] : h0 + 4 * j == M ? 1.0 : 0.0;
+          if (it + CW < nst * pairs) fetch(it + CW);
+          const double* va = l.v + (2 * p * 16 + lr) * si + lk;
+          const double* vb = va + 16 * si;
+          v4d z0 = {0.0, 0.0, 0.0, 0.0}, z1 = z0;
+          for (int k8 = 0; k8 < KK >> 3; k8++)
+            row_steps<8>(va + k8 * 32, vb + k8 * 32, bw[k8] >> lk, z0, z1);
+          if (KK & 7) {
+            const double *pa = va + (KK >> 3) * 32, *pb = vb + (KK >> 3) * 32;
+            const unsigned m = bw[KK >> 3] >> lk;
+            switch (KK & 7) {
+              case 1: row_steps<1>(pa, pb, m, z0, z1); break;
+              case 2: row_steps<2>(pa, pb, m, z0, z1); break;
+              case 3: row_steps<3>(pa, pb, m, z0, z1); break;
+              case 4: row_steps<4>(pa, pb, m, z0, z1); break;
+              case 5: row_steps<5>(pa, pb, m, z0, z1); break;
+              case 6: row_steps<6>(pa, pb, m, z0, z1); break;
+              default: row_steps<7>(pa, pb, m, z0, z1);
+            }
+          }
+          double x = 0.0;
+#pragma unroll
+          for (int r = 0; r < 4; r++) x = fma(z0[r], w[r], x);
+#pragma unroll
+          for (int r = 0; r < 4; r++) x = fma(z1[r], w[4 + r], x);
+          l.up[(p * 4 + lk) * q.zb + s] = x;
+        }
+        __syncthreads();
+        // the eight chains of a tile of 64 rows (two pairs) in order, then the tiles
+        if (tid < nb) {
+          const int s = b0 + tid;
+          double cur = l.cur[s], u = l.u[s];
+          for (int p = 0; p < pairs; p++) {
+            const int g = c / 2 + p;
+            if (!(g & 1)) cur = 0.0;
+#pragma unroll
+            for (int k = 0; k < 4; k++) cur += l.up[(p * 4 + k) * q.zb + tid];
+            if ((g & 1) || 2 * g + 2 >= HT) u = g < 2 ? cur : u + cur;
+          }
+          l.cur[s] = cur;
+          l.u[s] = u;
+          if (c + nh >= HT) st_x(q.u + g0 + s, u);
+        }
+      }
+    }
+  }
 }
 
-// Block partial -> problem scalar.  Every thread passes its value; the
-// block that arrives last among `nblk` returns true with the sum of all
-// partials (block order) in `total`; the others return false.
+// ---- G: O^T w -------------------------------------------------------------------
+// 16 samples of a wave's chain, from the first of y, wu and wbits: NT site
+// tiles from tile tl on; y the t of the 16 hidden units as MFMA operands, the
+// samples' weights and words (those of tiles tl ..) in LDS
+template <int NT>
+__device__ __forceinline__ void chain16(const double* y, const double* wu, const unsigned* wbits, int tl,
+                                        v4d* acc) {
+  const int lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    const int s = 4 * j + lk;
+    const double a = y[j] * wu[s];
+    const unsigned n0 = wbits[s], n1 = NT > 1 ? wbits[64 + s] : 0u, n2 = NT > 3 ? wbits[128 + s] : 0u;
+    // tile tl + c sits in half (tl + c) & 1 of word (tl + c) / 2
+#pragma unroll
+    for (int c = 0; c < NT; c++) {
+      const int o = (tl & 1) + c;
+      const unsigned n = o < 2 ? n0 : o < 4 ? n1 : n2;
+      acc[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, spin_of(n >> ((o & 1) * 16 + lr)), acc[c], 0, 0, 0);
+    }
+  }
+}
+// 64 samples, or the `left` of them that there are (up to 15 past it have no
+// weight); x is refilled with the next samples' operands g0 .. of nA as it is used
+template <int NT>
+__device__ __forceinline__ void chain64(double* x, const double* wu, const unsigned* wbits, int tl,
+                                        int left, v4d* acc, const double* __restrict__ nA, int g0,
+                                        int B4) {
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    if (left > 16 * j) chain16<NT>(x + 4 * j, wu + 16 * j, wbits + 16 * j, tl, acc);
+#pragma unroll
+    for (int i = 4 * j; i < 4 * j + 4; i++) x[i] = nA[(long)(g0 + i < B4 ? g0 + i : B4 - 1) * 64];
+  }
+}
+
+// Units u0, u0 + us, .. of O^T w into out.  A unit: 16 hidden units by q.nt
+// site tiles for each of CW / ws groups of waves, the waves of a group on ws
+// slots at a time.  A lane fetches its sample's weight and words for the wave;
+// the next 64 samples (slot, unit) are under way while these are used.
+__device__ void cg_tiles(const MultiProb& q, const Lds& l, int u0, int us, int units, int mode,
+                         double* out) {
+  const int tid = threadIdx.x, wave = wave_of(), lane = tid & 63;
+  const int N1 = q.N + 1, M1 = q.M + 1, sts = (N1 + 15) >> 4, nw = q.nw;
+  const int ws = q.nsplit < CW ? q.nsplit : CW, tg = CW / ws;
+  const int ng = (sts + q.nt * tg - 1) / (q.nt * tg);
+  const int sl = wave % ws, grp = wave / ws, B4 = (q.B + 15) / 16 * 4;
+  double* wu = l.wu + wave * 64;
+  unsigned* wbits = l.wbits + wave * 192;
+  const int ne = q.nt * tg * 256;   // elements of a unit, at most kTiles * CT
+  double x[16], u = 0.0;
+  unsigned m0 = 0, m1 = 0, m2 = 0;
+  auto first_tile = [&](int unit) { return (unit % ng * tg + grp) * q.nt; };
+  auto operands = [&](int unit) { return q.tA + (long)(unit / ng) * B4 * 64 + lane; };
+  auto fetch = [&](int unit, int k0, int sub) {
+    const int b0 = (k0 + sl) * q.chunk + sub, end = (k0 + sl + 1) * q.chunk;
+    const int b1 = end < q.B ? end : q.B;
+    const int s = b0 + lane, sc = s < q.B ? s : q.B - 1;
+    const double w = mode == PH_G1 ? 1.0 : mode == PH_GE ? q.E[sc] : ld_x(q.u + sc);
+    u = s < b1 ? w : 0.0;
+    const int w0 = first_tile(unit) >> 1;
+    const unsigned* bw = q.bits + (long)sc * nw;
+    m0 = bw[w0 < nw ? w0 : nw - 1];
+    m1 = q.nt > 1 ? bw[w0 + 1 < nw ? w0 + 1 : nw - 1] : 0u;
+    m2 = q.nt > 3 ? bw[w0 + 2 < nw ? w0 + 2 : nw - 1] : 0u;
+  };
+  if (u0 >= units) return;
+  fetch(u0, 0, 0);
+  {
+    const double* __restrict__ tA = operands(u0);
+    const int g0 = sl * q.chunk / 4;
+#pragma unroll
+    for (int j = 0; j < 16; j++) x[j] = tA[(long)(g0 + j < B4 ? g0 + j : B4 - 1) * 64];
+  }
+  for (int unit = u0; unit < units; unit += us) {
+    const int tl = first_tile(unit), nt = sts - tl < q.nt ? sts - tl : q.nt;
+    double sum[kTiles] = {0.0, 0.0, 0.0, 0.0};
+    for (int k0 = 0; k0 < q.nsplit; k0 += ws) {
+      v4d acc[kTiles];
+#pragma unroll
+      for (int c = 0; c < kTiles; c++) acc[c] = (v4d){0.0, 0.0, 0.0, 0.0};
+      for (int sub = 0; sub < q.chunk; sub += 64) {
+        wu[lane] = u;
+        wbits[lane] = m0;
+        wbits[64 + lane] = m1;
+        wbits[128 + lane] = m2;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        const int s0 = (k0 + sl) * q.chunk + sub;
+        const int left = q.chunk - sub < q.B - s0 ? q.chunk - sub : q.B - s0;
+        // the next samples of this slot, of the next slots, of the next unit
+        int nu = unit, nk = k0, nsub = sub + 64;
+        if (nsub >= q.chunk) {
+          nsub = 0;
+          nk += ws;
+          if (nk >= q.nsplit) {
+            nk = 0;
+            nu = unit + us < units ? unit + us : unit;
+          }
+        }
+        fetch(nu, nk, nsub);
+        const double* __restrict__ nA = operands(nu);
+        const int g0 = ((nk + sl) * q.chunk + nsub) / 4;
+        if (nt >= 4) chain64<4>(x, wu, wbits, tl, left, acc, nA, g0, B4);
+        else if (nt == 3) chain64<3>(x, wu, wbits, tl, left, acc, nA, g0, B4);
+        else if (nt == 2) chain64<2>(x, wu, wbits, tl, left, acc, nA, g0, B4);
+        else if (nt == 1) chain64<1>(x, wu, wbits, tl, left, acc, nA, g0, B4);
+        else chain64<0>(x, wu, wbits, tl, left, acc, nA, g0, B4);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+      }
+      __syncthreads();
+#pragma unroll
+      for (int c = 0; c < kTiles; c++)
+        if (c < q.nt) {
+          double* d = l.tile + ((grp * q.nt + c) * ws + sl) * 256 + lane;
+#pragma unroll
+          for (int r = 0; r < 4; r++) d[r * 64] = acc[c][r];
+        }
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < kTiles; i++) {
+        const int e = i * CT + tid;
+        if (e < ne) {
+          const double* d = l.tile + (e >> 8) * ws * 256 + (e & 255);
+          if (ws == CW) {
+            double v[CW];
+#pragma unroll
+            for (int k = 0; k < CW; k++) v[k] = d[k * 256];
+#pragma unroll
+            for (int k = 0; k < CW; k++) sum[i] += v[k];
+          } else {
+            for (int k = 0; k < ws; k++) sum[i] += d[k * 256];
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < kTiles; i++) {
+      const int e = i * CT + tid;
+      if (e < ne) {
+        const int site = (unit % ng * q.nt * tg + (e >> 8)) * 16 + (e & 15);
+        const int h = unit / ng * 16 + ((e & 255) >> 4);
+        if (site < N1 && h < M1) st_x(out + (long)h * N1 + site, sum[i]);
+      }
+    }
+  }
+}
+__device__ __host__ inline int tile_units(const MultiProb& q, int nt) {
+  const int HT = (q.M + 16) >> 4, sts = (q.N + 16) >> 4;
+  const int per = nt * (CW / (q.nsplit < CW ? q.nsplit : CW));
+  return HT * ((sts + per - 1) / per);
+}
+
+// ---- the vectors -----------------------------------------------------------------
+// Elements by 256-element slices, two (a pair) to a workgroup's 512 threads;
+// kPairs pairs j0, j0 + js, .. are in hand at a time.
+struct Elem {
+  double x, r, p, ap, om;
+};
+struct Pairs {
+  int j0, js;
+  __device__ int pair(int i) const { return j0 + i * js; }
+  __device__ long at(int i) const { return (long)pair(i) * CT + threadIdx.x; }
+};
+__device__ inline long vec_len(const MultiProb& q) { return (long)(q.M + 1) * (q.N + 1); }
+
+// Partial sums of v over the slices in hand, each by halves (128 apart, 64,
+// .. 1), into part (shared: exchanged)
+__device__ inline void put_parts(const MultiProb& q, const Pairs& w, const double* v, double* part,
+                                 bool shared, double* red) {
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kPairs; i++) red[i * CT + tid] = v[i];
+  __syncthreads();
+  const double* d = red + wave * 256 + lane;
+  double s = (d[0] + d[128]) + (d[64] + d[192]);
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) s += __shfl_xor(s, m, 64);
+  const int sl = 2 * w.pair(wave >> 1) + (wave & 1);
+  if (lane == 0 && sl < q.nvec) {
+    if (shared) st_x(part + sl, s);
+    else part[sl] = s;
+  }
+}
+static_assert(2 * kPairs == CW, "a slice for each wave");
+
+// their sum to every thread: 256 strided sums, then by halves
+__device__ inline double total(const MultiProb& q, const double* part, bool shared, double* red) {
+  const int tid = threadIdx.x, lane = tid & 63;
+  double v = 0.0;
+  if (tid < 256)
+    for (int i = tid; i < q.nvec; i += 256) v += shared ? ld_x(part + i) : part[i];
+  __syncthreads();
+  if (tid < 256) red[tid] = v;
+  __syncthreads();
+  double s = (red[lane] + red[lane + 128]) + (red[lane + 64] + red[lane + 192]);
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) s += __shfl_xor(s, m, 64);
+  return s;
+}
+
+// Ap = (O^T u)/B - Om mean(u) + eps p, partial p.Ap (nqs_optimizer.c:103-106)
+__device__ inline void pairs_ap(const MultiProb& q, const Pairs& w, Elem* st, double* part, bool shared,
+                                double* red) {
+  const long L = vec_len(q);
+  const double inv = 1.0 / (double)q.B, gu = ld_x(q.g + L - 1);
+  double g[kPairs], pa[kPairs];
+#pragma unroll
+  for (int i = 0; i < kPairs; i++) g[i] = ld_x(q.g + (w.at(i) < L ? w.at(i) : L - 1));
+  const double mu = mul_only(gu, inv);
+#pragma unroll
+  for (int i = 0; i < kPairs; i++) {
+    const double ap = fma(q.eps, st[i].p, fma(g[i], inv, -mul_only(st[i].om, mu)));
+    st[i].ap = w.at(i) < L - 1 ? ap : 0.0;
+    pa[i] = w.at(i) < L ? st[i].p * st[i].ap : 0.0;
+  }
+  put_parts(q, w, pa, part, shared, red);
+}
+
+// x += alpha p, r -= alpha Ap, partial r.r (nqs_optimizer.c:113-120)
+__device__ inline void pairs_xr(const MultiProb& q, const Pairs& w, Elem* st, double a, double* part,
+                                bool shared, double* red) {
+  double rr[kPairs];
+#pragma unroll
+  for (int i = 0; i < kPairs; i++) {
+    st[i].x = fma(a, st[i].p, st[i].x);
+    st[i].r = fma(-a, st[i].ap, st[i].r);
+    rr[i] = w.at(i) < vec_len(q) ? st[i].r * st[i].r : 0.0;
+  }
+  put_parts(q, w, rr, part, shared, red);
+}
+
+__device__ inline void load_pairs(const MultiProb& q, const Pairs& w, Elem* st) {
+  const long L = vec_len(q);
+#pragma unroll
+  for (int i = 0; i < kPairs; i++) {
+    const long e = w.at(i) < L ? w.at(i) : L - 1;   // the last element is zero
+    st[i] = Elem{q.x[e], q.r[e], ld_x(q.p + e), q.Ap[e], q.Om[e]};
+    if (w.at(i) >= L) st[i].om = 0.0;
+  }
+}
+
+// |r|^2 before iteration it, of the launch sequence's partials
+__device__ inline double* part_rr(const MultiProb& q, int it) {
+  return q.part + (it < 0 ? 0 : 2 + (it & 1)) * (long)kMultiMaxPart;
+}
+__device__ inline bool broke(double pAp) { return !(fabs(pAp) >= 1e-30); }
+
+// ---------------------------------------------------------------------------
+// spin words [B][nw] (bit set: s = -1); t by hidden unit for Z (tT [M][B]) and,
+// with the unit column and zeros to whole tiles, as the A operand of G (tA:
+// tile of 16 hidden units, four samples, lane): 64 samples a workgroup
+__global__ __launch_bounds__(256) void k_mb_prep(MultiBatch mb) {
+  __shared__ double tile[64][33];
+  const MultiProb& q = mb.probs[find_prob<F_PREP>(mb, blockIdx.x)];
+  const long b0 = (blockIdx.x - q.blk_prep) * 64L;
+  const int nb = (int)(q.B - b0 < 64 ? q.B - b0 : 64);
+  for (int e = threadIdx.x; e < nb * q.nw; e += 256) {
+    const int b = e / q.nw, w = e - b * q.nw;
+    const int* s = q.spins + (b0 + b) * q.N;
+    unsigned m = 0;
+    for (int i = w * 32; i < q.N && i < w * 32 + 32; i++)
+      if (s[i] < 0) m |= 1u << (i & 31);
+    q.bits[b0 * q.nw + e] = m;
+  }
+  const int B4 = (q.B + 15) / 16 * 4, j1 = B4 - b0 / 4 < 16 ? B4 - (int)(b0 / 4) : 16;
+  for (int e = threadIdx.x; e < (q.M + 16) / 16 * j1 * 64; e += 256) {
+    const int lr = e & 15, lk = (e >> 4) & 3, ht = (e >> 6) / j1, j = (e >> 6) - ht * j1;
+    const int h = ht * 16 + lr, b = 4 * j + lk;
+    const double t = b >= nb || h > q.M ? 0.0 : h == q.M ? 1.0 : q.t[(b0 + b) * q.M + h];
+    q.tA[((long)ht * B4 + b0 / 4 + j) * 64 + (e & 63)] = t;
+  }
+  for (int h0 = 0; h0 < q.M; h0 += 32) {
+    __syncthreads();
+    for (int e = threadIdx.x; e < 64 * 32; e += 256) {
+      const int b = e >> 5, h = h0 + (e & 31);
+      if (b < nb && h < q.M) tile[b][e & 31] = q.t[(b0 + b) * q.M + h];
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < 64 * 32; e += 256) {
+      const int h = h0 + (e >> 6), b = e & 63;
+      if (b < nb && h < q.M) q.tT[(long)h * q.B + b0 + b] = tile[b][e >> 6];
+    }
+  }
+}
+
+// One phase of every problem as a launch of its own (iteration `it` of the CG
+// phases).  A problem's scalars are written by its first block in PH_P; a
+// block of that launch that reads `done` after the write has nothing left to do.
+__global__ __launch_bounds__(CT) void k_mb_phase(MultiBatch mb, int phase, int it) {
+  extern __shared__ double lds[];
+  __shared__ int done;   // read once: the whole workgroup takes one branch
+  const int blk = blockIdx.x;
+  const MultiProb& q = mb.probs[phase == PH_Z ? find_prob<F_Z>(mb, blk)
+                                : phase <= PH_GE || phase == PH_G ? find_prob<F_G>(mb, blk)
+                                                                  : find_prob<F_VEC>(mb, blk)];
+  const Lds l = carve(q, lds);
+  if (phase <= PH_GE) {
+    cg_tiles(q, l, blk - q.blk_g, 1, blk - q.blk_g + 1, phase, phase == PH_G1 ? q.g : q.Ap);
+    return;
+  }
+  const long L = vec_len(q);
+  const Pairs w{blk - q.blk_vec, (((q.nvec + 1) >> 1) + kPairs - 1) / kPairs};
+  double* red = l.red;
+  if (phase == PH_F) {
+    // Om = (O^T 1)/B, F = (O^T E)/B - Om <E>; CG start x = 0, r = p = F
+    // (cg_solve, nqs_optimizer.c:84-95)
+    double ff[kPairs];
+#pragma unroll
+    for (int i = 0; i < kPairs; i++) {
+      const long e = w.at(i);
+      ff[i] = 0.0;
+      if (e < L) {
+        const double inv = 1.0 / (double)q.B;
+        const double om = mul_only(q.g[e], inv);
+        const double f = e == L - 1 ? 0.0 : fma(q.Ap[e], inv, -mul_only(om, q.stats[0]));
+        q.Om[e] = om;
+        q.x[e] = 0.0;
+        q.r[e] = f;
+        q.p[e] = f;
+        ff[i] = f * f;
+      }
+    }
+    put_parts(q, w, ff, part_rr(q, -1), true, red);
+    if (w.j0 == 0 && threadIdx.x == 0) {
+      q.sc->iters = 0;
+      q.sc->converged = 0;
+      q.sc->breakdown = 0;
+      q.sc->done = q.max_it <= 0 ? 1 : 0;
+    }
+    return;
+  }
+  if (threadIdx.x == 0) done = q.sc->done;
+  __syncthreads();
+  if (done) return;
+  if (phase == PH_Z) {
+    const int t0 = (blk - q.blk_z) * (kZb / 16), nT = (q.B + 15) / 16;
+    cg_rows(q, l, t0, t0 + kZb / 16 < nT ? t0 + kZb / 16 : nT, false, false);
+    return;
+  }
+  if (phase == PH_G) {
+    cg_tiles(q, l, blk - q.blk_g, 1, blk - q.blk_g + 1, PH_G, q.g);
+    return;
+  }
+  Elem st[kPairs];
+  load_pairs(q, w, st);
+  double* part_pap = q.part + kMultiMaxPart;
+  if (phase == PH_AP) {
+    pairs_ap(q, w, st, part_pap, true, red);
+#pragma unroll
+    for (int i = 0; i < kPairs; i++)
+      if (w.at(i) < L) q.Ap[w.at(i)] = st[i].ap;
+    return;
+  }
+  const double pAp = total(q, part_pap, true, red), rs = total(q, part_rr(q, it - 1), true, red);
+  if (phase == PH_XR) {
+    if (broke(pAp)) return;
+    pairs_xr(q, w, st, rs / pAp, part_rr(q, it), true, red);
+#pragma unroll
+    for (int i = 0; i < kPairs; i++)
+      if (w.at(i) < L) {
+        q.x[w.at(i)] = st[i].x;
+        q.r[w.at(i)] = st[i].r;
+      }
+    return;
+  }
+  const double rs0 = total(q, part_rr(q, -1), true, red);
+  const double rn = broke(pAp) ? rs : total(q, part_rr(q, it), true, red);
+  const bool conv = !broke(pAp) && rn <= q.tol * q.tol * rs0;
+  if (!broke(pAp) && !conv) {
+    const double be = rn / rs;
+#pragma unroll
+    for (int i = 0; i < kPairs; i++)
+      if (w.at(i) < L) q.p[w.at(i)] = fma(be, st[i].p, st[i].r);
+  }
+  if (w.j0 == 0 && threadIdx.x == 0) {
+    CGScalars* sc = q.sc;
+    sc->rs0 = rs0;
+    sc->pAp = pAp;
+    sc->rs_new = rn;
+    sc->rs = rn;
+    if (broke(pAp)) sc->breakdown = 1;
+    else sc->iters = it + 1;
+    if (conv) sc->converged = 1;
+    if (broke(pAp) || conv || it + 1 >= q.max_it) sc->done = 1;
+  }
+}
+
+// The problem's nb workgroups meet: every thread's exchanged stores have
+// reached the agent's coherence point (the wait), then one arrival; `n` counts
+// the meetings.  False when the others do not arrive within the poll limit
+// (seconds): the kernel then ends.
+__device__ inline bool meet(const MultiProb& q, unsigned& n) {
+  __shared__ int ok;
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  if (q.nb == 1) return true;
+  n++;
+  if (threadIdx.x == 0) {
+    const unsigned want = n * (unsigned)q.nb;
+    __hip_atomic_fetch_add(q.bar, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    int got = 0;
+    for (int i = 0; i < (1 << 24); i++) {
+      if ((int)(__hip_atomic_load(q.bar, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - want) >= 0) {
+        got = 1;
+        break;
+      }
+      __builtin_amdgcn_s_sleep(1);
+    }
+    ok = got;
+  }
+  __syncthreads();
+  return ok != 0;
+}
+
+// Up to `iters` CG iterations of every problem (matvec_only: O^T O p once,
+// which changes nothing that the CG start has set).  Consecutive workgroups of
+// a problem sit on one XCD (block b runs on XCD b % 8), where its t stays in
+// that XCD's L2.
+__global__ __launch_bounds__(CT) void k_mb_cg(MultiBatch mb, int iters, int matvec_only) {
+  extern __shared__ double lds[];
+  const int lb = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  if (lb >= mb.nblk_cg) return;
+  const MultiProb& q = mb.probs[find_prob<F_CG>(mb, lb)];
+  if (q.max_it <= 0) return;   // nothing to do, and no meeting to pass
+  const Lds l = carve(q, lds);
+  double* red = l.red;
+  const int b = lb - q.blk_cg, nb = q.nb, J = (q.nvec + 1) >> 1, tid = threadIdx.x;
+  const int nT = (q.B + 15) / 16, t0 = (int)((long)nT * b / nb), t1 = (int)((long)nT * (b + 1) / nb);
+  const int units = tile_units(q, q.nt);
+  const long L = vec_len(q);
+  // every workgroup has the whole vectors, or every js-th pair of slices; in
+  // registers (one group) or, past kPairs pairs, in memory
+  const bool own = nb > 1 && J <= kPairs, local = own || nb == 1;
+  const int j0 = own ? 0 : b, js = own ? 1 : nb;
+  const int groups = ((J - j0 + js - 1) / js + kPairs - 1) / kPairs;
+  const bool kept = groups <= 1;
+  double* pp = local ? l.part : q.part + kMultiMaxPart;
+  double* pr = local ? l.part : q.part + 2 * kMultiMaxPart;
+  Elem st[kPairs];
+  Pairs w{j0, js};
+  if (kept) load_pairs(q, w, st);
+  unsigned n = 0;
+  bool live = true, conv = false, brk = false;
+  int it = 0;
+  double rs = total(q, q.part, true, red), rs0 = rs, rn = rs, pAp = 0.0;
+  if (own) {
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kPairs; i++) red[i * CT + tid] = st[i].p;
+  }
+  // what only this workgroup has is its own threads' business
+  auto pause = [&]() -> bool {
+    if (local) {
+      __syncthreads();
+      return true;
+    }
+    return meet(q, n);
+  };
+  const int cap = matvec_only ? 1 : iters < q.max_it ? iters : q.max_it;
+  while (it < cap) {
+    cg_rows(q, l, t0, t1, own, it > 0 && (t1 - t0) * 16 <= kZs);
+    if (!(live = meet(q, n))) break;
+    cg_tiles(q, l, b, nb, units, PH_G, q.g);
+    if (matvec_only) break;
+    if (!(live = meet(q, n))) break;
+    for (int g = 0; g < groups; g++) {
+      w.j0 = j0 + g * kPairs * js;
+      if (!kept) load_pairs(q, w, st);
+      pairs_ap(q, w, st, pp, !local, red);
+      if (!kept) {
+#pragma unroll
+        for (int i = 0; i < kPairs; i++)
+          if (w.at(i) < L) q.Ap[w.at(i)] = st[i].ap;
+      }
+    }
+    if (!(live = pause())) break;
+    pAp = total(q, pp, !local, red);
+    if (broke(pAp)) {
+      brk = true;
+      break;
+    }
+    const double a = rs / pAp;
+    for (int g = 0; g < groups; g++) {
+      w.j0 = j0 + g * kPairs * js;
+      if (!kept) load_pairs(q, w, st);
+      pairs_xr(q, w, st, a, pr, !local, red);
+      if (!kept) {
+#pragma unroll
+        for (int i = 0; i < kPairs; i++)
+          if (w.at(i) < L) {
+            q.x[w.at(i)] = st[i].x;
+            q.r[w.at(i)] = st[i].r;
+          }
+      }
+    }
+    if (!(live = pause())) break;
+    rn = total(q, pr, !local, red);
+    it++;
+    if (rn <= q.tol * q.tol * rs0) {
+      conv = true;
+      break;
+    }
+    const double be = rn / rs;
+    rs = rn;
+    if (it >= cap) break;
+    if (own) __syncthreads();   // the sums in red are read
+    for (int g = 0; g < groups; g++) {
+      w.j0 = j0 + g * kPairs * js;
+      if (!kept) load_pairs(q, w, st);
+#pragma unroll
+      for (int i = 0; i < kPairs; i++) {
+        st[i].p = fma(be, st[i].p, st[i].r);
+        if (own) red[i * CT + tid] = st[i].p;
+        else if (w.at(i) < L) st_x(q.p + w.at(i), st[i].p);
+      }
+    }
+    if (own) __syncthreads();
+    else if (!(live = meet(q, n))) break;
+  }
+  if (kept && !matvec_only && (!own || b == 0)) {
+#pragma unroll
+    for (int i = 0; i < kPairs; i++)
+      if (w.at(i) < L) q.x[w.at(i)] = st[i].x;
+  }
+  if (threadIdx.x == 0) {
+    if (b == 0 && !matvec_only) {
+      CGScalars* sc = q.sc;
+      sc->rs0 = rs0;
+      sc->pAp = pAp;
+      sc->rs_new = rn;
+      sc->rs = rn;
+      sc->iters = live ? it : -1;
+      sc->converged = conv ? 1 : 0;
+      sc->breakdown = brk ? 1 : 0;
+      sc->done = 1;
+    }
+    // the last workgroup to leave resets the counters for the next launch:
+    // all have passed their last meeting then
+    if (__hip_atomic_fetch_add(q.bar + 32, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+        (unsigned)nb - 1u) {
+      __hip_atomic_store(q.bar, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(q.bar + 32, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
+}
+
+// Block partial -> problem scalar: the block that arrives last among `nblk`
+// returns true with the sum of all partials (block order) in `total`.
 __device__ inline bool reduce_last(double v, double* red, double* part, unsigned* ticket,
                                    int blk, int nblk, double& total) {
   __shared__ int last;
@@ -157,277 +831,12 @@ __device__ inline bool reduce_last(double v, double* red, double* part, unsigned
   return true;
 }
 
-__device__ inline int vec_blocks(const MultiProb& q) {
-  return ((q.M + 1) * (q.N + 1) + kMultiVecBlock - 1) / kMultiVecBlock;
-}
-__device__ inline bool cg_done(const MultiProb& q) {
-  return __builtin_nontemporal_load(&q.sc->done) != 0;
-}
-
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_mb_prep(MultiBatch mb) {
-  const int qi = find_prob<F_PREP>(mb, blockIdx.x);
-  const MultiProb& q = mb.probs[qi];
-  const int b = (blockIdx.x - q.blk_prep) * 256 + threadIdx.x;
-  if (b >= q.B) return;
-  const int N = q.N, M = q.M, N1 = N + 1, B = q.B;
-  for (int j = 0; j <= N; j++) {
-    const double v = j < N ? (double)q.spins[(long)b * N + j] : 1.0;
-    q.S1[(long)b * N1 + j] = v;
-    q.S1t[(long)j * B + b] = v;
-  }
-  for (int h = 0; h <= M; h++) q.T1t[(long)h * B + b] = h < M ? q.t[(long)b * M + h] : 1.0;
-}
-
-// Row weights of the CG product, u_b = sum_h [t_b, 1]_h (V [s_b, 1]^T)_h, in
-// partial sums over 64-row tiles: work item (tile tm, samples 64 tb + [0,
-// 64)) forms its 64 x 64 tile of Z = V S1^T on MFMA (K = N+1), weights it by
-// [t_b, 1]_h as it leaves the accumulators (Z is not stored) and writes the
-// tile's column sums to u[tm][b].  A thread sums its 8 rows of the tile for
-// its 2 samples; the 8 threads that share a sample are added in a fixed
-// order.  The G product adds the tiles' partials in tile order.
-__device__ inline void mb_zu(const MultiBatch& mb, int blk) {
-  __shared__ double ured[8][MT];
-  const int qi = find_prob<F_Z>(mb, blk);
-  const MultiProb& q = mb.probs[qi];
-  if (cg_done(q)) return;
-  const int M1 = q.M + 1, N1 = q.N + 1;
-  const long B = q.B;
-  const int tiles_n = (q.B + MT - 1) / MT;
-  const int t = blk - q.blk_z, tm = t / tiles_n;
-  const int row0 = tm * MT, col0 = (t % tiles_n) * MT;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
-  const int lr = lane & 15, lk = lane >> 4;
-  v4d acc[2][2];
-  tile_acc(M1, q.B, 0, N1, q.p, N1, nullptr, 0, 0, q.S1, N1, row0, col0, acc);
-  double part[2] = {0.0, 0.0};
-#pragma unroll
-  for (int j = 0; j < 2; j++) {
-    const long gc = col0 + wc + 16 * j + lr;
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int gr = row0 + wr + 16 * i + lk + 4 * r;
-        if (gr < M1 && gc < B) part[j] += acc[i][j][r] * q.T1t[(long)gr * B + gc];
-      }
-  }
-  // slot (wave / 2) * 4 + lk of column wc + 16 j + lr: every (slot, column) once
-#pragma unroll
-  for (int j = 0; j < 2; j++) ured[(wave >> 1) * 4 + lk][wc + 16 * j + lr] = part[j];
-  __syncthreads();
-  if (tid < MT) {
-    double u = 0.0;
-#pragma unroll
-    for (int k = 0; k < 8; k++) u += ured[k][tid];
-    if (col0 + tid < B) q.u[(long)tm * B + col0 + tid] = u;
-  }
-  __syncthreads();   // ured is read before a later work item of this block writes it
-}
-
-// Gp[slot][split] = (T1t w)[:, Kchunk] S1t[:, Kchunk]^T, (M+1) x (N+1): the
-// operand [t_b, 1]_h times the sample weight w_b.  With two slots (the force)
-// slot 0 takes w = 1 and slot 1 w = E; with one slot (CG) w = u = O p, the
-// sum of the row-tile partials of mb_zu.
-__device__ inline void mb_gemm_g(const MultiBatch& mb, int blk, int force) {
-  const int qi = force ? find_prob<F_G2>(mb, blk) : find_prob<F_G>(mb, blk);
-  const MultiProb& q = mb.probs[qi];
-  if (!force && cg_done(q)) return;
-  const int M1 = q.M + 1, N1 = q.N + 1;
-  const int tm = (M1 + MT - 1) / MT, tn = (N1 + MT - 1) / MT;
-  int t = blk - (force ? q.blk_g2 : q.blk_g);
-  const int per_slot = tm * tn * q.nsplit;
-  const int slot = t / per_slot;
-  t -= slot * per_slot;
-  const int split = t / (tm * tn);
-  t -= split * tm * tn;
-  const int chunk = ((q.B + q.nsplit - 1) / q.nsplit + MKS - 1) / MKS * MKS;
-  const int k0 = split * chunk, k1 = min(q.B, k0 + chunk);
-  const double* w = force ? (slot == 0 ? nullptr : q.E) : q.u;
-  const int nw = force ? 1 : tm;   // row tiles of mb_zu
-  double* C = q.Gp + ((long)slot * q.nsplit + split) * M1 * N1;
-  if (k0 >= k1) {
-    // empty chunk: its partial is zero
-    for (int e = threadIdx.x; e < MT * MT; e += 256) {
-      const int r = (t / tn) * MT + e / MT, c = (t % tn) * MT + e % MT;
-      if (r < M1 && c < N1) C[(long)r * N1 + c] = 0.0;
-    }
-    return;
-  }
-  tile_nt(M1, N1, k0, k1, q.T1t, q.B, w, nw, q.B, q.S1t, q.B, C, N1, (t / tn) * MT,
-          (t % tn) * MT);
-}
-
-// Om = (O^T 1)/B, F = (O^T E)/B - Om <E>; CG start x = 0, r = p = F,
-// rs = rs0 = F.F (cg_solve, nqs_optimizer.c:84-95)
-__global__ __launch_bounds__(kMultiVecBlock) void k_mb_force(MultiBatch mb) {
-  __shared__ double red[kMultiVecBlock];
-  const int qi = find_prob<F_VEC>(mb, blockIdx.x);
-  const MultiProb& q = mb.probs[qi];
-  const int blk = blockIdx.x - q.blk_vec, nblk = vec_blocks(q);
-  const int N1 = q.N + 1, L = (q.M + 1) * N1;
-  const int e = blk * kMultiVecBlock + threadIdx.x;
-  double ff = 0.0;
-  if (e < L) {
-    const long plane = (long)q.nsplit * L;
-    double g1 = 0.0, gE = 0.0;
-    for (int k = 0; k < q.nsplit; k++) {
-      g1 += q.Gp[(long)k * L + e];
-      gE += q.Gp[plane + (long)k * L + e];
-    }
-    const double inv = 1.0 / (double)q.B;
-    const double om = g1 * inv;
-    const double f = (e == L - 1) ? 0.0 : gE * inv - om * q.stats[0];
-    q.Om[e] = om;
-    q.F[e] = f;
-    q.x[e] = 0.0;
-    q.r[e] = f;
-    q.p[e] = f;
-    ff = f * f;
-  }
-  double tot;
-  if (reduce_last(ff, red, q.part, q.ticket, blk, nblk, tot) && threadIdx.x == 0) {
-    CGScalars* sc = q.sc;
-    sc->rs = tot;
-    sc->rs0 = tot;
-    sc->beta = 0.0;
-    sc->iters = 0;
-    sc->converged = 0;
-    sc->breakdown = 0;
-    sc->done = q.max_it <= 0 ? 1 : 0;
-  }
-}
-
-// Ap = (O^T u)/B - Om mean(u) + eps p, pAp; alpha = rs / pAp or breakdown
-// when |pAp| < 1e-30 (nqs_optimizer.c:103-112)
-__device__ inline void mb_finish(const MultiBatch& mb, int gblk) {
-  __shared__ double red[kMultiVecBlock];
-  const int qi = find_prob<F_VEC>(mb, gblk);
-  const MultiProb& q = mb.probs[qi];
-  if (cg_done(q)) return;
-  const int blk = gblk - q.blk_vec, nblk = vec_blocks(q);
-  const int L = (q.M + 1) * (q.N + 1);
-  const int e = blk * kMultiVecBlock + threadIdx.x;
-  double pa = 0.0;
-  if (e < L) {
-    double g = 0.0, gu = 0.0;
-    for (int k = 0; k < q.nsplit; k++) {
-      g += q.Gp[(long)k * L + e];
-      gu += q.Gp[(long)k * L + L - 1];
-    }
-    const double inv = 1.0 / (double)q.B;
-    const double ap = (e == L - 1) ? 0.0 : g * inv - q.Om[e] * (gu * inv) + q.eps * q.p[e];
-    q.Ap[e] = ap;
-    pa = q.p[e] * ap;
-  }
-  double tot;
-  if (reduce_last(pa, red, q.part, q.ticket, blk, nblk, tot) && threadIdx.x == 0) {
-    CGScalars* sc = q.sc;
-    sc->pAp = tot;
-    if (!(fabs(tot) >= 1e-30)) {
-      sc->breakdown = 1;
-      sc->done = 1;
-    } else {
-      sc->alpha = sc->rs / tot;
-    }
-  }
-}
-
-// x += alpha p, r -= alpha Ap, rs_new = r.r; converged when
-// rs_new <= tol^2 rs0, else beta = rs_new / rs (nqs_optimizer.c:113-136)
-__device__ inline void mb_update(const MultiBatch& mb, int gblk) {
-  __shared__ double red[kMultiVecBlock];
-  const int qi = find_prob<F_VEC>(mb, gblk);
-  const MultiProb& q = mb.probs[qi];
-  if (cg_done(q)) return;
-  const int blk = gblk - q.blk_vec, nblk = vec_blocks(q);
-  const int L = (q.M + 1) * (q.N + 1);
-  const int e = blk * kMultiVecBlock + threadIdx.x;
-  const double a = q.sc->alpha;
-  double rr = 0.0;
-  if (e < L) {
-    q.x[e] += a * q.p[e];
-    const double rn = q.r[e] + (-a) * q.Ap[e];
-    q.r[e] = rn;
-    rr = rn * rn;
-  }
-  double tot;
-  if (reduce_last(rr, red, q.part, q.ticket, blk, nblk, tot) && threadIdx.x == 0) {
-    CGScalars* sc = q.sc;
-    sc->iters += 1;
-    sc->rs_new = tot;
-    if (tot <= q.tol * q.tol * sc->rs0) {
-      sc->converged = 1;
-      sc->done = 1;
-    } else {
-      sc->beta = tot / sc->rs;
-      sc->rs = tot;
-      if (sc->iters >= q.max_it) sc->done = 1;
-    }
-  }
-}
-
-// p = r + beta p
-__device__ inline void mb_dir(const MultiBatch& mb, int gblk) {
-  const int qi = find_prob<F_VEC>(mb, gblk);
-  const MultiProb& q = mb.probs[qi];
-  if (cg_done(q)) return;
-  const int L = (q.M + 1) * (q.N + 1);
-  const int e = (gblk - q.blk_vec) * kMultiVecBlock + threadIdx.x;
-  if (e < L) q.p[e] = q.r[e] + q.sc->beta * q.p[e];
-}
-
-// the CG launches: one block per work item
-__global__ __launch_bounds__(256) void k_mb_zu(MultiBatch mb) { mb_zu(mb, blockIdx.x); }
-__global__ __launch_bounds__(256) void k_mb_gemm_g(MultiBatch mb, int force) {
-  mb_gemm_g(mb, blockIdx.x, force);
-}
-__global__ __launch_bounds__(kMultiVecBlock) void k_mb_finish(MultiBatch mb) {
-  mb_finish(mb, blockIdx.x);
-}
-__global__ __launch_bounds__(kMultiVecBlock) void k_mb_update(MultiBatch mb) {
-  mb_update(mb, blockIdx.x);
-}
-__global__ __launch_bounds__(kMultiVecBlock) void k_mb_dir(MultiBatch mb) { mb_dir(mb, blockIdx.x); }
-
-// Every CG iteration of every problem in one cooperative launch: the five
-// phases of an iteration walk their work items (the blocks of the launch
-// sequence above, same device functions, so the same results bit for bit)
-// grid-stride, with a grid barrier between phases.  Every block passes every
-// barrier: the phase loops only skip items, and the loop ends for all blocks
-// together when, after an iteration's last barrier, every problem reads done
-// (its flags were written before that barrier).  The launch is cooperative,
-// so it either has all its blocks resident or does not start.
-// matvec_only: one iteration's A p, p.Ap and alpha only (idempotent at the
-// CG start; the autotuner times it against the launch sequence's).
-__global__ __launch_bounds__(256) void k_mb_cg_persist(MultiBatch mb, int iters, int matvec_only) {
-  static_assert(kMultiVecBlock == 256, "one block size for every phase");
-  cooperative_groups::grid_group grid = cooperative_groups::this_grid();
-  for (int it = 0; it < iters; it++) {
-    for (int b = blockIdx.x; b < mb.nblk_z; b += gridDim.x) mb_zu(mb, b);
-    grid.sync();
-    for (int b = blockIdx.x; b < mb.nblk_g; b += gridDim.x) mb_gemm_g(mb, b, 0);
-    grid.sync();
-    for (int b = blockIdx.x; b < mb.nblk_vec; b += gridDim.x) mb_finish(mb, b);
-    if (matvec_only) break;   // uniform: a kernel argument
-    grid.sync();
-    for (int b = blockIdx.x; b < mb.nblk_vec; b += gridDim.x) mb_update(mb, b);
-    grid.sync();
-    for (int b = blockIdx.x; b < mb.nblk_vec; b += gridDim.x) mb_dir(mb, b);
-    grid.sync();
-    bool all = true;
-    for (int i = 0; i < mb.n; i++) all = all && cg_done(mb.probs[i]);
-    if (all) break;
-  }
-}
-
 // theta -= lr delta in the reference layout [a | b | W], |delta|^2
 __global__ __launch_bounds__(kMultiVecBlock) void k_mb_apply(MultiBatch mb) {
   __shared__ double red[kMultiVecBlock];
-  const int qi = find_prob<F_VEC>(mb, blockIdx.x);
+  const int qi = find_prob<F_APPLY>(mb, blockIdx.x);
   const MultiProb& q = mb.probs[qi];
-  const int blk = blockIdx.x - q.blk_vec, nblk = vec_blocks(q);
+  const int blk = blockIdx.x - q.blk_apply, nblk = q.nvec;
   const int N = q.N, M = q.M, N1 = N + 1, L = (M + 1) * N1;
   const int e = blk * kMultiVecBlock + threadIdx.x;
   double xx = 0.0;
@@ -467,31 +876,121 @@ __global__ void k_mb_gather(MultiBatch mb, double* out) {
   o[10] = q.range_flag ? (double)*q.range_flag : 0.0;
 }
 
+constexpr size_t kCgLds = 156 * 1024;   // of the CU's 160 KB: one workgroup per CU
+
+size_t lds_bytes(const MultiProb& q, int hct, int zb) {
+  const size_t z = (size_t)hct * 16 * q.si + (size_t)hct * 2 * zb;
+  const size_t g = (size_t)CW * (kTiles * 256 + 64 + 96);
+  return sizeof(double) * (lds_head(q.nw) + (z > g ? z : g));
+}
+
+// Cycles of a CG iteration of q on nb workgroups of a CU each (FP64 16x16x4
+// MFMAs take a SIMD 64): Z by 16-sample tiles, G by units (the site tiles of a
+// wave, nt, for the fewest), the meetings and the vector work.
+double iter_cost(const MultiProb& q, int nb, int& nt) {
+  const int HT = (q.M + 16) / 16, KK = (q.N + 4) / 4, nT = (q.B + 15) / 16;
+  const double z = 16.0 * ((nT + nb - 1) / nb) * HT * (KK + 4) + (q.M + 1.0) * (q.N + 1.0) / 8;
+  const int ws = q.nsplit < CW ? q.nsplit : CW, rounds = q.nsplit / ws;
+  double g = 0.0;
+  for (int t = 1; t <= kTiles && t <= kTiles * 2 * ws / CW + 1; t++) {
+    // a unit's elements are at most kTiles per thread
+    if (t * (CW / ws) > 2 * kTiles) break;
+    const int n = (tile_units(q, t) + nb - 1) / nb;
+    const double c = n * (2000.0 + rounds * (1200.0 + (q.chunk + 63) / 64 * (600.0 + 2048.0 * t)));
+    if (t == 1 || c < g) {
+      g = c;
+      nt = t;
+    }
+  }
+  const int J = (q.nvec + 1) / 2;
+  return z + g + (nb == 1 ? 8000.0 : J <= kPairs ? 16000.0 : 26000.0) + 4000.0 * J / (kPairs * nb);
+}
+
 }  // namespace
 
+int multi_words(int N) { return (N + 1 + 31) / 32; }
+size_t multi_ta_elems(int B, int M) { return (size_t)((M + 16) / 16) * ((B + 15) / 16 * 4) * 64; }
+
+// nsplit slots of equal runs of samples (multiples of 16)
+void multi_shape(MultiProb& q, int nsplit) {
+  const int N1 = q.N + 1, M1 = q.M + 1, n4 = (N1 + 3) / 4 * 4;
+  q.nsplit = nsplit;
+  q.chunk = ((q.B + nsplit - 1) / nsplit + 15) / 16 * 16;
+  q.nw = multi_words(q.N);
+  q.si = n4 + 2;   // 2 mod 4: the 16 x 2 operands of half a wave fall on 32 bank pairs
+  q.nvec = (M1 * N1 + kMultiVecBlock - 1) / kMultiVecBlock;
+}
+
+// Hidden tiles of a chunk of p and samples of a pass over it in Z, by what the
+// LDS holds for a workgroup's share of the samples
+void shape_rows(MultiProb& q) {
+  const int HT = (q.M + 16) / 16, nT = (q.B + 15) / 16;
+  q.zb = (nT + q.nb - 1) / q.nb * 16;
+  if (q.zb > kZs) q.zb = kZs;
+  q.hct = (HT + 1) / 2 * 2;
+  while (q.zb > kZb && lds_bytes(q, q.hct < 8 ? q.hct : 8, q.zb) > kCgLds) q.zb -= 16;
+  while (q.hct > 2 && lds_bytes(q, q.hct, q.zb) > kCgLds) q.hct -= 2;
+  const int nc = (HT + q.hct - 1) / q.hct;   // equal chunks
+  q.hct = ((HT + nc - 1) / nc + 1) / 2 * 2;
+}
+
+// First blocks of every launch, and the workgroups of the cooperative one:
+// every problem gets one; the rest go, to the next count that shortens its
+// iteration, to the problem with the longest.
 void multi_layout(MultiProb* probs, int n, MultiBatch& mb) {
-  int prep = 0, z = 0, g = 0, g2 = 0, vec = 0;
+  int cus = 0, dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    cus = 0;
+  (void)hipGetLastError();
+  size_t lds = 0;
+  std::vector<double> cost(n);
   for (int i = 0; i < n; i++) {
     MultiProb& q = probs[i];
-    const int M1 = q.M + 1, N1 = q.N + 1;
+    q.nb = 1;
+    cost[i] = iter_cost(q, 1, q.nt);
+  }
+  for (int left = cus - n; left > 0;) {
+    int at = 0;
+    for (int i = 1; i < n; i++)
+      if (cost[i] > cost[at]) at = i;
+    MultiProb& q = probs[at];
+    int nb = q.nb + 1, nt = 1;
+    double c = iter_cost(q, nb, nt);
+    while (c >= 0.98 * cost[at] && nb - q.nb <= left) c = iter_cost(q, ++nb, nt);
+    if (nb - q.nb > left) break;
+    left -= nb - q.nb;
+    q.nb = nb;
+    q.nt = nt;
+    cost[at] = c;
+  }
+  int prep = 0, z = 0, g = 0, vec = 0, apply = 0, cg = 0;
+  for (int i = 0; i < n; i++) {
+    MultiProb& q = probs[i];
+    shape_rows(q);
+    const size_t b = lds_bytes(q, q.hct, q.zb);
+    if (b > lds) lds = b;
     q.blk_prep = prep;
     q.blk_z = z;
     q.blk_g = g;
-    q.blk_g2 = g2;
     q.blk_vec = vec;
-    prep += (q.B + 255) / 256;
-    z += ((M1 + MT - 1) / MT) * ((q.B + MT - 1) / MT);
-    const int gt = ((M1 + MT - 1) / MT) * ((N1 + MT - 1) / MT) * q.nsplit;
-    g += gt;
-    g2 += 2 * gt;
-    vec += (M1 * N1 + kMultiVecBlock - 1) / kMultiVecBlock;
+    q.blk_apply = apply;
+    q.blk_cg = cg;
+    prep += (q.B + 63) / 64;
+    z += (q.B + kZb - 1) / kZb;
+    g += tile_units(q, q.nt);
+    vec += ((q.nvec + 1) / 2 + kPairs - 1) / kPairs;
+    apply += q.nvec;
+    cg += q.nb;
   }
   mb.n = n;
   mb.nblk_prep = prep;
   mb.nblk_z = z;
   mb.nblk_g = g;
-  mb.nblk_g2 = g2;
   mb.nblk_vec = vec;
+  mb.nblk_apply = apply;
+  mb.nblk_cg = n <= cus ? cg : 0;   // more problems than CUs: launch by launch
+  mb.lds = lds;
 }
 
 int launch_multi_prep(const MultiBatch& mb, hipStream_t st) {
@@ -503,77 +1002,63 @@ int launch_multi_prep(const MultiBatch& mb, hipStream_t st) {
   return 0;
 }
 
+namespace {
+
+int phase(const MultiBatch& mb, int ph, int it, const char* tag, hipStream_t st) {
+  static bool set = false;
+  if (!set) {
+    NQS_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k_mb_phase),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)kCgLds));
+    set = true;
+  }
+  const bool g = ph <= PH_GE || ph == PH_G, z = ph == PH_Z;
+  KScope ks(tag, st);
+  hipLaunchKernelGGL(k_mb_phase, dim3((unsigned)(z ? mb.nblk_z : g ? mb.nblk_g : mb.nblk_vec)), dim3(CT),
+                     z || g ? mb.lds : sizeof(double) * kPairs * CT, st, mb, ph, it);
+  count_launch();
+  NQS_HIP_CHECK(hipGetLastError());
+  return 0;
+}
+
+}  // namespace
+
 int launch_multi_force(const MultiBatch& mb, hipStream_t st) {
   if (mb.n <= 0) return 0;
-  {
-    KScope ks("multi_gemm_g", st);
-    hipLaunchKernelGGL(k_mb_gemm_g, dim3((unsigned)mb.nblk_g2), dim3(256), 0, st, mb, 1);
-  }
-  hipLaunchKernelGGL(k_mb_force, dim3((unsigned)mb.nblk_vec), dim3(kMultiVecBlock), 0, st, mb);
-  count_launch(2);
-  NQS_HIP_CHECK(hipGetLastError());
+  if (phase(mb, PH_G1, 0, "multi_gemm_g", st) || phase(mb, PH_GE, 0, "multi_gemm_g", st) ||
+      phase(mb, PH_F, 0, "multi_vec", st))
+    return -1;
   return 0;
 }
 
-int launch_multi_cg_iter(const MultiBatch& mb, int matvec_only, hipStream_t st) {
+int launch_multi_cg_iter(const MultiBatch& mb, int it, int matvec_only, hipStream_t st) {
   if (mb.n <= 0) return 0;
-  {
-    KScope ks("multi_gemm_z", st);
-    hipLaunchKernelGGL(k_mb_zu, dim3((unsigned)mb.nblk_z), dim3(256), 0, st, mb);
-  }
-  {
-    KScope ks("multi_gemm_g", st);
-    hipLaunchKernelGGL(k_mb_gemm_g, dim3((unsigned)mb.nblk_g), dim3(256), 0, st, mb, 0);
-  }
-  {
-    KScope ks("multi_vec", st);
-    hipLaunchKernelGGL(k_mb_finish, dim3((unsigned)mb.nblk_vec), dim3(kMultiVecBlock), 0, st, mb);
-    if (!matvec_only) {
-      hipLaunchKernelGGL(k_mb_update, dim3((unsigned)mb.nblk_vec), dim3(kMultiVecBlock), 0, st,
-                         mb);
-      hipLaunchKernelGGL(k_mb_dir, dim3((unsigned)mb.nblk_vec), dim3(kMultiVecBlock), 0, st, mb);
-    }
-  }
-  count_launch(matvec_only ? 3 : 5);
-  NQS_HIP_CHECK(hipGetLastError());
+  if (phase(mb, PH_Z, it, "multi_gemm_z", st) || phase(mb, PH_G, it, "multi_gemm_g", st)) return -1;
+  if (matvec_only) return 0;
+  if (phase(mb, PH_AP, it, "multi_vec", st) || phase(mb, PH_XR, it, "multi_vec", st) ||
+      phase(mb, PH_P, it, "multi_vec", st))
+    return -1;
   return 0;
-}
-
-int multi_persist_grid(const MultiBatch& mb) {
-  static int cap = -1;
-  if (cap < 0) {
-    int dev = 0, per_cu = 0;
-    hipDeviceProp_t prop;
-    if (hipGetDevice(&dev) != hipSuccess || hipGetDeviceProperties(&prop, dev) != hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_mb_cg_persist, 256, 0) !=
-            hipSuccess) {
-      (void)hipGetLastError();
-      cap = 0;
-    } else {
-      // two blocks per CU: the grid barrier's cost grows with the block
-      // count (measured 768 us per CG iteration at 512 blocks, 926 at 768)
-      cap = (per_cu < 2 ? per_cu : 2) * prop.multiProcessorCount;
-    }
-  }
-  int need = mb.nblk_z;
-  if (mb.nblk_g > need) need = mb.nblk_g;
-  if (mb.nblk_vec > need) need = mb.nblk_vec;
-  return need < cap ? need : cap;
 }
 
 int launch_multi_cg_persist(const MultiBatch& mb, int iters, hipStream_t st, int matvec_only) {
   if (mb.n <= 0 || iters <= 0) return 0;
-  const int grid = multi_persist_grid(mb);
-  if (grid <= 0) {
-    fprintf(stderr, "nqs_hip: no occupancy for the persistent CG launch\n");
+  if (mb.nblk_cg <= 0) {
+    fprintf(stderr, "nqs_hip: more problems than CUs for the persistent CG launch\n");
     return -1;
   }
+  static bool set = false;
+  if (!set) {
+    NQS_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k_mb_cg),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)kCgLds));
+    set = true;
+  }
   MultiBatch a = mb;
-  int it = matvec_only ? 1 : iters, mv = matvec_only ? 1 : 0;
-  void* args[] = {&a, &it, &mv};
+  void* args[] = {&a, &iters, &matvec_only};
   KScope ks("multi_cg", st);
-  const hipError_t e = hipLaunchCooperativeKernel(reinterpret_cast<const void*>(k_mb_cg_persist),
-                                                  dim3((unsigned)grid), dim3(256), args, 0, st);
+  // a grid of whole XCD rounds; the workgroups past the last problem return
+  const unsigned grid = (unsigned)(mb.nblk_cg + 7) / 8 * 8;
+  const hipError_t e = hipLaunchCooperativeKernel(reinterpret_cast<const void*>(k_mb_cg), dim3(grid),
+                                                  dim3(CT), args, (unsigned)mb.lds, st);
   count_launch();
   if (e != hipSuccess) {
     (void)hipGetLastError();
@@ -585,7 +1070,7 @@ int launch_multi_cg_persist(const MultiBatch& mb, int iters, hipStream_t st, int
 
 int launch_multi_apply(const MultiBatch& mb, hipStream_t st) {
   if (mb.n <= 0) return 0;
-  hipLaunchKernelGGL(k_mb_apply, dim3((unsigned)mb.nblk_vec), dim3(kMultiVecBlock), 0, st, mb);
+  hipLaunchKernelGGL(k_mb_apply, dim3((unsigned)mb.nblk_apply), dim3(kMultiVecBlock), 0, st, mb);
   count_launch();
   NQS_HIP_CHECK(hipGetLastError());
   return 0;

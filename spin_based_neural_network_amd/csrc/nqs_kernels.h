@@ -492,8 +492,8 @@ int launch_cg_rest(CGScalars* sc, double* x, double* r, double* p, const double*
 // sample b is the outer product [t_b, 1] (x) [s_b, 1] (t = tanh theta), so
 // O v = rowsum([t, 1] * ([s, 1] V^T)) and O^T w = ([t, 1] * w)^T [s, 1]:
 // two small GEMMs through the spins and t instead of two passes over O.
-constexpr int kMultiVecBlock = 256;      // threads of the vector kernels
-constexpr int kMultiMaxPart = 512;       // block partials per problem
+constexpr int kMultiVecBlock = 256;      // elements of a slice of the vectors
+constexpr int kMultiMaxPart = 512;       // slices per problem
 struct MultiProb {
   int B = 0, N = 0, M = 0, nsplit = 1, max_it = 0, C = 0;
   double eps = 0.0, tol = 0.0, lr = 0.0;
@@ -502,44 +502,50 @@ struct MultiProb {
   const int* spins = nullptr;    // [B][N]
   const double* t = nullptr;     // [B][M]
   const double* E = nullptr;     // [B]
-  double* S1 = nullptr;          // [B][N+1]   [s_b, 1]
-  double* S1t = nullptr;         // [N+1][B]
-  double* T1t = nullptr;         // [M+1][B]   [t_b, 1]^T
-  double* u = nullptr;           // [(M+64)/64][B] row weights of the CG product,
-                                 // (O p)_b, in partial sums over 64-row tiles
-  double* Gp = nullptr;          // [2][nsplit][M+1][N+1] split-K partials
-  double *x = nullptr, *r = nullptr, *p = nullptr, *Ap = nullptr, *Om = nullptr,
-         *F = nullptr;           // padded vectors
-  double* part = nullptr;        // [kMultiMaxPart] block partials
+  unsigned* bits = nullptr;      // [B][multi_words(N)] spin words (bit set: s = -1)
+  double* tT = nullptr;          // [M][B]
+  double* tA = nullptr;          // multi_ta_elems: [t, 1] by MFMA operands
+  double* u = nullptr;           // [B] row weights O p
+  double *g = nullptr;           // O^T u, padded vector
+  double *x = nullptr, *r = nullptr, *p = nullptr, *Ap = nullptr, *Om = nullptr;  // padded vectors
+  double* part = nullptr;        // [4][kMultiMaxPart] partial sums of the slices
+  unsigned* bar = nullptr;       // meeting counter, leaving counter at +32 (both start at 0)
   unsigned* ticket = nullptr;    // arrival counter of the last-block reductions
   CGScalars* sc = nullptr;
   const double* stats = nullptr; // [0] <E> (reference order), read by the force
   double* norm2 = nullptr;       // |delta|^2
   double* par = nullptr;         // [P] parameters, reference layout
   const int* range_flag = nullptr;  // the ansatz tables' range verdict (nonzero: refused)
-  // first block of this problem in each batched launch
-  // (blk_g: one G product per problem, CG; blk_g2: two, the force)
-  int blk_prep = 0, blk_z = 0, blk_g = 0, blk_g2 = 0, blk_vec = 0;
+  // set by multi_shape: samples per slot, spin words, LDS row stride, slices
+  int chunk = 16, nw = 1, si = 2, nvec = 1;
+  // set by multi_layout: workgroups in the cooperative launch, site tiles of
+  // a wave in O^T u, hidden tiles of a chunk of p, samples of a pass over it
+  int nb = 1, nt = 1, hct = 2, zb = 16;
+  // first block of this problem in each launch
+  int blk_prep = 0, blk_z = 0, blk_g = 0, blk_vec = 0, blk_apply = 0, blk_cg = 0;
 };
 struct MultiBatch {
   int n = 0;
   const MultiProb* probs = nullptr;   // device copy
-  int nblk_prep = 0, nblk_z = 0, nblk_g = 0, nblk_g2 = 0, nblk_vec = 0;
+  int nblk_prep = 0, nblk_z = 0, nblk_g = 0, nblk_vec = 0, nblk_apply = 0, nblk_cg = 0;
+  size_t lds = 0;
 };
+int multi_words(int N);
+size_t multi_ta_elems(int B, int M);
+void multi_shape(MultiProb& q, int nsplit);   // B, N, M set
 // fills the problems' first-block offsets of every launch and the totals
 void multi_layout(MultiProb* probs, int n, MultiBatch& mb);
-// [s, 1], [t, 1] operands and the two weight sets (1, E) of the force
+// spin words and transposed t of every problem
 int launch_multi_prep(const MultiBatch& mb, hipStream_t st);
-// Om, F, CG start (x = 0, r = p = F, rs = |F|^2)
+// Om, F, CG start (x = 0, r = p = F, |F|^2)
 int launch_multi_force(const MultiBatch& mb, hipStream_t st);
-// one CG iteration (A p, alpha, x / r update, beta, p) on every problem
-// not yet done; `matvec_only` stops after A p and alpha (idempotent at the
-// CG start, used to time the split factors)
-int launch_multi_cg_iter(const MultiBatch& mb, int matvec_only, hipStream_t st);
+// CG iteration `it` (A p, alpha, x / r update, beta, p) on every problem not
+// yet done, a launch per phase; `matvec_only` stops after A p (idempotent at
+// the CG start, used to time the split factors)
+int launch_multi_cg_iter(const MultiBatch& mb, int it, int matvec_only, hipStream_t st);
 // up to `iters` CG iterations of every problem in one cooperative launch
-// (same results as as many launch_multi_cg_iter calls; matvec_only: one
-// iteration's A p and alpha, as launch_multi_cg_iter's); -1 when the device
-// refuses the cooperative launch
+// (same results as as many launch_multi_cg_iter calls; matvec_only: one A p);
+// -1 when the device refuses the cooperative launch
 int launch_multi_cg_persist(const MultiBatch& mb, int iters, hipStream_t st, int matvec_only = 0);
 // par -= lr * x (reference layout), |x|^2
 int launch_multi_apply(const MultiBatch& mb, hipStream_t st);

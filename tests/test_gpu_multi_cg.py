@@ -1,0 +1,97 @@
+"""Batched CG at the edges of its kernels' tiles and splits.
+
+* A batch of one against the same step through the stored O rows (the
+  library's own gradient as callback): three CG iterations, which 64 bits
+  determine, so the two summation orders agree to rounding times the
+  amplification of three iterations.  Sizes around the 16-row and 16-site
+  tiles, the 32-site words, the 64-row sums and the 256-element slices;
+  samples around the 16-sample tiles, one slot and many, slots that hold no
+  sample, more samples in a workgroup than it has in hand.
+* The cooperative launch against the launch sequence, bit for bit, for
+  batches with fewer workgroups than the vectors want (vectors in memory) and
+  with more problems than CUs (no cooperative launch).
+"""
+import ctypes
+
+import numpy as np
+import pytest
+
+import scenarios
+from spin_based_neural_network_amd.abi import SrInfo, config_defaults, fnptr, options_defaults
+
+pytestmark = pytest.mark.gpu
+
+RBM, TFIM = 5, 0
+GRAD_CB = ctypes.CFUNCTYPE(ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
+                           ctypes.c_int, ctypes.c_void_p)
+
+
+def _problem(hip, r, N, M, B, chains, iters, seed):
+    cfg = config_defaults(ansatz=RBM, hamiltonian=TFIM, transverse_field=0.9, rbm_hidden_units=M,
+                          rbm_init_scale=0.3, num_samples=B, num_thermalize=N, num_decorrelate=2,
+                          rng_seed=seed, learning_rate=1e-2, sr_diag_shift=1e-2,
+                          sr_cg_max_iters=iters, sr_cg_tol=1e-10)
+    a = r.ansatz(cfg, N)
+    fn = fnptr(hip, "nqs_ansatz_log_amp")
+    opt = options_defaults(num_chains=chains, periodic=1)
+    s = hip.nqs_hip_sampler_create_ex(N, ctypes.byref(cfg), ctypes.byref(opt), fn, a)
+    assert s
+    return dict(cfg=cfg, N=N, a=a, s=s, fn=fn)
+
+
+def _free(hip, probs):
+    for p in probs:
+        hip.nqs_sampler_free(p["s"])
+        hip.nqs_ansatz_free(p["a"])
+
+
+@pytest.mark.parametrize("N,M,B,chains", [
+    (2, 1, 1, 1), (3, 5, 17, 17), (15, 15, 64, 16), (16, 16, 65, 13), (17, 31, 130, 10),
+    (31, 33, 1000, 100), (32, 63, 200, 50), (63, 64, 2050, 205), (64, 65, 300, 60),
+    (96, 129, 128, 64), (4, 300, 3000, 100), (128, 256, 33, 33), (200, 20, 516, 129),
+])
+def test_one_problem_equals_stored_rows(hip, N, M, B, chains):
+    print("batch of one:", N, M, B, flush=True)
+    r = scenarios.Runner(hip, "nqs_")
+    out = []
+    for rows in (False, True):
+        p = _problem(hip, r, N, M, B, chains, 3, 7 + N + M)
+        cb = GRAD_CB(lambda u, x, sp, n, g: hip.nqs_ansatz_logpsi_gradient(x, sp, n, g)) if rows else None
+        p0, info = r.params(p["a"]), SrInfo()
+        assert hip.nqs_sr_step_custom_full(ctypes.byref(p["cfg"]), N, 1, p["a"], p["s"], p["fn"],
+                                           p["a"], ctypes.cast(cb, ctypes.c_void_p), None,
+                                           ctypes.byref(info)) == 0
+        out.append((r.params(p["a"]) - p0, info.mean_energy, info.cg_iterations))
+        _free(hip, [p])
+    (got, e, it), (ref, e_ref, it_ref) = out
+    assert abs(e - e_ref) <= 1e-12 * abs(e_ref) and it == it_ref
+    # |delta| is subtracted from parameters of order 1: 2^-52 each, and the
+    # products' sums over B samples and P terms enter three times
+    tol = 3 * 2.0 ** -52 * (B + N * M) * np.abs(ref).max() + 2.0 ** -50
+    assert np.abs(got - ref).max() <= tol, (np.abs(got - ref).max(), tol)
+
+
+@pytest.mark.parametrize("n,N,M,B", [(160, 64, 64, 48), (300, 6, 8, 64), (40, 20, 90, 520)])
+def test_cooperative_launch_equals_launch_sequence(hip, n, N, M, B):
+    print("cooperative launch:", n, N, M, B, flush=True)
+    r = scenarios.Runner(hip, "nqs_")
+    params = []
+    for on in (0, 1):
+        probs = [_problem(hip, r, N + i % 2, M + i % 3, B, 16, 12, 5 + i) for i in range(n)]
+        cfgs = (type(probs[0]["cfg"]) * n)(*[p["cfg"] for p in probs])
+        lx = (ctypes.c_int * n)(*[p["N"] for p in probs])
+        ly = (ctypes.c_int * n)(*[1] * n)
+        av = (ctypes.c_void_p * n)(*[p["a"] for p in probs])
+        sv = (ctypes.c_void_p * n)(*[p["s"] for p in probs])
+        m = hip.nqs_hip_multi_create(n, cfgs, lx, ly, av, sv)
+        assert m
+        assert hip.nqs_hip_multi_use_persistent(m, on) == 0
+        info = (SrInfo * n)()
+        for _ in range(2):
+            assert hip.nqs_hip_multi_step(m, info) == 0
+        assert hip.nqs_hip_multi_sync(m) == 0
+        params.append([r.params(p["a"]) for p in probs])
+        hip.nqs_hip_multi_free(m)
+        _free(hip, probs)
+    for p, q in zip(*params):
+        assert np.array_equal(p, q)
