@@ -19,6 +19,7 @@
 #include <algorithm>
 #include <array>
 #include <atomic>
+#include <map>
 #include <mutex>
 #include <string>
 #include <type_traits>
@@ -3476,23 +3477,34 @@ void tridiag_vec(const double* d, const double* e, int K, double lam, double* z)
 }
 
 // the reference's deterministic start vector (src/mps/lanczos.c:160-176):
-// xorshift64 from seed ^ dim, element i = (x_i >> 11) / 2^53 - 1/2;
-// generated on the host in slices and uploaded
+// xorshift64 from seed ^ dim, element i = (x_i >> 11) / 2^53 - 1/2; made on
+// the device in runs, each from its own power of the generator's matrix
 int ed_seed_vector(double* d_v, long dim, unsigned long long seed) {
-  const long slice = 1L << 22;
-  std::vector<double> h((size_t)std::min(dim, slice));
-  unsigned long long x = seed ^ (unsigned long long)dim;
-  for (long s0 = 0; s0 < dim; s0 += slice) {
-    const long n = std::min(slice, dim - s0);
-    for (long i = 0; i < n; i++) {
-      x ^= x << 13;
-      x ^= x >> 7;
-      x ^= x << 17;
-      h[(size_t)i] = (double)(x >> 11) / 9007199254740992.0 - 0.5;
+  std::vector<unsigned long long> jump;
+  int nj = 0;
+  for (; nj < 32 && (1L << nj) < dim; nj++) {
+    for (int i = 0; i < 64; i++) {
+      unsigned long long x = 1ULL << i;
+      if (nj == 0) {
+        x ^= x << 13;
+        x ^= x >> 7;
+        x ^= x << 17;
+      } else {
+        const unsigned long long* m = &jump[(size_t)(nj - 1) * 64];
+        x = 0;
+        for (unsigned long long c = m[i]; c; c &= c - 1) x ^= m[__builtin_ctzll(c)];
+      }
+      jump.push_back(x);
     }
-    CK(hipMemcpyAsync(d_v + s0, h.data(), sizeof(double) * n, hipMemcpyHostToDevice, g_stream));
-    CK(hipStreamSynchronize(g_stream));
   }
+  ScopedBuf d_jump;
+  CKR(d_jump.b.ensure(sizeof(unsigned long long) * jump.size()));
+  if (nj)
+    CK(hipMemcpyAsync(d_jump.b.p, jump.data(), sizeof(unsigned long long) * jump.size(),
+                      hipMemcpyHostToDevice, g_stream));
+  CKR(nqs::launch_ed_seed(seed ^ (unsigned long long)dim, d_jump.b.as<unsigned long long>(), nj, dim, d_v,
+                          g_stream));
+  CK(hipStreamSynchronize(g_stream));
   return 0;
 }
 
@@ -3508,6 +3520,7 @@ double ed_read(const double* d) {
 struct EdHam {
   ScopedBuf bonds;
   nqs::EdOp op;
+  std::vector<std::array<int, 2>> list;
 };
 
 int ed_ham_bonds(const std::vector<std::array<int, 2>>& bl, int N, EdHam& h) {
@@ -3521,6 +3534,7 @@ int ed_ham_bonds(const std::vector<std::array<int, 2>>& bl, int N, EdHam& h) {
     CK(hipMemcpyAsync(h.bonds.b.p, flat.data(), sizeof(int) * flat.size(), hipMemcpyHostToDevice,
                       g_stream));
   CK(hipStreamSynchronize(g_stream));
+  h.list = bl;
   h.op.bonds = h.bonds.b.as<int>();
   h.op.nb = (int)bl.size();
   h.op.N = N;
@@ -3572,6 +3586,8 @@ struct EdProj {
   bool identity = true;
   int G = 1, nchunk = 0;
   ScopedBuf tab, chi;
+  std::vector<std::vector<int>> perm;   // host copies
+  std::vector<double> chars;
 };
 
 int ed_proj_build(const int* perm, const double* chars, int G, int N, const char* who,
@@ -3581,6 +3597,8 @@ int ed_proj_build(const int* perm, const double* chars, int G, int N, const char
   if (proj_tables(perm, G, N, true, who, tab, &id)) return -1;
   p.identity = id && G == 1 && chars[0] == 1.0;
   p.G = G;
+  for (int g = 0; g < G; g++) p.perm.emplace_back(perm + (size_t)g * N, perm + (size_t)(g + 1) * N);
+  p.chars.assign(chars, chars + G);
   p.nchunk = (N + 2) / 3;
   if (stream_ready()) return -1;
   CKR(p.tab.b.ensure(sizeof(unsigned long long) * tab.size()));
@@ -3870,6 +3888,228 @@ int seeded_lanczos(nqs_log_amp_fn_t fn, void* user, const EdHam& H, const EdProj
   return full_lanczos(q, out_vec, out_vals, out);
 }
 
+// One symmetry sector's orbits (k_edsym.hip)
+struct EdSector {
+  nqs::EdSym y;
+  ScopedBuf tab, chi, reps, code, len, ell, diag;
+  long R = 0;
+};
+
+// Whether H and P are what the sector path needs: the operations are a group,
+// each as often as the others, its characters are +-1 and multiply with it, and
+// the bond list is the same after every one; the tables fit the LDS, and the
+// couplings (4 bytes an orbit, bond and flipped site) fit what the four
+// full-basis vectors of the general path would take.  Operations left once
+// each in perm / chi.
+bool ed_sector_applies(const EdHam& H, const EdProj& P, int N, std::vector<std::vector<int>>& perm,
+                       std::vector<double>& chi) {
+  if (P.identity) return false;
+  std::map<std::vector<int>, std::pair<double, int>> ops;
+  for (int g = 0; g < P.G; g++) {
+    if (fabs(P.chars[g]) != 1.0) return false;
+    auto it = ops.emplace(P.perm[g], std::make_pair(P.chars[g], 0)).first;
+    if (it->second.first != P.chars[g]) return false;
+    it->second.second++;
+  }
+  const int D = (int)ops.size(), rows = (H.op.jo != 0.0 ? H.op.nb : 0) + (H.op.field != 0.0 ? N : 0);
+  if (D < 2 || rows > 8 * D || 4L * D * ((N + 2) / 3) * 8 > nqs::kEdSymLds) return false;
+  perm.clear();
+  chi.clear();
+  for (const auto& o : ops) {
+    if (o.second.second * D != P.G) return false;
+    perm.push_back(o.first);
+    chi.push_back(o.second.first);
+  }
+  std::vector<int> c(N);
+  for (const auto& a : ops)
+    for (const auto& b : ops) {
+      for (int i = 0; i < N; i++) c[i] = a.first[b.first[i]];
+      const auto it = ops.find(c);
+      if (it == ops.end() || it->second.first != a.second.first * b.second.first) return false;
+    }
+  auto sorted = [&](const std::vector<int>* p) {
+    std::vector<std::array<int, 2>> l;
+    for (const auto& e : H.list) {
+      const int u = p ? (*p)[e[0]] : e[0], v = p ? (*p)[e[1]] : e[1];
+      l.push_back({std::min(u, v), std::max(u, v)});
+    }
+    std::sort(l.begin(), l.end());
+    return l;
+  };
+  const auto bonds = sorted(nullptr);
+  for (const auto& p : perm)
+    if (sorted(&p) != bonds) return false;
+  return true;
+}
+
+int ed_sector_build(const EdHam& H, const std::vector<std::vector<int>>& perm,
+                    const std::vector<double>& chi, int N, EdSector& S) {
+  const int G = (int)perm.size();
+  const long dim = 1L << N;
+  // the longest runs of bits whose tables fit
+  int bits = 6;
+  while (bits > 3 && 4L * G * ((N + bits - 1) / bits) * (1L << bits) > nqs::kEdSymLds) bits--;
+  const int nc = (N + bits - 1) / bits;
+  std::vector<unsigned> tab((size_t)G * nc << bits, 0u);
+  for (int g = 0; g < G; g++)
+    for (int i = 0; i < N; i++) {   // bit perm[i] of s is bit i of T(g) s
+      const int j = perm[g][i], c = j / bits, b = j % bits;
+      for (int v = 0; v < 1 << bits; v++)
+        if ((v >> b) & 1) tab[((size_t)(g * nc + c) << bits) + v] |= 1u << i;
+    }
+  CKR(S.tab.b.ensure(sizeof(unsigned) * tab.size()));
+  CKR(S.chi.b.ensure(sizeof(double) * G));
+  CK(hipMemcpyAsync(S.tab.b.p, tab.data(), sizeof(unsigned) * tab.size(), hipMemcpyHostToDevice,
+                    g_stream));
+  CK(hipMemcpyAsync(S.chi.b.p, chi.data(), sizeof(double) * G, hipMemcpyHostToDevice, g_stream));
+  S.y.tab = S.tab.b.as<unsigned>();
+  S.y.chi = S.chi.b.as<double>();
+  S.y.G = G;
+  S.y.bits = bits;
+  S.y.nc = nc;
+  const long nb = nqs::ed_state_blocks(dim);
+  ScopedBuf flags, counts, first;
+  CKR(flags.b.ensure(sizeof(unsigned long long) * 64 * nb));
+  CKR(counts.b.ensure(sizeof(unsigned) * 32 * nb));
+  CKR(first.b.ensure(sizeof(unsigned) * 32 * nb));
+  CKR(nqs::launch_eds_flags(S.y, dim, flags.b.as<unsigned long long>(), counts.b.as<unsigned>(), g_stream));
+  std::vector<unsigned> n(32 * nb), at(32 * nb);
+  CK(hipMemcpyAsync(n.data(), counts.b.p, sizeof(unsigned) * 32 * nb, hipMemcpyDeviceToHost, g_stream));
+  CK(hipStreamSynchronize(g_stream));
+  S.R = 0;
+  for (int p = 0; p < 32; p++)   // by set bits, then by block
+    for (long i = 0; i < nb; i++) {
+      at[32 * i + p] = (unsigned)S.R;
+      S.R += n[32 * i + p];
+    }
+  CK(hipMemcpyAsync(first.b.p, at.data(), sizeof(unsigned) * 32 * nb, hipMemcpyHostToDevice, g_stream));
+  const size_t rows = (H.op.jo != 0.0 ? H.op.nb : 0) + (H.op.field != 0.0 ? N : 0);
+  CKR(S.reps.b.ensure(sizeof(unsigned) * S.R));
+  CKR(S.code.b.ensure(sizeof(unsigned) * dim));
+  CKR(S.len.b.ensure(sizeof(double) * S.R));
+  CKR(S.diag.b.ensure(sizeof(double) * S.R));
+  CKR(S.ell.b.ensure(sizeof(unsigned) * rows * S.R));
+  CKR(nqs::launch_eds_orbits(S.y, dim, flags.b.as<unsigned long long>(), first.b.as<unsigned>(),
+                             S.reps.b.as<unsigned>(), S.R, S.code.b.as<unsigned>(),
+                             S.len.b.as<double>(), H.op, S.ell.b.as<unsigned>(), S.diag.b.as<double>(),
+                             g_stream));
+  CK(hipStreamSynchronize(g_stream));   // at, flags, counts and first end here
+  return 0;
+}
+
+// lean_lanczos on the sector's orbits.  The next product is under way while the
+// host takes a step's alpha, beta and Ritz value; past the last step it is not used.
+int sector_lanczos(const EdHam& H, const EdSector& S, int N, int max_iters, double tol,
+                   double* out_val, double* out_vec, lanczos_result_t* out) {
+  const long dim = 1L << N, R = S.R;
+  ScopedBuf vb[5], part, scal, big;
+  for (int i = 0; i < (out_vec ? 5 : 3); i++) CKR(vb[i].b.ensure(sizeof(double) * (R + 1)));
+  CKR(part.b.ensure(sizeof(double) * nqs::ed_partials()));
+  CKR(scal.b.ensure(sizeof(double) * 8));
+  CKR(big.b.ensure(sizeof(double) * dim));
+  double *vc = vb[0].b.as<double>(), *vp = vb[1].b.as<double>(), *w = vb[2].b.as<double>();
+  double *sc = scal.b.as<double>(), *pt = part.b.as<double>();
+  const double* len = S.len.b.as<double>();
+  auto start = [&](unsigned long long seed) -> double {
+    if (ed_seed_vector(big.b.as<double>(), dim, seed) ||
+        nqs::launch_eds_restrict(S.y, S.reps.b.as<unsigned>(), R, big.b.as<double>(), len, vc, pt, sc + 1,
+                                 g_stream))
+      return NAN;
+    return ed_read(sc + 1);
+  };
+  double n2 = start(0xA5A5A5A5A5A5A5A5ULL);
+  if (!(sqrt(n2) >= 1e-14)) n2 = start(0xBEEFBABEULL);
+  if (!std::isfinite(n2)) return -1;
+  if (n2 > 0.0) CKR(nqs::launch_ed_scale(vc, vc, 1.0 / sqrt(n2), R, pt, nullptr, g_stream));
+  double* seed = out_vec ? vb[3].b.as<double>() : nullptr;
+  if (seed)
+    CK(hipMemcpyAsync(seed, vc, sizeof(double) * (R + 1), hipMemcpyDeviceToDevice, g_stream));
+  std::vector<double> alpha(max_iters), beta(max_iters + 1, 0.0), d(max_iters), e(max_iters);
+  struct Event {
+    hipEvent_t e = nullptr;
+    double* h = nullptr;
+    ~Event() {
+      if (e) (void)hipEventDestroy(e);
+      if (h) (void)hipHostFree(h);
+    }
+  } ev;
+  CK(hipEventCreateWithFlags(&ev.e, hipEventDisableTiming));
+  CK(hipHostMalloc((void**)&ev.h, 2 * sizeof(double), hipHostMallocDefault));
+  auto matvec = [&]() {
+    return nqs::launch_eds_matvec(H.op, vc, w, R, S.ell.b.as<unsigned>(), S.diag.b.as<double>(), len, pt,
+                                  sc, g_stream);
+  };
+  // w = H v_cur - alpha v_cur - beta_k v_prev and |w|^2, alpha from the product
+  auto rest = [&](int k) {
+    return nqs::launch_eds_axpy2(w, vc, sc, k > 0 ? vp : nullptr, beta[k], R, len, pt, sc + 1, g_stream);
+  };
+  double lambda = 0.0, prev = 0.0;
+  int k = 0, converged = 0, K = 0;
+  CKR(matvec());
+  for (k = 0; k < max_iters; k++) {
+    CKR(rest(k));
+    CK(hipMemcpyAsync(ev.h, sc, 2 * sizeof(double), hipMemcpyDeviceToHost, g_stream));
+    CK(hipEventRecord(ev.e, g_stream));
+    std::swap(vp, vc);   // v_prev <- v_cur, v_cur <- w / beta
+    CKR(nqs::launch_eds_unit(w, vc, sc + 1, R, g_stream));
+    if (k + 1 < max_iters) CKR(matvec());
+    CK(hipEventSynchronize(ev.e));
+    alpha[k] = ev.h[0];
+    const double b2 = ev.h[1];
+    if (!std::isfinite(alpha[k]) || !std::isfinite(b2)) {
+      (void)hipStreamSynchronize(g_stream);
+      return -1;
+    }
+    beta[k + 1] = sqrt(b2);
+    K = k + 1;
+    if (beta[k + 1] < 1e-14) {
+      k++;
+      break;
+    }
+    for (int i = 0; i < K; i++) d[i] = alpha[i];
+    for (int i = 0; i + 1 < K; i++) e[i] = beta[i + 1];
+    prev = lambda;
+    lambda = tridiag_smallest(d.data(), e.data(), K);
+    if (k > 5 && fabs(lambda - prev) < tol) {
+      converged = 1;
+      k++;
+      break;
+    }
+  }
+  CK(hipStreamSynchronize(g_stream));
+  if (!out_vec) {
+    *out_val = lambda;
+    if (out) *out = lanczos_result_t{lambda, k, converged, k > 0 ? fabs(lambda - prev) : 0.0};
+    return 0;
+  }
+  for (int i = 0; i < K; i++) d[i] = alpha[i];
+  for (int i = 0; i + 1 < K; i++) e[i] = beta[i + 1];
+  lambda = tridiag_eig(d.data(), e.data(), K, 0);
+  std::vector<double> z(K);
+  tridiag_vec(d.data(), e.data(), K, lambda, z.data());
+  double* acc = vb[4].b.as<double>();
+  CK(hipMemcpyAsync(vc, seed, sizeof(double) * (R + 1), hipMemcpyDeviceToDevice, g_stream));
+  CKR(nqs::launch_ed_scale(seed, acc, z[0], R + 1, pt, nullptr, g_stream));
+  for (int j = 0; j + 1 < K; j++) {
+    if (matvec() || rest(j)) return -1;
+    if (beta[j + 1] < 1e-14) break;
+    std::swap(vp, vc);
+    CKR(nqs::launch_eds_unit(w, vc, sc + 1, R, g_stream));
+    CKR(nqs::launch_ed_axpy2(acc, vc, -z[j + 1], nullptr, 0.0, R, pt, nullptr, g_stream));
+  }
+  double* full = big.b.as<double>();
+  CKR(nqs::launch_eds_expand(S.code.b.as<unsigned>(), acc, dim, 1.0, full, g_stream));
+  const double a2 = ed_norm2(full, dim, pt, sc);
+  if (!std::isfinite(a2)) return -1;
+  if (a2 > 0.0) CKR(nqs::launch_ed_scale(full, full, 1.0 / sqrt(a2), dim, pt, nullptr, g_stream));
+  CK(hipMemcpyAsync(out_vec, full, sizeof(double) * dim, hipMemcpyDeviceToHost, g_stream));
+  CK(hipStreamSynchronize(g_stream));
+  *out_val = lambda;
+  const double dl = fabs(lambda - prev);
+  if (out) *out = lanczos_result_t{lambda, K, (K >= 6 && dl < tol) ? 1 : 0, K >= 2 ? dl : 0.0};
+  return 0;
+}
+
 // Memory-lean projecting Lanczos (src/mps/lanczos.c:824-970): three vectors
 // and the projector's output in HBM; alpha and beta are device reductions
 // read back every step, the tridiagonal's smallest eigenvalue is taken on
@@ -3887,6 +4127,13 @@ int lean_lanczos(const EdHam& H, const EdProj& P, int N, int max_iters, double t
   const long dim = 1L << N;
   if (out) *out = lanczos_result_t{0.0, 0, 0, 0.0};
   if (max_iters > dim) max_iters = (int)dim;
+  std::vector<std::vector<int>> perm;
+  std::vector<double> chi;
+  if (ed_sector_applies(H, P, N, perm, chi)) {
+    EdSector S;
+    CKR(ed_sector_build(H, perm, chi, N, S));
+    return sector_lanczos(H, S, N, max_iters, tol, out_val, out_vec, out);
+  }
   const int nvec = out_vec ? 6 : 4;
   ScopedBuf vb[6], part, scal;
   for (int i = 0; i < nvec; i++) CKR(vb[i].b.ensure(sizeof(double) * dim));

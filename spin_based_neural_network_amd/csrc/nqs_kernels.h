@@ -343,6 +343,37 @@ int launch_ed_project(const double* in, double* out, long dim, const unsigned lo
 int launch_ed_scale(const double* x, double* y, double c, long dim, double* part, double* norm2,
                     hipStream_t st);
 int launch_ed_state_spins(long s0, long n, int N, int* out, hipStream_t st);
+// start vector: xorshift64 from x0, element i = (x_{i+1} >> 11) / 2^53 - 1/2;
+// jump: columns of the 2^k-th powers of its step's matrix, k < nj (2^nj >= dim)
+int launch_ed_seed(unsigned long long x0, const unsigned long long* jump, int nj, long dim, double* v,
+                   hipStream_t st);
+// ---- Lanczos inside a symmetry sector (k_edsym.hip) ---------------------------
+constexpr int kEdSymLds = 40 * 1024;   // tables of the operations at most
+struct EdSym {
+  const unsigned* tab = nullptr;   // device [G][nc][2^bits]: bits of T(g) s from a run of s
+  const double* chi = nullptr;     // device [G], +-1
+  int G = 0, bits = 0, nc = 0;
+};
+// workgroups of the orbit search: flags 64 words each, counts and first 32
+// entries (by number of set bits)
+long ed_state_blocks(long dim);
+int launch_eds_flags(const EdSym& y, long dim, unsigned long long* flags, unsigned* counts,
+                     hipStream_t st);
+// representatives by set bits and block (first: sums of counts), codes of all
+// states, orbit lengths, couplings [bonds, sites][R] and diagonal
+int launch_eds_orbits(const EdSym& y, long dim, const unsigned long long* flags, const unsigned* first,
+                      unsigned* reps, long R, unsigned* code, double* len, const EdOp& op, unsigned* ell,
+                      double* diag, hipStream_t st);
+// vectors of R + 1 entries, the last 0
+int launch_eds_restrict(const EdSym& y, const unsigned* reps, long R, const double* v, const double* len,
+                        double* x, double* part, double* norm2, hipStream_t st);
+int launch_eds_matvec(const EdOp& op, const double* in, double* out, long R, const unsigned* ell,
+                      const double* diag, const double* len, double* part, double* dot, hipStream_t st);
+int launch_eds_axpy2(double* w, const double* v, const double* a, const double* u, double b, long R,
+                     const double* len, double* part, double* norm2, hipStream_t st);
+int launch_eds_unit(const double* x, double* y, const double* n2, long R, hipStream_t st);
+int launch_eds_expand(const unsigned* code, const double* v, long dim, double c, double* out,
+                      hipStream_t st);
 // Krylov basis V [nv][dim]: h[j] = <V_j, w> (part: ed_mdot_partials(dim, nv)
 // doubles); w = (keep ? w : 0) - sum_j h[j] V_j, norm2 = |w|^2 when given
 size_t ed_mdot_partials(long dim, int nv);

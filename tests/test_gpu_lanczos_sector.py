@@ -1,0 +1,127 @@
+"""The lean Lanczos inside a symmetry sector against the same recurrence in
+plain numpy on the full basis (src/mps/lanczos.c:824-1130): operations that are
+a symmetry group of the bonds (orbits), the same ones listed twice, and lists
+that are not (characters that do not multiply, a missing operation, bonds that
+an open edge breaks: full basis).  States below, at and above the 64-state
+words, the 4096-state blocks and the 8192-element runs of the start vector.
+"""
+import ctypes
+
+import numpy as np
+import pytest
+
+from spin_based_neural_network_amd.abi import LanczosResult, ptr
+
+pytestmark = pytest.mark.gpu
+
+
+def _bonds(Lx, Ly, pbc):
+    """up triangle of every cell; the down triangle of cells that have both
+    neighbours"""
+    out = []
+    for x in range(Lx):
+        for y in range(Ly):
+            A = 3 * (x * Ly + y)
+            out += [(A, A + 1), (A, A + 2), (A + 1, A + 2)]
+            if pbc or (x and y):
+                B, C = 3 * ((x - 1) % Lx * Ly + y) + 1, 3 * (x * Ly + (y - 1) % Ly) + 2
+                out += [(A, B), (A, C), (B, C)]
+    return out
+
+
+def _translations(Lx, Ly, sx, sy):
+    """(perm, +-1 character) of every translation; sx, sy the step characters"""
+    out = []
+    for a in range(Lx):
+        for b in range(Ly):
+            p = [3 * (((x + a) % Lx) * Ly + (y + b) % Ly) + k
+                 for x in range(Lx) for y in range(Ly) for k in range(3)]
+            out.append((p, float(sx ** a * sy ** b)))
+    return out
+
+
+def _apply(bonds, N, v):
+    s = np.arange(v.size)
+    out = np.zeros_like(v)
+    for u, w in bonds:
+        anti = ((s >> u) ^ (s >> w)) & 1
+        out += np.where(anti, -0.25, 0.25) * v + 0.5 * anti * v[s ^ (1 << u) ^ (1 << w)]
+    return out
+
+
+def _project(ops, N, v):
+    s = np.arange(v.size)
+    out = np.zeros_like(v)
+    for p, c in ops:
+        t = np.zeros_like(s)
+        for i in range(N):
+            t |= ((s >> p[i]) & 1) << i
+        out += c * v[t]
+    return out / len(ops)
+
+
+def _seed(dim):
+    mask = (1 << 64) - 1
+    x = 0xA5A5A5A5A5A5A5A5 ^ dim
+    v = np.zeros(dim)
+    for i in range(dim):
+        x ^= (x << 13) & mask
+        x ^= x >> 7
+        x ^= (x << 17) & mask
+        v[i] = (x >> 11) / 9007199254740992.0 - 0.5
+    return v
+
+
+def _lean(bonds, ops, N, iters):
+    v = _project(ops, N, _seed(1 << N))
+    v /= np.linalg.norm(v)
+    prev, al, be = 0.0 * v, [], []
+    for k in range(iters):
+        w = _apply(bonds, N, v)
+        al.append(v @ w)
+        w = _project(ops, N, w - al[-1] * v - (be[-1] * prev if k else 0.0))
+        be.append(np.linalg.norm(w))
+        if be[-1] < 1e-14:
+            break
+        prev, v = v, w / be[-1]
+    T = np.diag(al) + np.diag(be[:len(al) - 1], 1) + np.diag(be[:len(al) - 1], -1)
+    return np.linalg.eigvalsh(T)[0]
+
+
+CASES = [
+    ("group", 2, 2, 1, _translations(2, 2, 1, 1)), ("group", 2, 2, 1, _translations(2, 2, -1, 1)),
+    ("group", 2, 2, 1, _translations(2, 2, -1, -1)), ("group", 2, 1, 1, _translations(2, 1, -1, 1)),
+    ("group", 4, 1, 1, _translations(4, 1, -1, 1)), ("group", 5, 1, 1, _translations(5, 1, 1, 1)),
+    ("twice", 2, 2, 1, _translations(2, 2, 1, -1) * 2),
+    ("uneven", 2, 2, 1, _translations(2, 2, 1, 1) + _translations(2, 2, 1, 1)[:1]),
+    ("part", 4, 1, 1, _translations(4, 1, 1, 1)[:3]),
+    ("characters", 3, 1, 1, [(p, c) for (p, _), c in zip(_translations(3, 1, 1, 1), (1., -1., 1.))]),
+    ("open", 2, 2, 0, _translations(2, 2, 1, 1)), ("few", 2, 2, 1, _translations(2, 2, 1, 1)[:2]),
+]
+
+
+@pytest.mark.parametrize("what,Lx,Ly,pbc,ops", CASES)
+def test_sector_lanczos(hip, what, Lx, Ly, pbc, ops):
+    print("sector Lanczos:", what, Lx, Ly, pbc, [c for _, c in ops], flush=True)
+    N, G = 3 * Lx * Ly, len(ops)
+    bonds = _bonds(Lx, Ly, pbc)
+    perm = np.ascontiguousarray([p for p, _ in ops], dtype=np.int32)
+    chi = np.array([c for _, c in ops])
+    # 6 sites: a few steps, before the sector's distinct levels are used up
+    for iters in (1, 2, 3 if N < 9 else 12):
+        val, res = ctypes.c_double(), LanczosResult()
+        assert hip.nqs_lanczos_e0_kagome_heisenberg_projected_lean(
+            Lx, Ly, 1.0, pbc, ptr(perm), ptr(chi), G, iters, 0.0, ctypes.byref(val),
+            ctypes.byref(res)) == 0
+        # an eigenvalue of a 12 x 12 matrix with entries summed over 2^N terms:
+        # rounding of both sides, times the norm of H
+        assert abs(val.value - _lean(bonds, ops, N, iters)) < 1e-12 * len(bonds), (iters, val.value)
+    vec = np.zeros(1 << N)
+    assert hip.nqs_lanczos_e0_kagome_heisenberg_projected_lean_eigvec(
+        Lx, Ly, 1.0, pbc, ptr(perm), ptr(chi), G, 60, 1e-13, ctypes.byref(val), ptr(vec),
+        ctypes.byref(res)) == 0
+    assert abs(np.linalg.norm(vec) - 1.0) < 1e-12
+    if what in ("group", "twice") and N > 6:
+        # converged Ritz pair of the sector
+        assert np.abs(_project(ops, N, vec) - vec).max() < 1e-12
+        assert np.linalg.norm(_apply(bonds, N, vec) - val.value * vec) < 1e-5
