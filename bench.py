@@ -202,7 +202,7 @@ SYMBOL = {"gemm_potrf": "nqs::k_gemm_big<1>", "gemm_chain": "nqs::k_gemm_lat",
           "multi_vec": "nqs::(anonymous namespace)::k_mb_phase",
           "gemm": "nqs::k_gemm_big<0>",
           "potrf_panel": "nqs::k_panel2",
-          "eloc": "nqs::k_eloc_terms<double, true>", "gen_O": "nqs::k_gen_O<double>",
+          "eloc": "nqs::k_eloc_terms<double>", "gen_O": "nqs::k_gen_O<double>",
           "colsum": "nqs::k_colsum_partial", "mh": "nqs::k_mh<double, true, 64, 4>",
           "trsv": "nqs::k_sbsv_fwd", "gram_x3": "nqs::k_gemm_x3"}
 

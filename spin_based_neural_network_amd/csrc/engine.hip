@@ -506,11 +506,72 @@ int ham_device(const nqs_config_t* cfg, int Lx, int Ly, int per, const AmpSource
   return 0;
 }
 
+// The off-diagonal terms in groups of gs that share a site (HamDev::slot_*):
+// by each pair's first site, or by the sites with the most terms left,
+// whichever takes fewer groups
+void ham_slots(const nqs::HamHost& H, int gs, std::vector<std::array<int, 3>>& best) {
+  const int nf = (int)H.flip_i.size(), np = (int)H.pair_a.size();
+  int N = H.n_sites;
+  for (int i : H.flip_i) N = std::max(N, i + 1);
+  for (int t = 0; t < np; t++) N = std::max(N, std::max(H.pair_a[t], H.pair_b[t]) + 1);
+  best.clear();
+  for (int greedy = 0; greedy < 2; greedy++) {
+    std::vector<std::vector<std::array<int, 3>>> at(N);   // (term, centre, other) by site
+    for (int t = 0; t < nf; t++) at[H.flip_i[t]].push_back({t, H.flip_i[t], -1});
+    for (int t = 0; t < np; t++) {
+      at[H.pair_a[t]].push_back({nf + t, H.pair_a[t], H.pair_b[t]});
+      if (greedy) at[H.pair_b[t]].push_back({nf + t, H.pair_b[t], H.pair_a[t]});
+    }
+    std::vector<std::array<int, 3>> slots;
+    std::vector<char> done(nf + np, 0);
+    auto take = [&](int i, size_t n) {
+      for (size_t k = 0; k < n; k++) {
+        slots.push_back(at[i][k]);
+        done[at[i][k][0]] = 1;
+      }
+      while (slots.size() % gs) slots.push_back({-1, i, -1});
+    };
+    if (!greedy) {
+      for (int i = 0; i < N; i++) take(i, at[i].size());
+    } else {
+      for (int left = nf + np; left > 0;) {
+        int i = 0;
+        for (int k = 0; k < N; k++) {
+          at[k].erase(std::remove_if(at[k].begin(), at[k].end(),
+                                     [&](const std::array<int, 3>& x) { return done[x[0]] != 0; }),
+                      at[k].end());
+          if (at[k].size() > at[i].size()) i = k;
+        }
+        const size_t n = std::min(at[i].size(), std::max<size_t>(at[i].size() / gs * gs, gs));
+        take(i, n);
+        left -= (int)n;
+      }
+    }
+    if (greedy == 0 || slots.size() < best.size()) best = slots;
+  }
+  while (best.size() % 8) best.push_back({-1, best.back()[1], -1});
+}
+
 // term lists of H (and the Marshall sublattice of src) into device buffers
 int ham_upload(const nqs::HamHost& H, const AmpSource& src, DBuf& store, DBuf& sub_store,
                nqs::HamDev& d) {
   const size_t nd = H.diag_a.size(), nf = H.flip_i.size(), np = H.pair_a.size();
-  const size_t ints = 2 * nd + nf + 2 * np + 4, dbls = nd + nf + np + 4;
+  // groups of 4, 2 or 1 terms: a slot costs two FP64 instructions and its share
+  // of four selects
+  std::vector<std::array<int, 3>> slots;
+  int gs = 1;
+  double cost = 0.0;
+  for (int g = 1; g <= 4 && nf + np > 0; g *= 2) {
+    std::vector<std::array<int, 3>> v;
+    ham_slots(H, g, v);
+    const double c = v.size() * (2.0 + 4.0 / g);
+    if (g == 1 || c < cost) {
+      cost = c;
+      gs = g;
+      slots.swap(v);
+    }
+  }
+  const size_t ints = 2 * nd + nf + 2 * np + 3 * slots.size() + 4, dbls = nd + nf + np + 4;
   CKR(store.ensure(ints * sizeof(int) + dbls * sizeof(double) + 64));
   char* base = store.as<char>();
   double* dc = (double*)base;
@@ -533,6 +594,8 @@ int ham_upload(const nqs::HamHost& H, const AmpSource& src, DBuf& store, DBuf& s
   std::copy(H.flip_i.begin(), H.flip_i.end(), hip_ + 2 * nd);
   std::copy(H.pair_a.begin(), H.pair_a.end(), hip_ + 2 * nd + nf);
   std::copy(H.pair_b.begin(), H.pair_b.end(), hip_ + 2 * nd + nf + np);
+  for (size_t i = 0; i < slots.size(); i++)
+    for (int k = 0; k < 3; k++) hip_[2 * nd + nf + 2 * np + k * slots.size() + i] = slots[i][k];
   CK(hipMemcpyAsync(base, stage.data(), stage.size(), hipMemcpyHostToDevice, g_stream));
   d = nqs::HamDev();
   d.n_diag = (int)nd;
@@ -541,6 +604,11 @@ int ham_upload(const nqs::HamHost& H, const AmpSource& src, DBuf& store, DBuf& s
   d.diag_a = da; d.diag_b = db; d.diag_c = dc;
   d.flip_i = fi; d.flip_c = fc;
   d.pair_a = pa; d.pair_b = pb; d.pair_c = pc;
+  d.n_oct = (int)(slots.size() / 8);
+  d.slot_gs = gs;
+  d.slot_t = pb + np;
+  d.slot_c = d.slot_t + slots.size();
+  d.slot_o = d.slot_c + slots.size();
   d.sublat = nullptr;
   if (src.marshall) {
     const int N = H.n_sites;

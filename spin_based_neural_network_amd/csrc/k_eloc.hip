@@ -299,12 +299,12 @@ __global__ __launch_bounds__(256) void k_eloc(ModelView<R> m, HamDev H,
 }
 
 // ---------------------------------------------------------------------------
-// Term-major local energies for many samples.  The off-diagonal terms
+// Term-major local energies for many samples (complex RBMs).  The off-diagonal terms
 // (flips, then pairs, in the Hamiltonian's order) get hidden-unit rows of
 // their own once per call, e^{d} and e^{-d} of the term for s_a = +1:
 //   flip of a:    Fp = EM_a,             Fm = EP_a
 //   pair (a, b):  Fp = EM_a EP_b,        Fm = EP_a EM_b
-// (complex products for complex RBMs); a sample with s_a = -1 swaps the two,
+// (complex products); a sample with s_a = -1 swaps the two,
 // so the factor of hidden unit h in psi(s')/psi(s) is
 //   s_a = +1: p_h Fp + q_h Fm,   s_a = -1: q_h Fp + p_h Fm.
 // A wave holds 64 samples in its lanes and 8 terms in registers; per tile of
@@ -316,7 +316,7 @@ __global__ __launch_bounds__(256) void k_eloc(ModelView<R> m, HamDev H,
 // adds the diagonal part and the contributions in term order, so E_loc sums
 // in the same order as the per-sample item lists.
 // ---------------------------------------------------------------------------
-template <typename R, bool CPLX>
+template <typename R>
 __global__ void k_term_tables(ModelView<R> m, HamDev H, int Tp, R* __restrict__ Fpr,
                               R* __restrict__ Fpi, R* __restrict__ Fmr, R* __restrict__ Fmi) {
   const int T = H.n_flip + H.n_pair, M = m.M;
@@ -327,42 +327,37 @@ __global__ void k_term_tables(ModelView<R> m, HamDev H, int Tp, R* __restrict__ 
       // padding rows: factor p + q = 1
       Fpr[e] = (R)1;
       Fmr[e] = (R)1;
-      if (CPLX) { Fpi[e] = (R)0; Fmi[e] = (R)0; }
+      Fpi[e] = (R)0;
+      Fmi[e] = (R)0;
       continue;
     }
     const int a = t < H.n_flip ? H.flip_i[t] : H.pair_a[t - H.n_flip];
     const int b = t < H.n_flip ? -1 : H.pair_b[t - H.n_flip];
     const size_t ea = (size_t)a * M + h;
     const R mar = m.EMT_re[ea], par_ = m.EPT_re[ea];
-    const R mai = CPLX ? m.EMT_im[ea] : (R)0, pai = CPLX ? m.EPT_im[ea] : (R)0;
+    const R mai = m.EMT_im[ea], pai = m.EPT_im[ea];
     if (b < 0) {
       Fpr[e] = mar;
       Fmr[e] = par_;
-      if (CPLX) { Fpi[e] = mai; Fmi[e] = pai; }
+      Fpi[e] = mai;
+      Fmi[e] = pai;
       continue;
     }
     const size_t eb = (size_t)b * M + h;
     const R pbr = m.EPT_re[eb], mbr = m.EMT_re[eb];
-    if (CPLX) {
-      const R pbi = m.EPT_im[eb], mbi = m.EMT_im[eb];
-      Fpr[e] = mar * pbr - mai * pbi;
-      Fpi[e] = mar * pbi + mai * pbr;
-      Fmr[e] = par_ * mbr - pai * mbi;
-      Fmi[e] = par_ * mbi + pai * mbr;
-    } else {
-      Fpr[e] = mar * pbr;
-      Fmr[e] = par_ * mbr;
-    }
+    const R pbi = m.EPT_im[eb], mbi = m.EMT_im[eb];
+    Fpr[e] = mar * pbr - mai * pbi;
+    Fpi[e] = mar * pbi + mai * pbr;
+    Fmr[e] = par_ * mbr - pai * mbi;
+    Fmi[e] = par_ * mbi + pai * mbr;
   }
 }
 
 constexpr int kEtTerms = 8;    // terms per wave (4 waves per workgroup)
 
-// hidden units per tile
-template <typename R, bool CPLX>
-struct EtTile { static constexpr int H = (sizeof(R) == 8 && !CPLX) ? 32 : 16; };
+constexpr int kEtH = 16;      // hidden units per tile
 
-template <typename R, bool CPLX>
+template <typename R>
 __global__ __launch_bounds__(256) void k_eloc_terms(ModelView<R> m, HamDev H,
                                                     const int* __restrict__ spins, int B,
                                                     const R* __restrict__ t_re,
@@ -374,15 +369,15 @@ __global__ __launch_bounds__(256) void k_eloc_terms(ModelView<R> m, HamDev H,
                                                     const R* __restrict__ Fmi,
                                                     double* __restrict__ res_r,
                                                     double* __restrict__ res_i) {
-  constexpr int HT = EtTile<R, CPLX>::H;
+  constexpr int HT = kEtH;
   constexpr int RS = RatioRange<R>::rescale;
   static_assert(HT % RS == 0, "tiles hold whole rescaling groups");
   constexpr int NTB = 4 * kEtTerms;                 // terms per workgroup
   __shared__ R tl_s[64][HT + 1];                     // Re t (its sign: which member)
   __shared__ R tl_r[64][HT + 1];                     // small logistic member
-  __shared__ R tl_i[CPLX ? 64 : 1][HT + 1];
+  __shared__ R tl_i[64][HT + 1];
   __shared__ R tp_r[NTB][HT], tm_r[NTB][HT];
-  __shared__ R tp_i[CPLX ? NTB : 1][HT], tm_i[CPLX ? NTB : 1][HT];
+  __shared__ R tp_i[NTB][HT], tm_i[NTB][HT];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int T = H.n_flip + H.n_pair, M = m.M, N = m.N;
@@ -422,7 +417,7 @@ __global__ __launch_bounds__(256) void k_eloc_terms(ModelView<R> m, HamDev H,
         const size_t g = (size_t)min(b0 + sm, B - 1) * M + h0 + min(hh, hn - 1);
         vts[u] = t_re[g];
         vtr[u] = q_re[g];
-        if (CPLX) vti[u] = q_im[g];
+        vti[u] = q_im[g];
       }
 #pragma unroll
       for (int u = 0; u < NQC; u++) {
@@ -430,21 +425,23 @@ __global__ __launch_bounds__(256) void k_eloc_terms(ModelView<R> m, HamDev H,
         const size_t g = (size_t)(tb0 + r) * M + h0 + min(hh, hn - 1);
         vpr[u] = Fpr[g];
         vmr[u] = Fmr[g];
-        if (CPLX) { vpi[u] = Fpi[g]; vmi[u] = Fmi[g]; }
+        vpi[u] = Fpi[g];
+        vmi[u] = Fmi[g];
       }
 #pragma unroll
       for (int u = 0; u < NQT; u++) {
         const int e = tid + 256 * u, sm = e / HT, hh = e - sm * HT;
         tl_s[sm][hh] = vts[u];
         tl_r[sm][hh] = vtr[u];
-        if (CPLX) tl_i[sm][hh] = vti[u];
+        tl_i[sm][hh] = vti[u];
       }
 #pragma unroll
       for (int u = 0; u < NQC; u++) {
         const int e = tid + 256 * u, r = e / HT, hh = e - r * HT;
         tp_r[r][hh] = vpr[u];
         tm_r[r][hh] = vmr[u];
-        if (CPLX) { tp_i[r][hh] = vpi[u]; tm_i[r][hh] = vmi[u]; }
+        tp_i[r][hh] = vpi[u];
+        tm_i[r][hh] = vmi[u];
       }
     }
     __syncthreads();
@@ -456,30 +453,25 @@ __global__ __launch_bounds__(256) void k_eloc_terms(ModelView<R> m, HamDev H,
         const int hh = g0 + u;
         if (hh >= hn) break;
         R ppr, ppi, qqr, qqi;
-        pq_of<R, CPLX>(tl_s[lane][hh], tl_r[lane][hh], CPLX ? tl_i[lane][hh] : (R)0, ppr, ppi,
-                       qqr, qqi);
+        pq_of<R, true>(tl_s[lane][hh], tl_r[lane][hh], tl_i[lane][hh], ppr, ppi, qqr, qqi);
         // term rows are padded to whole workgroups: no test on j
 #pragma unroll
         for (int j = 0; j < kEtTerms; j++) {
           const bool up = (upmask >> j) & 1u;
           const R ar = up ? ppr : qqr, ai = up ? ppi : qqi;
           const R br = up ? qqr : ppr, bi = up ? qqi : ppi;
-          if (CPLX) {
-            const R fpr = tp_r[rw + j][hh], fpi = tp_i[rw + j][hh];
-            const R fmr = tm_r[rw + j][hh], fmi = tm_i[rw + j][hh];
-            const R wr = (ar * fpr - ai * fpi) + (br * fmr - bi * fmi);
-            const R wi = (ar * fpi + ai * fpr) + (br * fmi + bi * fmr);
-            const R nr = pr[j] * wr - pim[j] * wi;
-            pim[j] = pr[j] * wi + pim[j] * wr;
-            pr[j] = nr;
-          } else {
-            pr[j] *= ar * tp_r[rw + j][hh] + br * tm_r[rw + j][hh];
-          }
+          const R fpr = tp_r[rw + j][hh], fpi = tp_i[rw + j][hh];
+          const R fmr = tm_r[rw + j][hh], fmi = tm_i[rw + j][hh];
+          const R wr = (ar * fpr - ai * fpi) + (br * fmr - bi * fmi);
+          const R wi = (ar * fpi + ai * fpr) + (br * fmi + bi * fmr);
+          const R nr = pr[j] * wr - pim[j] * wi;
+          pim[j] = pr[j] * wi + pim[j] * wr;
+          pr[j] = nr;
         }
       }
       // rescale by a power of two (exact)
 #pragma unroll
-      for (int j = 0; j < kEtTerms; j++) rescale2<R, CPLX>(pr[j], pim[j], ex[j]);
+      for (int j = 0; j < kEtTerms; j++) rescale2<R, true>(pr[j], pim[j], ex[j]);
     }
   }
   if (b0 + lane >= B) return;
@@ -497,22 +489,20 @@ __global__ __launch_bounds__(256) void k_eloc_terms(ModelView<R> m, HamDev H,
     const int bb = t < H.n_flip ? -1 : H.pair_b[t - H.n_flip];
     const double s_a = ((upmask >> j) & 1u) ? 1.0 : -1.0;
     double vr = -2.0 * (double)m.a_re[a] * s_a;
-    double vi = CPLX ? -2.0 * (double)m.a_im[a] * s_a : 0.0;
+    double vi = -2.0 * (double)m.a_im[a] * s_a;
     if (bb >= 0) {
       vr += 2.0 * (double)m.a_re[bb] * s_a;
-      if (CPLX) vi += 2.0 * (double)m.a_im[bb] * s_a;
+      vi += 2.0 * (double)m.a_im[bb] * s_a;
     }
-    const double xr = (double)pr[j], xi = CPLX ? (double)pim[j] : 0.0;
-    const double mg = CPLX ? sqrt(xr * xr + xi * xi) : fabs(xr);
+    const double xr = (double)pr[j], xi = (double)pim[j];
+    const double mg = sqrt(xr * xr + xi * xi);
     // a zero factor (psi(s') = 0) contributes nothing
     const double lm = mg > 0.0 ? log(mg) + (double)ex[j] * 0.69314718055994530942 : -INFINITY;
     double ph_r = mg > 0.0 ? xr / mg : 0.0, ph_i = mg > 0.0 ? xi / mg : 0.0;
-    if (CPLX) {
-      const double c = cos(vi), sn = sin(vi);
-      const double nr = ph_r * c - ph_i * sn;
-      ph_i = ph_r * sn + ph_i * c;
-      ph_r = nr;
-    }
+    const double c = cos(vi), sn = sin(vi);
+    const double nr = ph_r * c - ph_i * sn;
+    ph_i = ph_r * sn + ph_i * c;
+    ph_r = nr;
     const double mag = exp(lm + vr);
     double sign = 1.0;
     if (H.sublat) {
@@ -525,25 +515,274 @@ __global__ __launch_bounds__(256) void k_eloc_terms(ModelView<R> m, HamDev H,
   }
 }
 
-// E_loc(b) = diagonal part + sum over terms in order of res[t][b]
+// ---------------------------------------------------------------------------
+// The same contributions for real RBMs with less arithmetic.  With d the change
+// of theta for s_c = +1 (c: one of the term's sites) and E = e^{2d},
+//   s_c = +1: p e^d + q e^-d = e^-d (q + p E),   s_c = -1: e^-d (p + q E),
+// so a factor is one fused multiply-add of positive numbers that lies between
+// 1 and E, and the product of the e^-d is one number per term.  Terms sit in
+// octets (a wave's), in each octet groups of GS with one site c: p and q are
+// put in the order that s_c asks for once per group.  A lane has S samples for
+// which it uses an E that it has read; E and, [hidden unit][sample], p and q of
+// the workgroup's samples are staged in LDS.
+// The products are rescaled when the sum of the units' largest |log E| (bound,
+// per RG units) says that they could leave the type's range, for ordinary
+// weights once or twice.
+// What bounds it: vector issue, two FP64 instructions a factor and 4 / GS
+// selects of 32 bits (73 % of the issue cycles).  100 sites, 400 pairs, 800
+// hidden units, 16384 samples: 823 us, 1945 as k_eloc_terms had them (12
+// instructions a factor).
+// ---------------------------------------------------------------------------
+template <typename R>
+struct SlotRange;
+template <>
+struct SlotRange<double> { static constexpr int RG = 4; static constexpr double limit = 640.0; };
+template <>
+struct SlotRange<float> { static constexpr int RG = 1; static constexpr double limit = 80.0; };
+constexpr int kSlotH = 8;      // hidden units per tile
+constexpr int kSlotWaves = 4;
+
+static inline int slot_units(int M) { return (M + kSlotH - 1) / kSlotH * kSlotH; }
+
+// E [octet][unit][8], bound [octet][unit / RG]; the products of the e^-d as
+// mantissas cst [octet][0..7] and powers of two cst [octet][8..15];
+// a workgroup per octet, threads over the units (1 and 0 past them)
+template <typename R>
+__global__ __launch_bounds__(512) void k_slot_tables(ModelView<R> m, HamDev H, int Mp, R* __restrict__ E,
+                                                     double* __restrict__ bound,
+                                                     double* __restrict__ cst) {
+  constexpr int RG = SlotRange<R>::RG;
+  __shared__ double part[8][8];
+  __shared__ int pex[8][8];
+  const int o = blockIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63, M = m.M;
+  double c[8];
+  int ce[8];
+#pragma unroll
+  for (int j = 0; j < 8; j++) {
+    c[j] = 1.0;
+    ce[j] = 0;
+  }
+  for (int h = threadIdx.x; h < ((Mp + 511) & ~511); h += 512) {
+    double big = 0.0, d[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+      const int t = H.slot_t[o * 8 + j], s = H.slot_c[o * 8 + j], x = H.slot_o[o * 8 + j];
+      d[j] = 0.0;
+      if (t >= 0 && h < M)
+        d[j] = 2.0 * ((x >= 0 ? (double)m.WT_re[(size_t)x * M + h] : 0.0) - (double)m.WT_re[(size_t)s * M + h]);
+      int e2;
+      c[j] = frexp(c[j] * exp(-d[j]), &e2);
+      ce[j] += e2;
+      big = fmax(big, fabs(2.0 * d[j]));
+    }
+    if (h < Mp) {
+#pragma unroll
+      for (int j = 0; j < 8; j++) E[((size_t)o * Mp + h) * 8 + j] = (R)exp(2.0 * d[j]);
+    }
+    // over RG neighbouring units
+#pragma unroll
+    for (int k = 1; k < RG; k <<= 1) big += __shfl_xor(big, k, 64);
+    if (h < Mp && h % RG == 0) bound[((size_t)o * Mp + h) / RG] = big;
+  }
+#pragma unroll
+  for (int j = 0; j < 8; j++) {
+#pragma unroll
+    for (int k = 32; k >= 1; k >>= 1) {
+      c[j] *= __shfl_xor(c[j], k, 64);
+      ce[j] += __shfl_xor(ce[j], k, 64);
+    }
+    if (lane == 0) {
+      part[j][wave] = c[j];
+      pex[j][wave] = ce[j];
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x < 8) {
+    double v = 1.0;
+    int e = 0, e2;
+    for (int w = 0; w < 8; w++) {
+      v *= part[threadIdx.x][w];
+      e += pex[threadIdx.x][w];
+    }
+    v = frexp(v, &e2);
+    cst[o * 16 + threadIdx.x] = v;
+    cst[o * 16 + 8 + threadIdx.x] = (double)(e + e2);
+  }
+}
+
+template <typename R, int GS, int S>
+__global__ __launch_bounds__(64 * kSlotWaves) void k_eloc_slots(
+    ModelView<R> m, HamDev H, const int* __restrict__ spins, int B, const R* __restrict__ t_re,
+    const R* __restrict__ q_re, int Mp, const R* __restrict__ E, const double* __restrict__ bound,
+    const double* __restrict__ cst, double* __restrict__ res_r, double* __restrict__ res_i) {
+  constexpr int NG = 8 / GS, NS = 64 * S, LD = NS + 2;
+  constexpr int RG = SlotRange<R>::RG, NT = 64 * kSlotWaves, NL = NS * kSlotH / NT;
+  __shared__ R P[kSlotH][LD], Q[kSlotH][LD];
+  __shared__ R Es[kSlotWaves][kSlotH][8];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int N = m.N, M = m.M, b0 = blockIdx.x * NS;
+  const int o = blockIdx.y * kSlotWaves + wave;
+  const bool live = o < H.n_oct;
+  const int oc = live ? o : H.n_oct - 1;
+  bool up[NG][S];
+#pragma unroll
+  for (int g = 0; g < NG; g++) {
+    const int c = H.slot_c[oc * 8 + g * GS];
+#pragma unroll
+    for (int k = 0; k < S; k++) {
+      const int b = b0 + k * 64 + lane;
+      up[g][k] = spins[(size_t)(b < B ? b : B - 1) * N + c] > 0;
+    }
+  }
+  R acc[8][S];
+  int ex[8][S];
+#pragma unroll
+  for (int j = 0; j < 8; j++)
+#pragma unroll
+    for (int k = 0; k < S; k++) {
+      acc[j][k] = (R)1;
+      ex[j][k] = 0;
+    }
+  static_assert(kSlotH == 8, "one E a thread");
+  const R* __restrict__ Eo = E + (size_t)oc * Mp * 8 + lane;
+  const double* __restrict__ bo = bound + (size_t)oc * (Mp / RG);
+  double run = 0.0;
+  R vt[NL], vq[NL], ve = (R)0;
+  auto fetch = [&](int h0) {
+#pragma unroll
+    for (int u = 0; u < NL; u++) {
+      const int e = tid + NT * u, sm = e / kSlotH, h = h0 + e % kSlotH, b = b0 + sm;
+      const size_t g = (size_t)(b < B ? b : B - 1) * M + (h < M ? h : M - 1);
+      vt[u] = t_re[g];
+      vq[u] = q_re[g];
+    }
+    ve = Eo[(size_t)h0 * 8];
+  };
+  if (M > 0) fetch(0);
+  for (int h0 = 0; h0 < Mp; h0 += kSlotH) {
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < NL; u++) {
+      const int e = tid + NT * u, sm = e / kSlotH, hh = e % kSlotH;
+      R pr, pi, qr, qi;
+      pq_of<R, false>(vt[u], vq[u], (R)0, pr, pi, qr, qi);
+      const bool in = h0 + hh < M;   // past the last unit: factor 1
+      P[hh][sm] = in ? pr : (R)1;
+      Q[hh][sm] = in ? qr : (R)0;
+    }
+    Es[wave][lane >> 3][lane & 7] = ve;
+    __syncthreads();
+    if (h0 + kSlotH < Mp) fetch(h0 + kSlotH);
+#pragma unroll
+    for (int r = 0; r < kSlotH; r += RG) {
+      const double nb = bo[(h0 + r) / RG];
+      run += nb;
+      if (run > SlotRange<R>::limit) {
+        run = nb;
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+#pragma unroll
+          for (int k = 0; k < S; k++) {
+            int e2;
+            acc[j][k] = frexp(acc[j][k], &e2);
+            ex[j][k] += e2;
+          }
+      }
+#pragma unroll
+      for (int u = 0; u < RG; u++) {
+        const R* Eh = Es[wave][r + u];
+        R p[S], q[S];
+#pragma unroll
+        for (int k = 0; k < S; k++) {
+          p[k] = P[r + u][k * 64 + lane];
+          q[k] = Q[r + u][k * 64 + lane];
+        }
+#pragma unroll
+        for (int g = 0; g < NG; g++) {
+#pragma unroll
+          for (int k = 0; k < S; k++) {
+            const R x = up[g][k] ? p[k] : q[k], y = up[g][k] ? q[k] : p[k];
+#pragma unroll
+            for (int j = g * GS; j < g * GS + GS; j++) acc[j][k] *= fma(x, Eh[j], y);
+          }
+        }
+      }
+    }
+  }
+  if (!live) return;
+#pragma unroll
+  for (int j = 0; j < 8; j++) {
+    const int t = H.slot_t[o * 8 + j];
+    if (t < 0) continue;
+    const int c = H.slot_c[o * 8 + j], x = H.slot_o[o * 8 + j];
+    const double coef = t < H.n_flip ? H.flip_c[t] : H.pair_c[t - H.n_flip];
+    double sign = 1.0;
+    if (H.sublat && ((H.sublat[c] + (x >= 0 ? H.sublat[x] : 0)) & 1)) sign = -1.0;
+    const double ac = (double)m.a_re[c], ax = x >= 0 ? (double)m.a_re[x] : 0.0, cm = cst[o * 16 + j], cx = cst[o * 16 + 8 + j];
+#pragma unroll
+    for (int k = 0; k < S; k++) {
+      const int b = b0 + k * 64 + lane;
+      if (b >= B) continue;
+      const double s_c = up[j / GS][k] ? 1.0 : -1.0;
+      const size_t at = (size_t)t * B + b;
+      if (res_i) res_i[at] = 0.0;
+      if (x >= 0 && (spins[(size_t)b * N + x] > 0) == up[j / GS][k]) {
+        res_r[at] = 0.0;
+        continue;
+      }
+      const double vr = -2.0 * ac * s_c + 2.0 * ax * s_c;
+      const double v = (double)acc[j][k] * cm;
+      // a zero factor (psi(s') = 0) contributes nothing
+      const double lm = v > 0.0 ? log(v) + ((double)ex[j][k] + cx) * 0.69314718055994530942 : -INFINITY;
+      res_r[at] = coef * sign * exp(lm + vr);
+    }
+  }
+}
+
+// E_loc(b) = diagonal part + sum over terms in order of res[t][b] (res_i null:
+// real amplitudes).  Four waves fetch 128 terms of 64 samples at a time, the
+// first adds them: one wave's own loads took 269 us for 400 terms and 16384
+// samples.
 __global__ __launch_bounds__(256) void k_eloc_terms_sum(HamDev H, const int* __restrict__ spins,
                                                         int B, int N,
                                                         const double* __restrict__ res_r,
                                                         const double* __restrict__ res_i,
                                                         double* __restrict__ e_re,
                                                         double* __restrict__ e_im) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= B) return;
-  const int* s = spins + (size_t)b * N;
-  double diag = 0.0;
-  for (int d = 0; d < H.n_diag; d++)
-    diag += H.diag_c[d] * (double)(s[H.diag_a[d]] * s[H.diag_b[d]]);
+  __shared__ double v[128][64];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int b = blockIdx.x * 64 + lane, bc = b < B ? b : B - 1;
   const int T = H.n_flip + H.n_pair;
-  double orr = 0.0, oi = 0.0;
-  for (int t = 0; t < T; t++) {
-    orr += res_r[(size_t)t * B + b];
-    oi += res_i[(size_t)t * B + b];
-  }
+  const int* sp = spins + (size_t)bc * N;
+  // sum over i < n in order of at(i), which the four waves evaluate
+  auto sum = [&](int n, auto at) {
+    double s = 0.0;
+    for (int t0 = 0; t0 < n; t0 += 128) {
+      double r[32];
+#pragma unroll
+      for (int u = 0; u < 32; u++) {
+        const int t = t0 + wave * 32 + u;
+        r[u] = at(t < n ? t : n - 1);
+      }
+      __syncthreads();
+#pragma unroll
+      for (int u = 0; u < 32; u++) v[wave * 32 + u][lane] = r[u];
+      __syncthreads();
+      if (wave == 0) {
+        const int m = n - t0 < 128 ? n - t0 : 128;
+#pragma unroll 8
+        for (int u = 0; u < m; u++) s += v[u][lane];
+      }
+    }
+    return s;
+  };
+  const double orr = sum(T, [&](int t) { return res_r[(size_t)t * B + bc]; });
+  const double oi = res_i ? sum(T, [&](int t) { return res_i[(size_t)t * B + bc]; }) : 0.0;
+  const double diag = sum(H.n_diag, [&](int d) {
+    return H.diag_c[d] * (double)(sp[H.diag_a[d]] * sp[H.diag_b[d]]);
+  });
+  if (wave != 0 || b >= B) return;
   e_re[b] = diag + orr;
   if (e_im) e_im[b] = oi;
 }
@@ -551,10 +790,42 @@ __global__ __launch_bounds__(256) void k_eloc_terms_sum(HamDev H, const int* __r
 // term rows padded to whole workgroups (4 waves x 16 terms)
 static inline int padded_terms(int T) { return (T + 4 * kEtTerms - 1) / (4 * kEtTerms) * (4 * kEtTerms); }
 
+// E, bound and cst
+template <typename R>
+static size_t slot_bytes(const HamDev& h, int M) {
+  const size_t Mp = slot_units(M);
+  return sizeof(R) * h.n_oct * Mp * 8 + 256 + sizeof(double) * (h.n_oct * (Mp / SlotRange<R>::RG) + 16 * h.n_oct);
+}
+
+template <typename R, int GS, int S>
+static void slots_go(const ModelView<R>& m, const HamDev& h, const int* spins, int B, const R* t_re,
+                     const R* q_re, const R* E, const double* bound, const double* cst, double* res_r,
+                     double* res_i, hipStream_t st) {
+  const dim3 grid((B + 64 * S - 1) / (64 * S), (h.n_oct + kSlotWaves - 1) / kSlotWaves);
+  hipLaunchKernelGGL((k_eloc_slots<R, GS, S>), grid, dim3(64 * kSlotWaves), 0, st, m, h, spins, B, t_re,
+                     q_re, slot_units(m.M), E, bound, cst, res_r, res_i);
+}
+
+// Two samples a lane where that leaves two workgroups for every CU (100 sites,
+// 16384 samples: 823 us; four samples with half the waves 1010, workgroups of
+// eight waves 870)
+template <typename R>
+static void slots_any(const ModelView<R>& m, const HamDev& h, const int* spins, int B, const R* t_re,
+                      const R* q_re, const R* E, const double* bound, const double* cst, double* res_r,
+                      double* res_i, hipStream_t st) {
+  const bool two = (long)((B + 127) / 128) * ((h.n_oct + kSlotWaves - 1) / kSlotWaves) >= 512;
+#define NQS_SLOTS(G, K) slots_go<R, G, K>(m, h, spins, B, t_re, q_re, E, bound, cst, res_r, res_i, st)
+  if (h.slot_gs == 4) two ? NQS_SLOTS(4, 2) : NQS_SLOTS(4, 1);
+  else if (h.slot_gs == 2) two ? NQS_SLOTS(2, 2) : NQS_SLOTS(2, 1);
+  else two ? NQS_SLOTS(1, 2) : NQS_SLOTS(1, 1);
+#undef NQS_SLOTS
+}
+
 template <typename R>
 size_t eloc_ws_bytes(const ModelView<R>& m, const HamDev& h, int B) {
   const size_t T = (size_t)(h.n_flip + h.n_pair);
-  const size_t tab = (size_t)padded_terms((int)T) * (size_t)m.M * sizeof(R) * (m.cplx ? 4 : 2);
+  const size_t tab = m.cplx ? (size_t)padded_terms((int)T) * (size_t)m.M * sizeof(R) * 4
+                            : slot_bytes<R>(h, m.M);
   return ((tab + 255) & ~(size_t)255) + 2 * T * (size_t)B * sizeof(double) + 256;
 }
 
@@ -565,28 +836,37 @@ template <typename R, bool CPLX>
 static int eloc_terms_go(const ModelView<R>& m, const HamDev& h, const int* spins, int B,
                          const R* t_re, const R* q_re, const R* q_im, double* e_re, double* e_im,
                          void* ws, hipStream_t st, double** res_out = nullptr) {
-  const int T = h.n_flip + h.n_pair, M = m.M, Tp = padded_terms(T);
-  const size_t TM = (size_t)Tp * M;
+  const int T = h.n_flip + h.n_pair, M = m.M;
   unsigned char* p = (unsigned char*)ws;
-  R* Fpr = (R*)p;
-  R* Fmr = Fpr + TM;
-  R* Fpi = CPLX ? Fmr + TM : nullptr;
-  R* Fmi = CPLX ? Fpi + TM : nullptr;
-  const size_t tab = TM * sizeof(R) * (CPLX ? 4 : 2);
+  const size_t tab = CPLX ? (size_t)padded_terms(T) * M * sizeof(R) * 4 : slot_bytes<R>(h, M);
   double* res_r = (double*)(p + ((tab + 255) & ~(size_t)255));
   double* res_i = res_r + (size_t)T * B;
   KScope ks("eloc", st);
-  if (T > 0) {
+  if constexpr (CPLX) {
+    const int Tp = padded_terms(T);
+    const size_t TM = (size_t)Tp * M;
+    R *Fpr = (R*)p, *Fmr = Fpr + TM, *Fpi = Fmr + TM, *Fmi = Fpi + TM;
     if (TM > 0) {
       long blocks = ((long)TM + 255) / 256;
       if (blocks > 4096) blocks = 4096;
-      hipLaunchKernelGGL((k_term_tables<R, CPLX>), dim3((unsigned)blocks), dim3(256), 0, st, m, h,
-                         Tp, Fpr, Fpi, Fmr, Fmi);
+      hipLaunchKernelGGL((k_term_tables<R>), dim3((unsigned)blocks), dim3(256), 0, st, m, h, Tp, Fpr,
+                         Fpi, Fmr, Fmi);
       count_launch();
     }
-    const dim3 grid((B + 63) / 64, Tp / (4 * kEtTerms));
-    hipLaunchKernelGGL((k_eloc_terms<R, CPLX>), grid, dim3(256), 0, st, m, h, spins, B, t_re, q_re,
-                       q_im, Fpr, Fpi, Fmr, Fmi, res_r, res_i);
+    if (T > 0) {
+      const dim3 grid((B + 63) / 64, Tp / (4 * kEtTerms));
+      hipLaunchKernelGGL((k_eloc_terms<R>), grid, dim3(256), 0, st, m, h, spins, B, t_re, q_re, q_im,
+                         Fpr, Fpi, Fmr, Fmi, res_r, res_i);
+      count_launch();
+    }
+  } else if (T > 0) {
+    const int Mp = slot_units(M);
+    R* E = (R*)p;
+    double* bound = (double*)(p + ((sizeof(R) * h.n_oct * Mp * 8 + 255) & ~(size_t)255));
+    double* cst = bound + (size_t)h.n_oct * (Mp / SlotRange<R>::RG);
+    hipLaunchKernelGGL((k_slot_tables<R>), dim3(h.n_oct), dim3(512), 0, st, m, h, Mp, E, bound, cst);
+    count_launch();
+    slots_any<R>(m, h, spins, B, t_re, q_re, E, bound, cst, res_r, res_out ? res_i : nullptr, st);
     count_launch();
   }
   if (res_out) {
@@ -594,8 +874,8 @@ static int eloc_terms_go(const ModelView<R>& m, const HamDev& h, const int* spin
     res_out[1] = res_i;
   }
   if (e_re) {
-    hipLaunchKernelGGL(k_eloc_terms_sum, dim3((B + 255) / 256), dim3(256), 0, st, h, spins, B,
-                       m.N, res_r, res_i, e_re, e_im);
+    hipLaunchKernelGGL(k_eloc_terms_sum, dim3((B + 63) / 64), dim3(256), 0, st, h, spins, B,
+                       m.N, res_r, CPLX ? res_i : nullptr, e_re, e_im);
     count_launch();
   }
   NQS_HIP_CHECK(hipGetLastError());

@@ -66,6 +66,11 @@ struct HamDev {
   const int* pair_b = nullptr;
   const double* pair_c = nullptr;
   const signed char* sublat = nullptr;  // Marshall: 1 on sublattice A, or null
+  // off-diagonal terms (flips, then pairs) in octets, each octet in groups of
+  // slot_gs terms that share the site slot_c; slot_o: the pair's other site, -1
+  // for a flip; slot_t: the term, -1 for none
+  int n_oct = 0, slot_gs = 1;
+  const int *slot_t = nullptr, *slot_c = nullptr, *slot_o = nullptr;
 };
 
 // Metropolis chain state on the device.
