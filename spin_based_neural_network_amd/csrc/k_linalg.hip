@@ -779,7 +779,9 @@ static int gemm_chain(int M, int N, int K, const double* A, long lda, double* C,
 // is updated.  The inverses of the 64x64 diagonal blocks are kept for the
 // triangular solves.
 // --------------------------------------------------------------------------
-constexpr int NB = 64, NBO = 128;
+// LD: LDS row stride of a block; 2 mod 4 doubles, so that an MFMA operand (16
+// rows of 4) takes every bank pair twice
+constexpr int NB = 64, NBO = 128, LD = NB + 2;
 
 // Linv workspace (potrf_linv_elems): the inverses of the 64 x 64 diagonal
 // blocks, then the blocks' L (written by the panel kernel and copied into A
@@ -805,86 +807,21 @@ __device__ __attribute__((always_inline)) inline double rsqrt_nr(double d) {
   return fma(0.5 * y, e, y);
 }
 
-// Step 2 of a panel: D = L L^T by blocks of 16 columns.  Wave jb factors
-// its own 16 columns with the rows in its lanes (only 1/pivot is on the
-// column chain, L_ij = a_ij / sqrt(d) is formed after the update; each
-// column is broadcast through the wave's own LDS row), publishes them
-// through D, and every later wave subtracts the rank-16 product from its own
-// columns.  Returns the first column whose pivot is not positive, or nb.
-// Called by all 256 threads.
-__device__ __attribute__((always_inline)) inline int panel_factor(double (*D)[NB + 1], double (*colw)[NB], int* s_fail, int nb,
-                                   int wave, int lane) {
-  double rr[16];
-#pragma unroll
-  for (int t = 0; t < 16; t++) rr[t] = D[lane][16 * wave + t];
-  int jdone = nb;
-  for (int jb = 0; jb < 4 && 16 * jb < nb; jb++) {
-    if (wave == jb) {
-      // straight-line code (selects instead of branches) so that the
-      // square roots and scalings of column j overlap the chain of j + 1.
-      // The wave's LDS accesses complete in issue order, and the wavefront
-      // fence keeps the compiler from moving the reads above the write.
-      int jf = nb;
-#pragma unroll
-      for (int jj = 0; jj < 16; jj++) {
-        const int j = 16 * jb + jj;
-        const double ci = rr[jj];
-        colw[wave][lane] = ci;
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        const double d = colw[wave][j];
-        const bool live = j < nb && jf == nb;
-        const bool ok = live && d > 0.0;
-        jf = (live && !ok) ? j : jf;
-        const double rd = recip_nr(d);
-        const double si = (ok && lane > j) ? ci * rd : 0.0;
-#pragma unroll
-        for (int t = jj + 1; t < 16; t++) rr[t] -= si * colw[wave][16 * jb + t];
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        const double rs = rsqrt_nr(d);
-        rr[jj] = !ok ? ci : ((lane == j) ? d * rs : ((lane > j) ? ci * rs : ci));
-      }
-#pragma unroll
-      for (int t = 0; t < 16; t++) D[lane][16 * jb + t] = rr[t];
-      if (lane == 0) *s_fail = jf;
-    }
-    __syncthreads();
-    jdone = *s_fail;
-    if (jdone < nb) break;
-    if (wave > jb) {
-      double lp[16];
-#pragma unroll
-      for (int jj = 0; jj < 16; jj++) lp[jj] = D[lane][16 * jb + jj];
-#pragma unroll
-      for (int t = 0; t < 16; t++) {
-        const int c = 16 * wave + t;
-        double a0 = 0.0, a1 = 0.0;
-#pragma unroll
-        for (int jj = 0; jj < 16; jj += 2) {
-          a0 += lp[jj] * D[c][16 * jb + jj];
-          a1 += lp[jj + 1] * D[c][16 * jb + jj + 1];
-        }
-        rr[t] -= a0 + a1;
-      }
-    }
-  }
-#pragma unroll
-  for (int t = 0; t < 16; t++) D[lane][16 * wave + t] = rr[t];
-  __syncthreads();
-  return jdone;
+// v of lane l, in scalar registers
+__device__ __attribute__((always_inline)) inline double lane_value(double v, int l) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l),
+                          __builtin_amdgcn_readlane(__double2loint(v), l));
 }
 
-// Step 3: X = L^-1 by 16 x 16 blocks.  (a) wave w inverts diagonal block w
-// (lane c < 16 solves L_ww x = e_c with reciprocal pivots); (b) one block
-// diagonal at a time, X_ij = -X_ii sum_{k=j}^{i-1} L_ik X_kj, the blocks of a
-// diagonal on separate waves (two MFMA products each).  Rows beyond nb are
-// identity rows of L, so their part of X is the identity.  All 256 threads.
-__device__ __attribute__((always_inline)) inline void panel_inverse(double (*D)[NB + 1], double (*X)[NB + 1], double* rcp,
-                                     int wave, int lane, int tid) {
-  for (int e = tid; e < NB * NB; e += 256) X[e >> 6][e & 63] = 0.0;
-  if (tid < NB) rcp[tid] = 1.0 / D[tid][tid];
-  __syncthreads();
+// Inverse of the 16 x 16 diagonal block w of D into X by one wave (lane c < 16
+// solves L_ww x = e_c with reciprocal pivots)
+__device__ __attribute__((always_inline)) inline void block_inverse(double (*D)[LD], double (*X)[LD],
+                                                                    double* rcp, int w, int lane) {
+  if (lane < 16) rcp[16 * w + lane] = 1.0 / D[16 * w + lane][16 * w + lane];
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  __builtin_amdgcn_wave_barrier();
   if (lane < 16) {
-    const int b0 = 16 * wave, c = lane;
+    const int b0 = 16 * w, c = lane;
     double x[16];
 #pragma unroll
     for (int q = 0; q < 16; q++) {
@@ -899,7 +836,117 @@ __device__ __attribute__((always_inline)) inline void panel_inverse(double (*D)[
 #pragma unroll
     for (int q = 0; q < 16; q++) X[b0 + q][b0 + c] = x[q];
   }
-  __syncthreads();
+}
+
+// Step 2 of a panel: D = L L^T by blocks of 16 columns.  Wave jb factors
+// its own 16 columns with the rows in its lanes (only 1/pivot is on the
+// column chain, L_ij = a_ij / sqrt(d) is formed after the update; the
+// column's entries reach all lanes as scalars) and publishes them through D;
+// the four waves then subtract the rank-16 product from the 16 x 16 tiles
+// right of and below them on MFMA.  Returns the first column whose pivot is
+// not positive, or nb.  X is cleared and gets the inverses of the diagonal
+// blocks, each from the wave that has factored it, beside the next wave's
+// columns.  Called by all 256 threads.
+// What bounds it: the issue of the column chain, 64 x 180 ns (270 with the
+// column through LDS and the updates of later columns on the vector units); an
+// outer panel of 128 columns at n = 512 takes 53 us, 60 before.
+__device__ __attribute__((always_inline)) inline int panel_factor(double (*D)[LD], double (*X)[LD],
+                                                                  double* rcp, int* s_fail, int nb,
+                                                                  int wave, int lane) {
+  const int lr = lane & 15, lk = lane >> 4;
+  int jdone = nb;
+  for (int e = threadIdx.x; e < NB * NB; e += 256) X[e >> 6][e & 63] = 0.0;
+  for (int jb = 0; jb < 4 && 16 * jb < nb; jb++) {
+    if (wave == jb) {
+      double rr[16];
+#pragma unroll
+      for (int t = 0; t < 16; t++) rr[t] = D[lane][16 * jb + t];
+      // straight-line code (selects instead of branches); the square roots of
+      // the 16 pivots are taken together afterwards, a pivot in a lane
+      int jf = nb;
+      double piv = 1.0;
+      double d = lane_value(rr[0], 16 * jb);
+      asm("" : "+v"(d));   // a vector value: no branches on it
+      double rd = recip_nr(d);
+#pragma unroll
+      for (int jj = 0; jj < 16; jj++) {
+        const int j = 16 * jb + jj;
+        const double ci = rr[jj];
+        const bool live = j < nb && jf == nb;
+        const bool ok = live && d > 0.0;
+        jf = (live && !ok) ? j : jf;
+        piv = (lane & 15) == jj ? d : piv;
+        const double si = (ok && lane > j) ? ci * rd : 0.0;
+        auto update = [&](int t) {
+          rr[t] -= si * lane_value(ci, 16 * jb + t);
+          asm("" : "+v"(rr[t]));   // now, not when column t is reached
+        };
+        if (jj == 15) break;
+        // the next pivot's reciprocal (recip_nr) between the updates of the
+        // columns after it
+        update(jj + 1);
+        d = lane_value(rr[jj + 1], j + 1);
+        asm("" : "+v"(d));
+        double e;
+#pragma unroll
+        for (int q = 0; q < 5; q++) {
+          if (q == 0) rd = __builtin_amdgcn_rcp(d);
+          else if (q & 1) e = fma(-d, rd, 1.0);
+          else rd = fma(rd, e, rd);
+#pragma unroll
+          for (int t = jj + 2; t < 16; t++)
+            if ((t - jj - 2) * 5 / (14 - jj) == q) update(t);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      const double root = rsqrt_nr(piv);
+#pragma unroll
+      for (int jj = 0; jj < 16; jj++) {
+        const int j = 16 * jb + jj;
+        const double v = rr[jj] * lane_value(root, jj);
+        rr[jj] = j < jf && lane >= j ? v : rr[jj];
+      }
+#pragma unroll
+      for (int t = 0; t < 16; t++) D[lane][16 * jb + t] = rr[t];
+      if (lane == 0) *s_fail = jf;
+    }
+    __syncthreads();
+    jdone = *s_fail;
+    if (jdone < nb) break;
+    for (int q = wave; q < (3 - jb) * (4 - jb) / 2; q += 4) {
+      // tile q of the lower triangle: column block bc, row block bi >= bc
+      int bc = jb + 1, bi = q;
+      while (bi >= 4 - bc) bi -= 4 - bc++;
+      bi += bc;
+      v4d acc;
+#pragma unroll
+      for (int r = 0; r < 4; r++) acc[r] = D[16 * bi + lk + 4 * r][16 * bc + lr];
+#pragma unroll
+      for (int k = 0; k < 16; k += 4)
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(-D[16 * bi + lr][16 * jb + k + lk],
+                                                   D[16 * bc + lr][16 * jb + k + lk], acc, 0, 0, 0);
+#pragma unroll
+      for (int r = 0; r < 4; r++) D[16 * bi + lk + 4 * r][16 * bc + lr] = acc[r];
+    }
+    __syncthreads();
+    if (wave == jb) block_inverse(D, X, rcp, jb, lane);
+  }
+  if (jdone == nb) {
+    // identity blocks past nb
+    if (16 * wave >= nb) block_inverse(D, X, rcp, wave, lane);
+    __syncthreads();
+  }
+  return jdone;
+}
+
+// Step 3: X = L^-1 by 16 x 16 blocks.  (a) the diagonal blocks (block_inverse,
+// in panel_factor); (b) one block diagonal at a time, X_ij = -X_ii
+// sum_{k=j}^{i-1} L_ik X_kj, the blocks of a diagonal on separate waves (two
+// MFMA products each).  Rows beyond nb are identity rows of L, so their part
+// of X is the identity.  X's other blocks are zero (panel_factor).  All 256
+// threads.
+__device__ __attribute__((always_inline)) inline void panel_inverse(double (*D)[LD], double (*X)[LD],
+                                                                    int wave, int lane) {
   // (b) on MFMA, wave w forms block (w + dist, w): T = L[bi rows][bj, bi)
   // X[bj, bi)[bj cols], then X = -X_ii T.  T's accumulator is the second
   // product's B operand as it stands: lane l holds T[l/16 + 4r][l%16], the
@@ -923,7 +970,7 @@ __device__ __attribute__((always_inline)) inline void panel_inverse(double (*D)[
 }
 
 // acc = rows(16 rows of wave w) . X^T on MFMA: wave w, column block bj
-__device__ __attribute__((always_inline)) inline void panel_times_xt(const double (*R)[NB + 1], const double (*X)[NB + 1],
+__device__ __attribute__((always_inline)) inline void panel_times_xt(const double (*R)[LD], const double (*X)[LD],
                                       v4d (&acc)[4], int wave, int lr, int lk) {
 #pragma unroll
   for (int bj = 0; bj < 4; bj++) acc[bj] = (v4d){0.0, 0.0, 0.0, 0.0};
@@ -936,9 +983,32 @@ __device__ __attribute__((always_inline)) inline void panel_times_xt(const doubl
   }
 }
 
+// the same for two blocks of rows
+__device__ __attribute__((always_inline)) inline void panel_times_xt2(const double (*R)[LD],
+                                                                      const double (*S)[LD],
+                                                                      const double (*X)[LD],
+                                                                      v4d (&a)[4], v4d (&b)[4],
+                                                                      int wave, int lr, int lk) {
+#pragma unroll
+  for (int bj = 0; bj < 4; bj++) {
+    a[bj] = (v4d){0.0, 0.0, 0.0, 0.0};
+    b[bj] = a[bj];
+  }
+#pragma unroll 4
+  for (int kk = 0; kk < NB; kk += 4) {
+    const double r = R[16 * wave + lr][kk + lk], q = S[16 * wave + lr][kk + lk];
+#pragma unroll
+    for (int bj = 0; bj < 4; bj++) {
+      const double x = X[16 * bj + lr][kk + lk];
+      a[bj] = __builtin_amdgcn_mfma_f64_16x16x4f64(r, x, a[bj], 0, 0, 0);
+      b[bj] = __builtin_amdgcn_mfma_f64_16x16x4f64(q, x, b[bj], 0, 0, 0);
+    }
+  }
+}
+
 // the block's L and inverse to the workspace (rows / columns beyond nb of
 // the inverse zeroed)
-__device__ __attribute__((always_inline)) inline void panel_publish(const double (*D)[NB + 1], const double (*X)[NB + 1], int n,
+__device__ __attribute__((always_inline)) inline void panel_publish(const double (*D)[LD], const double (*X)[LD], int n,
                                      int k0, int nb, double* Linv, int tid) {
   double* Lg = Linv + ((size_t)((n + NB - 1) / NB) + k0 / NB) * NB * NB;
   double* Xg = Linv + (size_t)(k0 / NB) * NB * NB;
@@ -965,11 +1035,10 @@ __global__ __launch_bounds__(256) void k_panel(double* A, int n, int k0, int nb,
   // the failure flag is read with the first loads; nothing is written
   // before it is tested
   const int failed = *fail;
-  __shared__ double D[NB][NB + 1];
-  __shared__ double X[NB][NB + 1];     // Lp_d in step 1, L^-1 from step 3
-  __shared__ double Rs[NB][NB + 1];
+  __shared__ double D[NB][LD];
+  __shared__ double X[NB][LD];     // Lp_d in step 1, L^-1 from step 3
+  __shared__ double Rs[NB][LD];
   __shared__ double rcp[NB];
-  __shared__ double colw[4][NB];
   __shared__ int s_fail;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int lr = lane & 15, lk = lane >> 4;
@@ -1035,7 +1104,7 @@ __global__ __launch_bounds__(256) void k_panel(double* A, int n, int k0, int nb,
       }
   }
   __syncthreads();
-  const int jdone = panel_factor(D, colw, &s_fail, nb, wave, lane);
+  const int jdone = panel_factor(D, X, rcp, &s_fail, nb, wave, lane);
   // the block's L goes to the workspace (other workgroups may still be
   // reading the block from A); k_diag_copy moves it into A at the end
   if (jdone < nb) {
@@ -1051,7 +1120,7 @@ __global__ __launch_bounds__(256) void k_panel(double* A, int n, int k0, int nb,
     }
     return;
   }
-  panel_inverse(D, X, rcp, wave, lane, tid);
+  panel_inverse(D, X, wave, lane);
   if (blockIdx.x == 0) panel_publish(D, X, n, k0, nb, Linv, tid);
   // step 4: rows = R Dinv^T
   v4d acc[4];
@@ -1077,12 +1146,11 @@ __global__ __launch_bounds__(256) void k_panel(double* A, int n, int k0, int nb,
 __global__ __launch_bounds__(256) void k_panel2(double* A, int n, int k0, int nb2, double* Linv,
                                                 double* L21w, int* fail) {
   const int failed = *fail;
-  __shared__ double D[NB][NB + 1];
-  __shared__ double X[NB][NB + 1];
-  __shared__ double Rs[NB][NB + 1];
-  __shared__ double L2[NB][NB + 1];
+  __shared__ double D[NB][LD];
+  __shared__ double X[NB][LD];
+  __shared__ double Rs[NB][LD];
+  __shared__ double L2[NB][LD];
   __shared__ double rcp[NB];
-  __shared__ double colw[4][NB];
   __shared__ int s_fail;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int lr = lane & 15, lk = lane >> 4;
@@ -1111,10 +1179,20 @@ __global__ __launch_bounds__(256) void k_panel2(double* A, int n, int k0, int nb
       L2[r][c] = av[q];
     }
   }
+  // the own rows' second-panel columns, under way during the first panel
+  v4d accR[4];
+#pragma unroll
+  for (int bj = 0; bj < 4; bj++)
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const long row = rowbase + 16 * wave + lk + 4 * r;
+      const int cc = 16 * bj + lr;
+      accR[bj][r] = (!diag_rows && row < n && cc < nb2) ? A[row * n + k1 + cc] : 0.0;
+    }
   __syncthreads();
   if (failed) return;
   // ---- first panel (no pending update) ----
-  int jdone = panel_factor(D, colw, &s_fail, NB, wave, lane);
+  int jdone = panel_factor(D, X, rcp, &s_fail, NB, wave, lane);
   if (jdone < NB) {
     if (diag_rows) {
       double* Lg = Linv + ((size_t)((n + NB - 1) / NB) + k0 / NB) * NB * NB;
@@ -1124,12 +1202,11 @@ __global__ __launch_bounds__(256) void k_panel2(double* A, int n, int k0, int nb
     // the rows keep their input values
     return;
   }
-  panel_inverse(D, X, rcp, wave, lane, tid);
+  panel_inverse(D, X, wave, lane);
   if (diag_rows) panel_publish(D, X, n, k0, NB, Linv, tid);
   {
     v4d ar[4], al[4];
-    panel_times_xt(Rs, X, ar, wave, lr, lk);   // own rows' L (first panel)
-    panel_times_xt(L2, X, al, wave, lr, lk);   // L21
+    panel_times_xt2(Rs, L2, X, ar, al, wave, lr, lk);   // own rows' L (first panel), L21
     __syncthreads();                           // Rs, L2 and X have been read
 #pragma unroll
     for (int bj = 0; bj < 4; bj++)
@@ -1153,17 +1230,9 @@ __global__ __launch_bounds__(256) void k_panel2(double* A, int n, int k0, int nb
       const int e = tid + 256 * q, r = e >> 6, c = e & 63;
       D[r][c] = d2v[q];
     }
-    v4d accR[4], accD[4];
+    v4d accD[4];
 #pragma unroll
-    for (int bj = 0; bj < 4; bj++) {
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const long row = rowbase + 16 * wave + lk + 4 * r;
-        const int cc = 16 * bj + lr;
-        accR[bj][r] = (!diag_rows && row < n && cc < nb2) ? A[row * n + k1 + cc] : 0.0;
-      }
-      accD[bj] = (v4d){0.0, 0.0, 0.0, 0.0};
-    }
+    for (int bj = 0; bj < 4; bj++) accD[bj] = (v4d){0.0, 0.0, 0.0, 0.0};
     __syncthreads();   // Rs, L2 and D are in place
     const long arow = rowbase + 16 * wave + lr;
 #pragma unroll
@@ -1188,7 +1257,7 @@ __global__ __launch_bounds__(256) void k_panel2(double* A, int n, int k0, int nb
       }
   }
   __syncthreads();
-  jdone = panel_factor(D, colw, &s_fail, nb2, wave, lane);
+  jdone = panel_factor(D, X, rcp, &s_fail, nb2, wave, lane);
   if (jdone < nb2) {
     if (diag_rows) {
       double* Lg = Linv + ((size_t)((n + NB - 1) / NB) + k1 / NB) * NB * NB;
@@ -1203,7 +1272,7 @@ __global__ __launch_bounds__(256) void k_panel2(double* A, int n, int k0, int nb
     }
     return;
   }
-  panel_inverse(D, X, rcp, wave, lane, tid);
+  panel_inverse(D, X, wave, lane);
   if (diag_rows) {
     panel_publish(D, X, n, k1, nb2, Linv, tid);
     return;
@@ -1230,12 +1299,11 @@ __global__ __launch_bounds__(256) void k_panel2_rows(double* A, int n, int k0, i
                                                      double* Linv, double* L21w, int* fail,
                                                      int R) {
   const int failed = *fail;
-  __shared__ double D[NB][NB + 1];
-  __shared__ double X[NB][NB + 1];
-  __shared__ double Rs[NB][NB + 1];
-  __shared__ double L2[NB][NB + 1];
+  __shared__ double D[NB][LD];
+  __shared__ double X[NB][LD];
+  __shared__ double Rs[NB][LD];
+  __shared__ double L2[NB][LD];
   __shared__ double rcp[NB];
-  __shared__ double colw[4][NB];
   __shared__ int s_fail;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int lr = lane & 15, lk = lane >> 4;
@@ -1278,7 +1346,7 @@ __global__ __launch_bounds__(256) void k_panel2_rows(double* A, int n, int k0, i
   __syncthreads();
   if (failed) return;
   // ---- first panel ----
-  int jdone = panel_factor(D, colw, &s_fail, NB, wave, lane);
+  int jdone = panel_factor(D, X, rcp, &s_fail, NB, wave, lane);
   if (jdone < NB) {
     if (diag_rows) {
       double* Lg = Linv + ((size_t)((n + NB - 1) / NB) + k0 / NB) * NB * NB;
@@ -1287,7 +1355,7 @@ __global__ __launch_bounds__(256) void k_panel2_rows(double* A, int n, int k0, i
     }
     return;
   }
-  panel_inverse(D, X, rcp, wave, lane, tid);
+  panel_inverse(D, X, wave, lane);
   if (diag_rows) panel_publish(D, X, n, k0, NB, Linv, tid);
   {
     v4d al[4];
@@ -1376,7 +1444,7 @@ __global__ __launch_bounds__(256) void k_panel2_rows(double* A, int n, int k0, i
       }
   }
   __syncthreads();
-  jdone = panel_factor(D, colw, &s_fail, nb2, wave, lane);
+  jdone = panel_factor(D, X, rcp, &s_fail, nb2, wave, lane);
   if (jdone < nb2) {
     if (diag_rows) {
       double* Lg = Linv + ((size_t)((n + NB - 1) / NB) + k1 / NB) * NB * NB;
@@ -1386,7 +1454,7 @@ __global__ __launch_bounds__(256) void k_panel2_rows(double* A, int n, int k0, i
     // the updated, unsolved rows are already in A
     return;
   }
-  panel_inverse(D, X, rcp, wave, lane, tid);
+  panel_inverse(D, X, wave, lane);
   if (diag_rows) {
     panel_publish(D, X, n, k1, nb2, Linv, tid);
     return;
@@ -1443,7 +1511,7 @@ __global__ __launch_bounds__(256) void k_diag_copy(double* A, int n, const doubl
 // panel's factored columns when bringing a failed factorisation to the
 // unblocked algorithm's state.
 __global__ __launch_bounds__(256) void k_trsm_rows(double* A, int n, int k0, int ncols, int r0) {
-  __shared__ double L[NB][NB + 1];
+  __shared__ double L[NB][LD];
   for (int e = threadIdx.x; e < ncols * ncols; e += blockDim.x) {
     const int i = e / ncols, j = e % ncols;
     if (j <= i) L[i][j] = A[(long)(k0 + i) * n + k0 + j];
