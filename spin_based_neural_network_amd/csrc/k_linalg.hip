@@ -42,10 +42,19 @@ __global__ __launch_bounds__(256) void k_colsum_partial(const double* __restrict
   if (k >= P) return;
   const long b0 = c * kColChunk, b1 = (b0 + kColChunk < B) ? b0 + kColChunk : B;
   double s = 0.0;
-  if (w) {
-    for (long b = b0; b < b1; b++) s += O[b * P + k] * w[b];
-  } else {
-    for (long b = b0; b < b1; b++) s += O[b * P + k];
+  for (long t = b0; t < b1; t += 16) {   // 16 loads under way (512 x 1120: 32 us, 13 now)
+    double x[16];
+#pragma unroll
+    for (int u = 0; u < 16; u++) x[u] = O[(t + u < b1 ? t + u : b1 - 1) * P + k];
+    if (w) {
+#pragma unroll
+      for (int u = 0; u < 16; u++)
+        if (t + u < b1) s += x[u] * w[t + u];
+    } else {
+#pragma unroll
+      for (int u = 0; u < 16; u++)
+        if (t + u < b1) s += x[u];
+    }
   }
   work[c * P + k] = s;
 }
@@ -602,8 +611,19 @@ static int gemm_big_impl(int M, int N, int K, double alpha, const double* A, lon
   return 0;
 }
 
+static int gemm_lat_impl(int M, int N, int K, double alpha, const double* A, long lda, const double* B,
+                         long ldb, double beta, double* C, long ldc, int mask, const int* skip,
+                         const char* tag, hipStream_t st);
+
+// Up to 128 tiles of 128 x 128 leave half of the CUs without one: 64 x 64 tiles
+// then (512 x 512, K = 1120, lower: 151 us on 10 workgroups, 63 on 36; the
+// same chains over k, the same bits)
 int launch_gemm_nt(int M, int N, int K, double alpha, const double* A, long lda, const double* B,
                    long ldb, double beta, double* C, long ldc, int lower, hipStream_t st) {
+  const long tm = (M + BT - 1) / BT, tn = (N + BT - 1) / BT;
+  if (M >= 2 * BT && N >= 2 * BT && K >= 64 && (lower ? tm * (tm + 1) / 2 : tm * tn) <= 128 &&
+      !(lower && M != N))
+    return gemm_lat_impl(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, lower, nullptr, "gemm", st);
   if (M >= 2 * BT && N >= 2 * BT && K >= 64)
     return gemm_big_impl(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, lower, lower, nullptr, "gemm",
                          st);
@@ -749,6 +769,18 @@ static int chain_lat() {
   return !(e && e[0] == '0');
 }
 
+static int gemm_lat_impl(int M, int N, int K, double alpha, const double* A, long lda, const double* B,
+                         long ldb, double beta, double* C, long ldc, int mask, const int* skip,
+                         const char* tag, hipStream_t st) {
+  const int tm = (M + LT - 1) / LT, tn = (N + LT - 1) / LT;
+  KScope ks(tag, st);
+  hipLaunchKernelGGL(k_gemm_lat, dim3((unsigned)(tm * tn)), dim3(256), 0, st, M, N, K, alpha, A, lda, B,
+                     ldb, beta, C, ldc, mask, tn, skip);
+  count_launch();
+  NQS_HIP_CHECK(hipGetLastError());
+  return 0;
+}
+
 // C (rows x cols, lower elements when mask) -= A B^T for a panel-chain
 // update; `skip` is the Cholesky's failure flag
 static int gemm_chain(int M, int N, int K, const double* A, long lda, double* C, long ldc,
@@ -757,13 +789,7 @@ static int gemm_chain(int M, int N, int K, const double* A, long lda, double* C,
   if (!chain_lat())
     return gemm_big_impl(M, N, K, -1.0, A, lda, A, lda, 1.0, C, ldc, 0, mask, skip, "gemm_chain",
                          st);
-  const int tm = (M + LT - 1) / LT, tn = (N + LT - 1) / LT;
-  KScope ks("gemm_chain", st);
-  hipLaunchKernelGGL(k_gemm_lat, dim3((unsigned)(tm * tn)), dim3(256), 0, st, M, N, K, -1.0, A,
-                     lda, A, lda, 1.0, C, ldc, mask, tn, skip);
-  count_launch();
-  NQS_HIP_CHECK(hipGetLastError());
-  return 0;
+  return gemm_lat_impl(M, N, K, -1.0, A, lda, A, lda, 1.0, C, ldc, mask, skip, "gemm_chain", st);
 }
 
 // --------------------------------------------------------------------------
@@ -1816,93 +1842,99 @@ size_t potrf_linv_elems(int n) { return l21_offset(n) + l21_elems(n) + 4 * sb_co
 
 // acc (+)= sign * A B over 64 x 64 LDS tiles; the thread owns rows
 // rb .. rb + 3 and columns cb .. cb + 3
-__device__ inline void tile_fma(double (&acc)[4][4], const double (*A)[NB], const double (*Bm)[NB],
-                                double sign, int rb, int cb) {
-  for (int m = 0; m < NB; m++) {
-    double a[4], b[4];
+// acc (16 rows of this wave x 64 columns) += sign A B, both 64 x 64 in LDS:
+// each element one chain over k, as MFMA accumulates it
+__device__ inline void tile_mfma(v4d (&acc)[4], const double (*A)[LD], const double (*Bm)[LD],
+                                 double sign, int wave, int lr, int lk) {
+#pragma unroll 4
+  for (int k = 0; k < NB; k += 4) {
+    const double a = sign * A[16 * wave + lr][k + lk];
 #pragma unroll
-    for (int u = 0; u < 4; u++) a[u] = sign * A[rb + u][m];
-#pragma unroll
-    for (int v = 0; v < 4; v++) b[v] = Bm[m][cb + v];
-#pragma unroll
-    for (int u = 0; u < 4; u++)
-#pragma unroll
-      for (int v = 0; v < 4; v++) acc[u][v] += a[u] * b[v];
+    for (int bj = 0; bj < 4; bj++)
+      acc[bj] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, Bm[k + lk][16 * bj + lr], acc[bj], 0, 0, 0);
   }
 }
 
-// workgroup (s, j): block column j of super-block s's inverse.  The
-// operands of every 64 x 64 product are staged in LDS by coalesced loads;
-// each thread owns a 4 x 4 piece of the product.
+// workgroup (s, j): block column j of super-block s's inverse.  The left
+// operand of every 64 x 64 product is staged in LDS, the next one under way
+// meanwhile; a wave owns 16 rows of the product.  n = 512: 80 us with 4 x 4
+// pieces on the vector units (LDS-bound), 44 now.
 __global__ __launch_bounds__(256) void k_sb_inverse(const double* __restrict__ L,
                                                     const double* __restrict__ Linv, int n,
                                                     double* __restrict__ X, double* __restrict__ XT) {
-  __shared__ double Xs[3][NB][NB];   // X_jj, X_(j+1)j, X_(j+2)j
-  __shared__ double Ts[NB][NB];      // staged L_ik or Linv_i
-  __shared__ double Ss[NB][NB];      // S = sum_k L_ik X_kj
+  __shared__ double Xs[3][NB][LD];   // X_jj, X_(j+1)j, X_(j+2)j
+  __shared__ double Ts[NB][LD];      // staged L_ik or Linv_i
+  // S = sum_k L_ik X_kj, where X_(j+2)j is not there yet or read for the last time
+  double (*Ss)[LD] = Xs[2];
   const int s = blockIdx.x, j = blockIdx.y, tid = threadIdx.x;
+  const int wave = tid >> 6, lr = tid & 15, lk = (tid & 63) >> 4;
   const int k0 = s * SB, ncol = min(SB, n - k0), ng = (ncol + NB - 1) / NB;
-  const int rb = 4 * (tid >> 4), cb = 4 * (tid & 15);
   double* Xo = X + (size_t)s * SB * SB;
   double* XTo = XT + (size_t)s * SB * SB;
-  auto put = [&](int i, int r, int c, double v) {
-    Xo[(size_t)(NB * i + r) * SB + NB * j + c] = v;
-    XTo[(size_t)(NB * j + c) * SB + NB * i + r] = v;
-  };
-  auto product = [&](double (&acc)[4][4], const double (*Bm)[NB], double sign) {
-    tile_fma(acc, Ts, Bm, sign, rb, cb);
-  };
   for (int i = 0; i < 4; i++) {
     if (i < j || j >= ng || i >= ng) {
-      for (int e = tid; e < NB * NB; e += 256) put(i, e >> 6, e & 63, 0.0);
+      for (int e = tid; e < NB * NB; e += 256) {
+        const int r = e >> 6, c = e & 63;
+        Xo[(size_t)(NB * i + r) * SB + NB * j + c] = 0.0;
+        XTo[(size_t)(NB * j + c) * SB + NB * i + r] = 0.0;
+      }
       continue;
     }
-    double acc[4][4];
+    const double* D = Linv + (size_t)(k0 / NB + i) * NB * NB;
+    double st[NB * NB / 256];
+    // L_ik (rows of block i beyond ncol are zero), then Linv_i
+    auto fetch = [&](int k) {
+      const double* Lik = L + (size_t)(k0 + NB * i) * n + k0 + NB * k;
 #pragma unroll
-    for (int u = 0; u < 4; u++)
+      for (int q = 0; q < NB * NB / 256; q++) {
+        const int e = tid + 256 * q, r = e >> 6, c = e & 63;
+        st[q] = k == i ? D[e] : (NB * i + r < ncol) ? Lik[(size_t)r * n + c] : 0.0;
+      }
+    };
+    auto store = [&]() {
 #pragma unroll
-      for (int v = 0; v < 4; v++) acc[u][v] = 0.0;
+      for (int q = 0; q < NB * NB / 256; q++) {
+        const int e = tid + 256 * q;
+        Ts[e >> 6][e & 63] = st[q];
+      }
+    };
+    v4d acc[4];
+#pragma unroll
+    for (int bj = 0; bj < 4; bj++) acc[bj] = (v4d){0.0, 0.0, 0.0, 0.0};
     if (i == j) {
-      const double* D = Linv + (size_t)(k0 / NB + j) * NB * NB;
 #pragma unroll
-      for (int u = 0; u < 4; u++)
+      for (int bj = 0; bj < 4; bj++)
 #pragma unroll
-        for (int v = 0; v < 4; v++) acc[u][v] = D[(rb + u) * NB + cb + v];
+        for (int r = 0; r < 4; r++) acc[bj][r] = D[(16 * wave + lk + 4 * r) * NB + 16 * bj + lr];
     } else {
-      // S = sum_{k=j}^{i-1} L_ik X_kj  (rows of block i beyond ncol are zero)
+      fetch(j);
       for (int k = j; k < i; k++) {
-        const double* Lik = L + (size_t)(k0 + NB * i) * n + k0 + NB * k;
-        for (int e = tid; e < NB * NB; e += 256) {
-          const int r = e >> 6, c = e & 63;
-          Ts[r][c] = (NB * i + r < ncol) ? Lik[(size_t)r * n + c] : 0.0;
-        }
+        store();
         __syncthreads();
-        product(acc, Xs[k - j], 1.0);
+        fetch(k + 1);
+        tile_mfma(acc, Ts, Xs[k - j], 1.0, wave, lr, lk);
         __syncthreads();
       }
 #pragma unroll
-      for (int u = 0; u < 4; u++)
+      for (int bj = 0; bj < 4; bj++) {
 #pragma unroll
-        for (int v = 0; v < 4; v++) {
-          Ss[rb + u][cb + v] = acc[u][v];
-          acc[u][v] = 0.0;
-        }
-      // X_ij = -Linv_i S
-      const double* D = Linv + (size_t)(k0 / NB + i) * NB * NB;
-      for (int e = tid; e < NB * NB; e += 256) Ts[e >> 6][e & 63] = D[e];
+        for (int r = 0; r < 4; r++) Ss[16 * wave + lk + 4 * r][16 * bj + lr] = acc[bj][r];
+        acc[bj] = (v4d){0.0, 0.0, 0.0, 0.0};
+      }
+      store();
       __syncthreads();
-      product(acc, Ss, -1.0);
-    }
-    if (i - j < 3) {
-#pragma unroll
-      for (int u = 0; u < 4; u++)
-#pragma unroll
-        for (int v = 0; v < 4; v++) Xs[i - j][rb + u][cb + v] = acc[u][v];
+      tile_mfma(acc, Ts, Ss, -1.0, wave, lr, lk);   // X_ij = -Linv_i S
+      __syncthreads();
     }
 #pragma unroll
-    for (int u = 0; u < 4; u++)
+    for (int bj = 0; bj < 4; bj++)
 #pragma unroll
-      for (int v = 0; v < 4; v++) put(i, rb + u, cb + v, acc[u][v]);
+      for (int r = 0; r < 4; r++) {
+        const int row = 16 * wave + lk + 4 * r, c = 16 * bj + lr;
+        if (i - j < 3) Xs[i - j][row][c] = acc[bj][r];
+        Xo[(size_t)(NB * i + row) * SB + NB * j + c] = acc[bj][r];
+        XTo[(size_t)(NB * j + c) * SB + NB * i + row] = acc[bj][r];
+      }
     __syncthreads();
   }
 }
@@ -1983,44 +2015,55 @@ __global__ __launch_bounds__(512) void k_sbsv_first(const double* __restrict__ M
 // transposed, and Q_b = L_ba X_a, row-major.  The next block's solution then
 // needs no update of its right-hand side first:
 //   forward   x_b = X_b w_b - P_b x_a,    backward   x_a = X_a^T z_a - Q_b^T x_b.
-// Workgroup (b - 1, tile, P or Q): one 64 x 64 output tile.
+// Workgroup (b - 1, tile, P or Q): one 64 x 64 output tile on MFMA, the next
+// operands under way meanwhile (n = 512: 52 us on the vector units, 21 now).
 __global__ __launch_bounds__(256) void k_sb_couple(const double* __restrict__ L,
                                                    const double* __restrict__ X, int n,
                                                    double* __restrict__ PT, double* __restrict__ Q) {
-  __shared__ double As[NB][NB], Bs[NB][NB];
+  __shared__ double As[NB][LD], Bs[NB][LD];
   const int b = blockIdx.x + 1, i = blockIdx.y >> 2, j = blockIdx.y & 3, isq = blockIdx.z;
-  const int tid = threadIdx.x, rb = 4 * (tid >> 4), cb = 4 * (tid & 15);
+  const int tid = threadIdx.x, wave = tid >> 6, lr = tid & 15, lk = (tid & 63) >> 4;
   const int kb = b * SB, ka = kb - SB, ncolb = min(SB, n - kb);
   const double* Xb = X + (size_t)b * SB * SB;
   const double* Xa = X + (size_t)(b - 1) * SB * SB;
-  double acc[4][4];
+  double as[NB * NB / 256], bs[NB * NB / 256];
+  auto fetch = [&](int mt) {
 #pragma unroll
-  for (int u = 0; u < 4; u++)
-#pragma unroll
-    for (int v = 0; v < 4; v++) acc[u][v] = 0.0;
-  for (int mt = 0; mt < SB / NB; mt++) {
-    for (int e = tid; e < NB * NB; e += 256) {
-      const int r = e >> 6, c = e & 63;
+    for (int q = 0; q < NB * NB / 256; q++) {
+      const int e = tid + 256 * q, r = e >> 6, c = e & 63;
       if (!isq) {
-        As[r][c] = Xb[(size_t)(NB * i + r) * SB + NB * mt + c];
-        Bs[r][c] = (NB * mt + r < ncolb) ? L[(size_t)(kb + NB * mt + r) * n + ka + NB * j + c] : 0.0;
+        as[q] = Xb[(size_t)(NB * i + r) * SB + NB * mt + c];
+        bs[q] = (NB * mt + r < ncolb) ? L[(size_t)(kb + NB * mt + r) * n + ka + NB * j + c] : 0.0;
       } else {
-        As[r][c] = (NB * i + r < ncolb) ? L[(size_t)(kb + NB * i + r) * n + ka + NB * mt + c] : 0.0;
-        Bs[r][c] = Xa[(size_t)(NB * mt + r) * SB + NB * j + c];
+        as[q] = (NB * i + r < ncolb) ? L[(size_t)(kb + NB * i + r) * n + ka + NB * mt + c] : 0.0;
+        bs[q] = Xa[(size_t)(NB * mt + r) * SB + NB * j + c];
       }
     }
+  };
+  v4d acc[4];
+#pragma unroll
+  for (int bj = 0; bj < 4; bj++) acc[bj] = (v4d){0.0, 0.0, 0.0, 0.0};
+  fetch(0);
+  for (int mt = 0; mt < SB / NB; mt++) {
+#pragma unroll
+    for (int q = 0; q < NB * NB / 256; q++) {
+      const int e = tid + 256 * q;
+      As[e >> 6][e & 63] = as[q];
+      Bs[e >> 6][e & 63] = bs[q];
+    }
     __syncthreads();
-    tile_fma(acc, As, Bs, 1.0, rb, cb);
+    if (mt + 1 < SB / NB) fetch(mt + 1);
+    tile_mfma(acc, As, Bs, 1.0, wave, lr, lk);
     __syncthreads();
   }
   double* out = (isq ? Q : PT) + (size_t)b * SB * SB;
 #pragma unroll
-  for (int u = 0; u < 4; u++)
+  for (int bj = 0; bj < 4; bj++)
 #pragma unroll
-    for (int v = 0; v < 4; v++) {
-      const int r = NB * i + rb + u, c = NB * j + cb + v;
-      if (isq) out[(size_t)r * SB + c] = acc[u][v];
-      else out[(size_t)c * SB + r] = acc[u][v];
+    for (int q = 0; q < 4; q++) {
+      const int r = NB * i + 16 * wave + lk + 4 * q, c = NB * j + 16 * bj + lr;
+      if (isq) out[(size_t)r * SB + c] = acc[bj][q];
+      else out[(size_t)c * SB + r] = acc[bj][q];
     }
 }
 
