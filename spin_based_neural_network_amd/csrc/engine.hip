@@ -3959,7 +3959,7 @@ int seeded_lanczos(nqs_log_amp_fn_t fn, void* user, const EdHam& H, const EdProj
 // One symmetry sector's orbits (k_edsym.hip)
 struct EdSector {
   nqs::EdSym y;
-  ScopedBuf tab, chi, reps, code, len, ell, diag;
+  ScopedBuf tab, chi, reps, code, len, ell, used, diag;
   long R = 0;
 };
 
@@ -4057,10 +4057,11 @@ int ed_sector_build(const EdHam& H, const std::vector<std::vector<int>>& perm,
   CKR(S.len.b.ensure(sizeof(double) * S.R));
   CKR(S.diag.b.ensure(sizeof(double) * S.R));
   CKR(S.ell.b.ensure(sizeof(unsigned) * rows * S.R));
+  CKR(S.used.b.ensure(sizeof(int) * ((S.R + 255) / 256 * 4)));
   CKR(nqs::launch_eds_orbits(S.y, dim, flags.b.as<unsigned long long>(), first.b.as<unsigned>(),
                              S.reps.b.as<unsigned>(), S.R, S.code.b.as<unsigned>(),
-                             S.len.b.as<double>(), H.op, S.ell.b.as<unsigned>(), S.diag.b.as<double>(),
-                             g_stream));
+                             S.len.b.as<double>(), H.op, S.ell.b.as<unsigned>(), S.used.b.as<int>(),
+                             S.diag.b.as<double>(), g_stream));
   CK(hipStreamSynchronize(g_stream));   // at, flags, counts and first end here
   return 0;
 }
@@ -4104,8 +4105,8 @@ int sector_lanczos(const EdHam& H, const EdSector& S, int N, int max_iters, doub
   CK(hipEventCreateWithFlags(&ev.e, hipEventDisableTiming));
   CK(hipHostMalloc((void**)&ev.h, 2 * sizeof(double), hipHostMallocDefault));
   auto matvec = [&]() {
-    return nqs::launch_eds_matvec(H.op, vc, w, R, S.ell.b.as<unsigned>(), S.diag.b.as<double>(), len, pt,
-                                  sc, g_stream);
+    return nqs::launch_eds_matvec(H.op, vc, w, R, S.ell.b.as<unsigned>(), S.used.b.as<int>(),
+                                  S.diag.b.as<double>(), len, pt, sc, g_stream);
   };
   // w = H v_cur - alpha v_cur - beta_k v_prev and |w|^2, alpha from the product
   auto rest = [&](int k) {

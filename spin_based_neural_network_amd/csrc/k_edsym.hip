@@ -11,21 +11,23 @@
 //   reps   smallest state of each orbit, by its number of set bits, then ascending
 //   code   per basis state: its orbit, bit 31 set where chi = -1; orbits that
 //          P removes point at entry R of every vector, which is 0
-//   ell    per bond (and flipped site) and orbit: the code of the state that
-//          H couples the representative to
+//   ell    per orbit the codes of the states that H couples the representative
+//          to, antiparallel bonds first to last, then flipped sites; used: the
+//          most bonds of a wave's 64 orbits (the others' lists end in entry R)
 // Sums over basis states are sums over orbits times the orbit's length.
 //
-// What bounds it: a product reads ell once (4 bytes a bond and orbit) and
-// gathers one double a bond; in the full basis it gathers as often from 2^N
+// What bounds it: a product reads ell once (4 bytes a listed bond and orbit)
+// and gathers one double for each; in the full basis it gathers as often from 2^N
 // states, and the projector G times more.  Exchange bonds keep the number of
 // set bits, so in this order a stretch of orbits gathers from a window of one
 // magnetisation's orbits (24 sites, 8 operations: 2.7 MB at most, of 17);
 // consecutive stretches go to one XCD, whose L2 holds its window.
 //
 // Measured (24 sites, 48 bonds, 8 operations, 60 steps): 145.5 ms in the full
-// basis, 15.9 here; a step's product and projection 505 + 1177 us, now one
-// product of 161 us (190 with the orbits in ascending order); making the orbits
-// and couplings 0.8 ms once; the start vector 35 ms on the host, 0.19 here.
+// basis, 15.2 here (17.6 with the orbits in ascending order, 15.9 with the
+// parallel bonds in the lists); a step's product and projection took 505 + 1177
+// us; making the orbits and couplings 0.8 ms once; the start vector 35 ms on
+// the host, 0.19 here.
 #include "nqs_kernels.h"
 
 namespace nqs {
@@ -166,31 +168,39 @@ __global__ __launch_bounds__(256) void k_eds_restrict(EdSym y, const unsigned* _
 // couplings and the diagonal of every representative
 __global__ __launch_bounds__(256) void k_eds_ell(EdOp op, const unsigned* __restrict__ reps, long R,
                                                  const unsigned* __restrict__ code,
-                                                 unsigned* __restrict__ ell,
+                                                 unsigned* __restrict__ ell, int* __restrict__ used,
                                                  double* __restrict__ diag) {
-  for (long r = blockIdx.x * 256L + threadIdx.x; r < R; r += (long)gridDim.x * 256) {
-    const unsigned s = reps[r];
+  for (long r0 = blockIdx.x * 256L; r0 < R; r0 += (long)gridDim.x * 256) {
+    const long r = r0 + threadIdx.x;
+    const bool in = r < R;
+    const unsigned s = in ? reps[r] : 0u;
     double d = 0.0;
-    unsigned* e = ell + r;
+    int n = 0;
     for (int b = 0; b < op.nb; b++) {
       const int u = op.bonds[2 * b], v = op.bonds[2 * b + 1];
       const bool anti = ((s >> u) ^ (s >> v)) & 1u;
       d += anti ? -op.jd : op.jd;
-      if (op.jo != 0.0) {
-        *e = anti ? code[s ^ ((1u << u) | (1u << v))] : (unsigned)R;
-        e += R;
-      }
+      if (in && anti && op.jo != 0.0) ell[(long)n++ * R + r] = code[s ^ ((1u << u) | (1u << v))];
     }
+    int most = n;
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) most = max(most, __shfl_xor(most, m, 64));
+    if ((threadIdx.x & 63) == 0) used[r >> 6] = most;
+    if (!in) continue;
+    for (; n < most; n++) ell[(long)n * R + r] = (unsigned)R;
     diag[r] = d;
-    if (op.field != 0.0)
+    if (op.field != 0.0) {
+      unsigned* e = ell + (op.jo != 0.0 ? op.nb : 0) * R + r;
       for (int i = 0; i < op.N; i++, e += R) *e = code[s ^ (1u << i)];
+    }
   }
 }
 
 // out = H in; partial <in, out>
 __global__ __launch_bounds__(256) void k_eds_matvec(const double* __restrict__ in,
                                                     double* __restrict__ out, long R,
-                                                    const unsigned* __restrict__ ell, int nb, double jo,
+                                                    const unsigned* __restrict__ ell,
+                                                    const int* __restrict__ used, int nb, double jo,
                                                     int nf, double field,
                                                     const double* __restrict__ diag,
                                                     const double* __restrict__ len,
@@ -204,18 +214,21 @@ __global__ __launch_bounds__(256) void k_eds_matvec(const double* __restrict__ i
   for (long t = T * x0 / xcds + blockIdx.x / xcds; t < end; t += (gridDim.x - x0 + xcds - 1) / xcds) {
     const long r = t * 256 + threadIdx.x;
     if (r >= R) break;
-    const unsigned* e = ell + r;
     double off = 0.0;
-    for (int b = 0; b < nb + nf; b += 8) {
-      unsigned c[8];
-      double v[8];
+    auto couple = [&](const unsigned* e, int n, double h) {
+      for (int b = 0; b < n; b += 8) {
+        unsigned c[8];
+        double v[8];
 #pragma unroll
-      for (int j = 0; j < 8; j++) c[j] = b + j < nb + nf ? e[(long)(b + j) * R] : (unsigned)R;
+        for (int j = 0; j < 8; j++) c[j] = b + j < n ? e[(long)(b + j) * R] : (unsigned)R;
 #pragma unroll
-      for (int j = 0; j < 8; j++) v[j] = at(in, c[j]);
+        for (int j = 0; j < 8; j++) v[j] = at(in, c[j]);
 #pragma unroll
-      for (int j = 0; j < 8; j++) off += (b + j < nb ? jo : field) * v[j];
-    }
+        for (int j = 0; j < 8; j++) off += h * v[j];
+      }
+    };
+    if (nb) couple(ell + r, __builtin_amdgcn_readfirstlane(used[r >> 6]), jo);
+    if (nf) couple(ell + nb * R + r, nf, field);
     const double x = in[r], z = diag[r] * x + off;
     out[r] = z;
     dot += len[r] * x * z;
@@ -322,12 +335,13 @@ int launch_eds_flags(const EdSym& y, long dim, unsigned long long* flags, unsign
 
 int launch_eds_orbits(const EdSym& y, long dim, const unsigned long long* flags, const unsigned* first,
                       unsigned* reps, long R, unsigned* code, double* len, const EdOp& op, unsigned* ell,
-                      double* diag, hipStream_t st) {
+                      int* used, double* diag, hipStream_t st) {
   KScope ks("ed_orbits", st);
   hipLaunchKernelGGL(k_eds_list, dim3((unsigned)ed_state_blocks(dim)), dim3(64), 0, st, flags, first,
                      reps);
   hipLaunchKernelGGL(k_eds_orbit, dim3(blocks_of(R)), dim3(256), tab_bytes(y), st, y, reps, R, code, len);
-  hipLaunchKernelGGL(k_eds_ell, dim3(blocks_of(R)), dim3(256), 0, st, op, reps, R, code, ell, diag);
+  hipLaunchKernelGGL(k_eds_ell, dim3(blocks_of(R)), dim3(256), 0, st, op, reps, R, code, ell, used,
+                     diag);
   for (int i = 0; i < 3; i++) count_launch();
   NQS_HIP_CHECK(hipGetLastError());
   return 0;
@@ -346,10 +360,10 @@ int launch_eds_restrict(const EdSym& y, const unsigned* reps, long R, const doub
 }
 
 int launch_eds_matvec(const EdOp& op, const double* in, double* out, long R, const unsigned* ell,
-                      const double* diag, const double* len, double* part, double* dot, hipStream_t st) {
+                      const int* used, const double* diag, const double* len, double* part, double* dot, hipStream_t st) {
   const int g = blocks_of(R);
   KScope ks("ed_matvec", st);
-  hipLaunchKernelGGL(k_eds_matvec, dim3(g), dim3(256), 0, st, in, out, R, ell, op.jo != 0.0 ? op.nb : 0,
+  hipLaunchKernelGGL(k_eds_matvec, dim3(g), dim3(256), 0, st, in, out, R, ell, used, op.jo != 0.0 ? op.nb : 0,
                      op.jo, op.field != 0.0 ? op.N : 0, op.field, diag, len, part);
   hipLaunchKernelGGL(k_eds_sum, dim3(1), dim3(256), 0, st, part, g, dot);
   count_launch();

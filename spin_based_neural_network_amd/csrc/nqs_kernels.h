@@ -365,15 +365,16 @@ long ed_state_blocks(long dim);
 int launch_eds_flags(const EdSym& y, long dim, unsigned long long* flags, unsigned* counts,
                      hipStream_t st);
 // representatives by set bits and block (first: sums of counts), codes of all
-// states, orbit lengths, couplings [bonds, sites][R] and diagonal
+// states, orbit lengths, couplings [bonds, sites][R], their bonds in use per 64
+// orbits, diagonal
 int launch_eds_orbits(const EdSym& y, long dim, const unsigned long long* flags, const unsigned* first,
                       unsigned* reps, long R, unsigned* code, double* len, const EdOp& op, unsigned* ell,
-                      double* diag, hipStream_t st);
+                      int* used, double* diag, hipStream_t st);
 // vectors of R + 1 entries, the last 0
 int launch_eds_restrict(const EdSym& y, const unsigned* reps, long R, const double* v, const double* len,
                         double* x, double* part, double* norm2, hipStream_t st);
 int launch_eds_matvec(const EdOp& op, const double* in, double* out, long R, const unsigned* ell,
-                      const double* diag, const double* len, double* part, double* dot, hipStream_t st);
+                      const int* used, const double* diag, const double* len, double* part, double* dot, hipStream_t st);
 int launch_eds_axpy2(double* w, const double* v, const double* a, const double* u, double b, long R,
                      const double* len, double* part, double* norm2, hipStream_t st);
 int launch_eds_unit(const double* x, double* y, const double* n2, long R, hipStream_t st);
