@@ -869,7 +869,12 @@ __device__ __attribute__((always_inline)) inline void block_inverse(double (*D)[
 // column chain, L_ij = a_ij / sqrt(d) is formed after the update; the
 // column's entries reach all lanes as scalars) and publishes them through D;
 // the four waves then subtract the rank-16 product from the 16 x 16 tiles
-// right of and below them on MFMA.  Returns the first column whose pivot is
+// right of and below them on MFMA.  The product is summed from zero over the
+// even and over the odd columns, two chains of eight, and subtracted once: a
+// factor must not change with the way it is computed, since an optimisation
+// that goes through hundreds of solves ends elsewhere when one does (one chain
+// of 16 on the element itself took as long, and sent some mixed-precision MinSR
+// runs out of the tables' range).  Returns the first column whose pivot is
 // not positive, or nb.  X is cleared and gets the inverses of the diagonal
 // blocks, each from the wave that has factored it, beside the next wave's
 // columns.  Called by all 256 threads.
@@ -944,15 +949,15 @@ __device__ __attribute__((always_inline)) inline int panel_factor(double (*D)[LD
       int bc = jb + 1, bi = q;
       while (bi >= 4 - bc) bi -= 4 - bc++;
       bi += bc;
-      v4d acc;
+      v4d even = (v4d){0.0, 0.0, 0.0, 0.0}, odd = even;
+      const double *a = &D[16 * bi + lr][16 * jb + 2 * lk], *b = &D[16 * bc + lr][16 * jb + 2 * lk];
 #pragma unroll
-      for (int r = 0; r < 4; r++) acc[r] = D[16 * bi + lk + 4 * r][16 * bc + lr];
+      for (int k = 0; k < 16; k += 8) {
+        even = __builtin_amdgcn_mfma_f64_16x16x4f64(a[k], b[k], even, 0, 0, 0);
+        odd = __builtin_amdgcn_mfma_f64_16x16x4f64(a[k + 1], b[k + 1], odd, 0, 0, 0);
+      }
 #pragma unroll
-      for (int k = 0; k < 16; k += 4)
-        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(-D[16 * bi + lr][16 * jb + k + lk],
-                                                   D[16 * bc + lr][16 * jb + k + lk], acc, 0, 0, 0);
-#pragma unroll
-      for (int r = 0; r < 4; r++) D[16 * bi + lk + 4 * r][16 * bc + lr] = acc[r];
+      for (int r = 0; r < 4; r++) D[16 * bi + lk + 4 * r][16 * bc + lr] -= even[r] + odd[r];
     }
     __syncthreads();
     if (wave == jb) block_inverse(D, X, rcp, jb, lane);

@@ -34,3 +34,27 @@ def test_cholesky_solve(hip, n):
     # of |A| |x| (the blocks' inverses add their condition, here below 100)
     res = np.abs(A @ x - b).max()
     assert res <= 100 * 2.0 ** -53 * (n + 8) * np.linalg.norm(A, np.inf) * np.abs(x).max()
+
+
+@pytest.mark.parametrize("o", [0, 64, 128, 512, 576])
+@pytest.mark.parametrize("past", [1, 46, 300])
+def test_panel_sum_order(hip, o, past):
+    """The rank-16 updates inside a diagonal block: sums from zero over the even
+    and over the odd columns, subtracted once.  Pivots of 1, so the factor's
+    entries are those sums: 2^-53 is lost eight times over where it is added to
+    a 1, and kept where its own sum is added."""
+    print("panel sums:", o, past, flush=True)
+    n = o + 18 + past
+    A, w = np.eye(n), 2.0 ** -53
+    A[o + 16, o:o + 16] = 1.0
+    A[o + 16, o + 16] = 17.0
+    A[o + 17, o:o + 16] = [1.0, w] + [0.0, w] * 7
+    A[o + 17, o + 17] = A[o + 18, o + 18] = 64.0
+    A[o + 18, o:o + 16] = -w
+    A[o + 18, o + 16] = 1.0
+    A = np.ascontiguousarray(A + np.tril(A, -1).T)
+    x = np.zeros(n)
+    assert hip.nqs_hip_cholesky_solve(ptr(A), n, ptr(np.ones(n)), ptr(x)) == 1
+    assert np.array_equal(A[o + 16, o:o + 17], np.ones(17))
+    assert A[o + 17, o + 16] == -(1.0 + 8 * w), float(A[o + 17, o + 16]).hex()
+    assert A[o + 18, o + 16] == 1.0 + 16 * w, float(A[o + 18, o + 16]).hex()
