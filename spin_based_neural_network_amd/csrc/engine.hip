@@ -5060,19 +5060,23 @@ int multi_issue_front(nqs_hip_multi* m) {
   return multi_join(m);
 }
 
-int multi_issue_back(nqs_hip_multi* m) {
-  if (m->persist && nqs::launch_multi_cg_persist(m->mb, m->max_iters, g_stream) != 0) {
-    fprintf(stderr, "nqs_hip_multi_step: the CG runs as a launch sequence from here on\n");
-    m->persist = 0;
-    if (m->exec) {
-      (void)hipGraphExecDestroy(m->exec);
-      m->exec = nullptr;
-    }
-    if (m->graph) {
-      (void)hipGraphDestroy(m->graph);
-      m->graph = nullptr;
-    }
+// the cooperative launch is not used any more; the captured graph ends where it began
+void multi_leave_persist(nqs_hip_multi* m) {
+  fprintf(stderr, "nqs_hip_multi_step: the CG runs as a launch sequence from here on\n");
+  m->persist = 0;
+  if (m->exec) {
+    (void)hipGraphExecDestroy(m->exec);
+    m->exec = nullptr;
   }
+  if (m->graph) {
+    (void)hipGraphDestroy(m->graph);
+    m->graph = nullptr;
+  }
+}
+
+int multi_issue_back(nqs_hip_multi* m) {
+  if (m->persist && nqs::launch_multi_cg_persist(m->mb, m->max_iters, g_stream) != 0)
+    multi_leave_persist(m);
   if (!m->persist)
     for (int it = 0; it < m->max_iters; it++) CKR(nqs::launch_multi_cg_iter(m->mb, it, 0, g_stream));
   CKR(nqs::launch_multi_apply(m->mb, g_stream));
@@ -5208,22 +5212,29 @@ int multi_step(nqs_hip_multi* m, nqs_sr_step_info_t* infos) {
   }
   CK(hipEventRecord(m->ev_t1, g_stream));
   CK(hipStreamSynchronize(g_stream));
+  // a cooperative CG whose workgroups did not meet has changed nothing that the
+  // launch sequence does not make again: the samples, energies, factors and
+  // parameters are those before it
+  auto gave_up = [&]() {
+    for (size_t i = 0; i < m->p.size(); i++)
+      if (m->h_out[i * nqs::kMultiOut + 3] < 0.0) return (long)i;
+    return -1L;
+  };
+  if (const long i = gave_up(); i >= 0 && m->persist) {
+    fprintf(stderr, "nqs_hip_multi_step: problem %ld: the workgroups of the cooperative CG launch "
+                    "did not meet\n", i);
+    multi_leave_persist(m);
+    for (nqs_hip_multi::Prob& q : m->p) CK(hipMemsetAsync(q.ticket.p, 0, 512, g_stream));
+    CKR(nqs::launch_multi_force(m->mb, g_stream));
+    CKR(multi_issue_back(m));
+    CK(hipEventRecord(m->ev_t1, g_stream));
+    CK(hipStreamSynchronize(g_stream));
+  }
   float sms = 0.f, tms = 0.f;
   m->sample_ms = hipEventElapsedTime(&sms, m->ev_s0, m->ev_s1) == hipSuccess ? sms : -1.0;
   m->step_ms = hipEventElapsedTime(&tms, m->ev_t0, m->ev_t1) == hipSuccess ? tms : -1.0;
   multi_fill_info(m, infos);
   for (nqs_hip_multi::Prob& q : m->p) q.a->m64.valid = 0;
-  bool met = true;
-  for (size_t i = 0; i < m->p.size(); i++)
-    if (m->h_out[i * nqs::kMultiOut + 3] < 0.0) {
-      fprintf(stderr, "nqs_hip_multi_step: problem %zu: the workgroups of the cooperative CG launch "
-                      "did not meet\n", i);
-      met = false;
-    }
-  if (!met) {
-    for (nqs_hip_multi::Prob& q : m->p) CK(hipMemsetAsync(q.ticket.p, 0, 512, g_stream));
-    return -1;
-  }
   // weights beyond the ratio tables' range (flagged by the tables of this
   // step): the step's moves and energies are not trusted
   for (size_t i = 0; i < m->p.size(); i++)
@@ -5250,6 +5261,10 @@ nqs_hip_multi* multi_new(int n, const nqs_config_t* cfgs, const int* size_x, con
     const char* e = getenv("NQS_HIP_MULTI_PERSIST");
     m->persist = (e && e[0] == '1') ? 1 : 0;
     m->persist_set = (e && (e[0] == '0' || e[0] == '1')) ? 1 : 0;
+    // NQS_HIP_MULTI_POLLS=n: a meeting of the cooperative launch is given up
+    // after n looks
+    const char* polls = getenv("NQS_HIP_MULTI_POLLS");
+    if (polls) m->mb.polls = std::max(0, atoi(polls));
   }
   m->p.resize(n);
   m->mp.resize(n);

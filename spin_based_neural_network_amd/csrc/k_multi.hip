@@ -650,9 +650,9 @@ __global__ __launch_bounds__(CT) void k_mb_phase(MultiBatch mb, int phase, int i
 
 // The problem's nb workgroups meet: every thread's exchanged stores have
 // reached the agent's coherence point (the wait), then one arrival; `n` counts
-// the meetings.  False when the others do not arrive within the poll limit
+// the meetings.  False when the others do not arrive within `polls` looks
 // (seconds): the kernel then ends.
-__device__ inline bool meet(const MultiProb& q, unsigned& n) {
+__device__ inline bool meet(const MultiProb& q, unsigned& n, int polls) {
   __shared__ int ok;
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
   __builtin_amdgcn_s_waitcnt(0);
@@ -663,7 +663,7 @@ __device__ inline bool meet(const MultiProb& q, unsigned& n) {
     const unsigned want = n * (unsigned)q.nb;
     __hip_atomic_fetch_add(q.bar, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     int got = 0;
-    for (int i = 0; i < (1 << 24); i++) {
+    for (int i = 0; i < polls; i++) {
       if ((int)(__hip_atomic_load(q.bar, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - want) >= 0) {
         got = 1;
         break;
@@ -718,15 +718,15 @@ __global__ __launch_bounds__(CT) void k_mb_cg(MultiBatch mb, int iters, int matv
       __syncthreads();
       return true;
     }
-    return meet(q, n);
+    return meet(q, n, mb.polls);
   };
   const int cap = matvec_only ? 1 : iters < q.max_it ? iters : q.max_it;
   while (it < cap) {
     cg_rows(q, l, t0, t1, own, it > 0 && (t1 - t0) * 16 <= kZs);
-    if (!(live = meet(q, n))) break;
+    if (!(live = meet(q, n, mb.polls))) break;
     cg_tiles(q, l, b, nb, units, PH_G, q.g);
     if (matvec_only) break;
-    if (!(live = meet(q, n))) break;
+    if (!(live = meet(q, n, mb.polls))) break;
     for (int g = 0; g < groups; g++) {
       w.j0 = j0 + g * kPairs * js;
       if (!kept) load_pairs(q, w, st);
@@ -779,7 +779,7 @@ __global__ __launch_bounds__(CT) void k_mb_cg(MultiBatch mb, int iters, int matv
       }
     }
     if (own) __syncthreads();
-    else if (!(live = meet(q, n))) break;
+    else if (!(live = meet(q, n, mb.polls))) break;
   }
   if (kept && !matvec_only && (!own || b == 0)) {
 #pragma unroll
@@ -831,7 +831,9 @@ __device__ inline bool reduce_last(double v, double* red, double* part, unsigned
   return true;
 }
 
-// theta -= lr delta in the reference layout [a | b | W], |delta|^2
+// theta -= lr delta in the reference layout [a | b | W], |delta|^2; nothing in
+// the whole batch when the workgroups of a problem gave up a meeting (iters
+// -1): its x may be of different iterations, and a step is taken for all or none
 __global__ __launch_bounds__(kMultiVecBlock) void k_mb_apply(MultiBatch mb) {
   __shared__ double red[kMultiVecBlock];
   const int qi = find_prob<F_APPLY>(mb, blockIdx.x);
@@ -839,8 +841,11 @@ __global__ __launch_bounds__(kMultiVecBlock) void k_mb_apply(MultiBatch mb) {
   const int blk = blockIdx.x - q.blk_apply, nblk = q.nvec;
   const int N = q.N, M = q.M, N1 = N + 1, L = (M + 1) * N1;
   const int e = blk * kMultiVecBlock + threadIdx.x;
+  int gave_up = 0;
+  for (int i = threadIdx.x; i < mb.n; i += kMultiVecBlock) gave_up |= mb.probs[i].sc->iters < 0;
+  gave_up = __syncthreads_or(gave_up);
   double xx = 0.0;
-  if (e < L - 1) {
+  if (e < L - 1 && !gave_up) {
     const int h = e / N1, i = e - h * N1;
     const long k = (h == M) ? i : (i == N ? (long)N + h : (long)N + M + (long)h * N + i);
     const double d = q.x[e];

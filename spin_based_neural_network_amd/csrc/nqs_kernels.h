@@ -565,6 +565,7 @@ struct MultiBatch {
   int n = 0;
   const MultiProb* probs = nullptr;   // device copy
   int nblk_prep = 0, nblk_z = 0, nblk_g = 0, nblk_vec = 0, nblk_apply = 0, nblk_cg = 0;
+  int polls = 1 << 24;                // looks at a meeting's counter before it is given up
   size_t lds = 0;
 };
 int multi_words(int N);
@@ -582,9 +583,10 @@ int launch_multi_force(const MultiBatch& mb, hipStream_t st);
 int launch_multi_cg_iter(const MultiBatch& mb, int it, int matvec_only, hipStream_t st);
 // up to `iters` CG iterations of every problem in one cooperative launch
 // (same results as as many launch_multi_cg_iter calls; matvec_only: one A p);
-// -1 when the device refuses the cooperative launch
+// -1 when the device refuses the cooperative launch; a problem whose workgroups
+// do not meet ends with iters = -1
 int launch_multi_cg_persist(const MultiBatch& mb, int iters, hipStream_t st, int matvec_only = 0);
-// par -= lr * x (reference layout), |x|^2
+// par -= lr * x (reference layout), |x|^2; nothing when a problem's iters is -1
 int launch_multi_apply(const MultiBatch& mb, hipStream_t st);
 // per problem kMultiOut doubles: <E>, <E^2>, |delta|^2, CG iterations,
 // converged, breakdown, pAp, rs_new, rs0, accepted / proposed moves, the

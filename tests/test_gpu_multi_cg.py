@@ -95,3 +95,39 @@ def test_cooperative_launch_equals_launch_sequence(hip, n, N, M, B):
         _free(hip, probs)
     for p, q in zip(*params):
         assert np.array_equal(p, q)
+
+
+def test_workgroups_that_do_not_meet(hip, monkeypatch, capfd):
+    """A cooperative launch that gives its meetings up at once (no look at the
+    counter: every workgroup of a problem that has several leaves): the step
+    ends on the launch sequence, with its bits, and so do the later ones."""
+    monkeypatch.setenv("NQS_HIP_MULTI_SPLIT", "64")
+    r = scenarios.Runner(hip, "nqs_")
+    out = []
+    for polls, on in (("0", 1), (None, 0)):
+        if polls:
+            monkeypatch.setenv("NQS_HIP_MULTI_POLLS", polls)
+        else:
+            monkeypatch.delenv("NQS_HIP_MULTI_POLLS")
+        probs = [_problem(hip, r, N, M, B, 16, 12, 3 + N) for N, M, B in
+                 ((20, 40, 512), (6, 5, 64), (64, 128, 256))]
+        n = len(probs)
+        cfgs = (type(probs[0]["cfg"]) * n)(*[p["cfg"] for p in probs])
+        m = hip.nqs_hip_multi_create(n, cfgs, (ctypes.c_int * n)(*[p["N"] for p in probs]),
+                                     (ctypes.c_int * n)(*[1] * n),
+                                     (ctypes.c_void_p * n)(*[p["a"] for p in probs]),
+                                     (ctypes.c_void_p * n)(*[p["s"] for p in probs]))
+        assert m
+        assert hip.nqs_hip_multi_use_persistent(m, on) == 0
+        info, steps = (SrInfo * n)(), []
+        for _ in range(3):
+            assert hip.nqs_hip_multi_step(m, info) == 0
+            assert hip.nqs_hip_multi_sync(m) == 0
+            steps.append(([i.as_dict() for i in info], [r.params(p["a"]) for p in probs]))
+        out.append(steps)
+        hip.nqs_hip_multi_free(m)
+        _free(hip, probs)
+        assert capfd.readouterr().err.count("did not meet") == (1 if on else 0)
+    for (gi, gp), (ri, rp) in zip(*out):
+        assert gi == ri
+        assert all(np.array_equal(g, q) for g, q in zip(gp, rp))
