@@ -477,11 +477,13 @@ bool same_ham(const nqs_config_t* c, int Lx, int Ly, int per, const AmpSource& s
 }
 
 int ham_upload(const nqs::HamHost& H, const AmpSource& src, DBuf& store, DBuf& sub_store,
-               nqs::HamDev& d);
+               nqs::HamDev& d, bool grouped);
 
+// grouped: with the terms' groups (the local energies of real RBMs)
 int ham_device(const nqs_config_t* cfg, int Lx, int Ly, int per, const AmpSource& src,
-               nqs::HamDev& out) {
-  if (same_ham(cfg, Lx, Ly, per, src)) {
+               nqs::HamDev& out, bool grouped = false) {
+  if (same_ham(cfg, Lx, Ly, per, src) &&
+      (!grouped || g_ham.dev.n_oct || g_ham.dev.n_flip + g_ham.dev.n_pair == 0)) {
     out = g_ham.dev;
     return 0;
   }
@@ -492,7 +494,7 @@ int ham_device(const nqs_config_t* cfg, int Lx, int Ly, int per, const AmpSource
     return -1;
   }
   nqs::HamDev d;
-  CKR(ham_upload(g_ham.host, src, g_ws.ham, g_ws.sublat, d));
+  CKR(ham_upload(g_ham.host, src, g_ws.ham, g_ws.sublat, d, grouped));
   g_ham.cfg = *cfg;
   g_ham.Lx = Lx;
   g_ham.Ly = Ly;
@@ -510,41 +512,51 @@ int ham_device(const nqs_config_t* cfg, int Lx, int Ly, int per, const AmpSource
 // by each pair's first site, or by the sites with the most terms left,
 // whichever takes fewer groups
 void ham_slots(const nqs::HamHost& H, int gs, std::vector<std::array<int, 3>>& best) {
-  const int nf = (int)H.flip_i.size(), np = (int)H.pair_a.size();
-  int N = H.n_sites;
-  for (int i : H.flip_i) N = std::max(N, i + 1);
-  for (int t = 0; t < np; t++) N = std::max(N, std::max(H.pair_a[t], H.pair_b[t]) + 1);
+  const int nf = (int)H.flip_i.size(), np = (int)H.pair_a.size(), N = H.n_sites;
+  auto first = [&](int t) { return t < nf ? H.flip_i[t] : H.pair_a[t - nf]; };
+  auto second = [&](int t) { return t < nf ? -1 : H.pair_b[t - nf]; };
+  // the terms of site i, ascending: at[from[i]] .. at[from[i + 1] - 1]
+  std::vector<int> from(N + 2, 0), at;
+  for (int t = 0; t < nf + np; t++) {
+    from[first(t) + 2]++;
+    if (second(t) >= 0 && second(t) != first(t)) from[second(t) + 2]++;
+  }
+  for (int i = 0; i < N; i++) from[i + 2] += from[i + 1];
+  at.resize(from[N + 1]);
+  for (int t = 0; t < nf + np; t++) {
+    at[from[first(t) + 1]++] = t;
+    if (second(t) >= 0 && second(t) != first(t)) at[from[second(t) + 1]++] = t;
+  }
   best.clear();
   for (int greedy = 0; greedy < 2; greedy++) {
-    std::vector<std::vector<std::array<int, 3>>> at(N);   // (term, centre, other) by site
-    for (int t = 0; t < nf; t++) at[H.flip_i[t]].push_back({t, H.flip_i[t], -1});
-    for (int t = 0; t < np; t++) {
-      at[H.pair_a[t]].push_back({nf + t, H.pair_a[t], H.pair_b[t]});
-      if (greedy) at[H.pair_b[t]].push_back({nf + t, H.pair_b[t], H.pair_a[t]});
-    }
-    std::vector<std::array<int, 3>> slots;
+    if (greedy && (int)best.size() < nf + np + gs) break;   // there are no fewer groups
+    std::vector<std::array<int, 3>> slots;   // (term, centre, other)
     std::vector<char> done(nf + np, 0);
-    auto take = [&](int i, size_t n) {
-      for (size_t k = 0; k < n; k++) {
-        slots.push_back(at[i][k]);
-        done[at[i][k][0]] = 1;
+    std::vector<int> left(N, 0);
+    for (int t = 0; t < nf + np; t++) {
+      left[first(t)]++;
+      if (greedy && second(t) >= 0 && second(t) != first(t)) left[second(t)]++;
+    }
+    // the first n of the terms that site i has left
+    auto take = [&](int i, int n) {
+      for (int k = from[i]; k < from[i + 1] && n > 0; k++) {
+        const int t = at[k], a = first(t), b = second(t);
+        if (done[t] || (!greedy && a != i)) continue;
+        slots.push_back({t, i, a == i ? b : a});
+        done[t] = 1;
+        left[a]--;
+        if (greedy && b >= 0 && b != a) left[b]--;
+        n--;
       }
       while (slots.size() % gs) slots.push_back({-1, i, -1});
     };
     if (!greedy) {
-      for (int i = 0; i < N; i++) take(i, at[i].size());
+      for (int i = 0; i < N; i++) take(i, left[i]);
     } else {
-      for (int left = nf + np; left > 0;) {
-        int i = 0;
-        for (int k = 0; k < N; k++) {
-          at[k].erase(std::remove_if(at[k].begin(), at[k].end(),
-                                     [&](const std::array<int, 3>& x) { return done[x[0]] != 0; }),
-                      at[k].end());
-          if (at[k].size() > at[i].size()) i = k;
-        }
-        const size_t n = std::min(at[i].size(), std::max<size_t>(at[i].size() / gs * gs, gs));
-        take(i, n);
-        left -= (int)n;
+      for (;;) {
+        const int i = (int)(std::max_element(left.begin(), left.end()) - left.begin());
+        if (left[i] == 0) break;
+        take(i, std::min(left[i], std::max(left[i] / gs * gs, gs)));
       }
     }
     if (greedy == 0 || slots.size() < best.size()) best = slots;
@@ -552,16 +564,19 @@ void ham_slots(const nqs::HamHost& H, int gs, std::vector<std::array<int, 3>>& b
   while (best.size() % 8) best.push_back({-1, best.back()[1], -1});
 }
 
-// term lists of H (and the Marshall sublattice of src) into device buffers
+// term lists of H (and the Marshall sublattice of src) into device buffers;
+// grouped: and the terms in groups, which the local energies and amplitude
+// ratios of real RBMs alone read (host work of 0.015 ms for 400 pairs of 100
+// periodic sites, 0.04 for 342 open)
 int ham_upload(const nqs::HamHost& H, const AmpSource& src, DBuf& store, DBuf& sub_store,
-               nqs::HamDev& d) {
+               nqs::HamDev& d, bool grouped) {
   const size_t nd = H.diag_a.size(), nf = H.flip_i.size(), np = H.pair_a.size();
   // groups of 4, 2 or 1 terms: a slot costs two FP64 instructions and its share
   // of four selects
   std::vector<std::array<int, 3>> slots;
   int gs = 1;
   double cost = 0.0;
-  for (int g = 1; g <= 4 && nf + np > 0; g *= 2) {
+  for (int g = 1; g <= 4 && grouped && nf + np > 0; g *= 2) {
     std::vector<std::array<int, 3>> v;
     ham_slots(H, g, v);
     const double c = v.size() * (2.0 + 4.0 / g);
@@ -572,7 +587,10 @@ int ham_upload(const nqs::HamHost& H, const AmpSource& src, DBuf& store, DBuf& s
     }
   }
   const size_t ints = 2 * nd + nf + 2 * np + 3 * slots.size() + 4, dbls = nd + nf + np + 4;
-  CKR(store.ensure(ints * sizeof(int) + dbls * sizeof(double) + 64));
+  // room for any groups (at most twice the terms in octets, else groups of one
+  // cost less): with and without them the terms stay where they are
+  const size_t room = 6 * ((nf + np + 7) / 8 * 8) - 3 * slots.size();
+  CKR(store.ensure((ints + room) * sizeof(int) + dbls * sizeof(double) + 64));
   char* base = store.as<char>();
   double* dc = (double*)base;
   double* fc = dc + nd;
@@ -673,7 +691,7 @@ template <typename R>
 int eloc_device_T(const nqs_config_t* cfg, int Lx, int Ly, int per, const AmpSource& src,
                   const int* d_spins, int B, double* d_re, double* d_im) {
   nqs::HamDev H;
-  CKR(ham_device(cfg, Lx, Ly, per, src, H));
+  CKR(ham_device(cfg, Lx, Ly, per, src, H, src.a->kind != NQS_ANSATZ_COMPLEX_RBM));
   if (g_ham.host.n_sites != src.a->N) {
     fprintf(stderr, "nqs_hip: lattice has %d sites but the ansatz %d\n", g_ham.host.n_sites,
             src.a->N);
@@ -3113,7 +3131,7 @@ NQS_EXPORT int nqs_compute_kagome_bond_phase(const nqs_config_t* cfg, int Lx_cel
   AmpSource src;
   src.a = a;
   nqs::HamDev H;
-  CKR(ham_upload(hh, src, g_ws.bond_ham, g_ws.bond_sub, H));
+  CKR(ham_upload(hh, src, g_ws.bond_ham, g_ws.bond_sub, H, a->kind != NQS_ANSATZ_COMPLEX_RBM));
   a->dev_fresh = 0;
   CKR(ansatz_upload(a));
   ModelView<double> v;
@@ -5300,7 +5318,7 @@ nqs_hip_multi* multi_new(int n, const nqs_config_t* cfgs, const int* size_x, con
     if (nqs::build_hamiltonian(&q.cfg, size_x[i], size_y[i], s->opt.periodic, hh) != 0 ||
         hh.n_sites != N)
       return fail(i, "Hamiltonian unavailable or of another size");
-    if (ham_upload(hh, s->src, q.ham, q.sublat, q.H)) return fail(i, "device memory");
+    if (ham_upload(hh, s->src, q.ham, q.sublat, q.H, false)) return fail(i, "device memory");
     q.max_split = 1;
     while (q.max_split * 2 <= 32 && q.max_split * 2 * 64 <= q.B) q.max_split *= 2;
     nqs::MultiProb& mp = m->mp[i];

@@ -882,15 +882,21 @@ static int eloc_terms_go(const ModelView<R>& m, const HamDev& h, const int* spin
   return 0;
 }
 
+// the real kernel reads the terms by their groups
+template <typename R>
+static bool grouped(const ModelView<R>& m, const HamDev& h) {
+  return m.cplx || h.n_oct > 0 || h.n_flip + h.n_pair == 0;
+}
+
 template <typename R>
 int launch_pair_ratios(const ModelView<R>& m, const HamDev& h, const int* spins, int B,
                        const R* t_re, const R* q_re, const R* q_im, void* ws, size_t ws_bytes,
                        double** res, hipStream_t st) {
   if (B <= 0) return 0;
   if (m.N > kMaxSites || h.n_flip + h.n_pair >= 65536 || !ws || ws_bytes < eloc_ws_bytes(m, h, B) ||
-      (m.M > 0 && !q_re)) {
-    fprintf(stderr, "nqs_hip: amplitude ratios need N <= %d, < 65536 terms, the logistic members "
-                    "and an E_loc workspace\n", kMaxSites);
+      (m.M > 0 && !q_re) || !grouped(m, h)) {
+    fprintf(stderr, "nqs_hip: amplitude ratios need N <= %d, < 65536 terms, the logistic members, "
+                    "grouped terms (real RBMs) and an E_loc workspace\n", kMaxSites);
     return -1;
   }
   return m.cplx ? eloc_terms_go<R, true>(m, h, spins, B, t_re, q_re, q_im, nullptr, nullptr, ws, st,
@@ -948,7 +954,7 @@ int launch_eloc(const ModelView<R>& m, const HamDev& h, const int* spins, int B,
     return -1;
   }
   const bool c = m.cplx != 0;
-  if (ws && ws_bytes >= eloc_ws_bytes(m, h, B))
+  if (ws && ws_bytes >= eloc_ws_bytes(m, h, B) && grouped(m, h))
     return c ? eloc_terms_go<R, true>(m, h, spins, B, t_re, q_re, q_im, e_re, e_im, ws, st)
              : eloc_terms_go<R, false>(m, h, spins, B, t_re, q_re, q_im, e_re, e_im, ws, st);
   if (T <= 256) {

@@ -68,7 +68,8 @@ struct HamDev {
   const signed char* sublat = nullptr;  // Marshall: 1 on sublattice A, or null
   // off-diagonal terms (flips, then pairs) in octets, each octet in groups of
   // slot_gs terms that share the site slot_c; slot_o: the pair's other site, -1
-  // for a flip; slot_t: the term, -1 for none
+  // for a flip; slot_t: the term, -1 for none (n_oct 0: not made; k_eloc_slots
+  // reads them)
   int n_oct = 0, slot_gs = 1;
   const int *slot_t = nullptr, *slot_c = nullptr, *slot_o = nullptr;
 };
@@ -244,9 +245,9 @@ int launch_bits_append(const int* spins, long n, int N, uint64_t* win, long cap,
 int launch_spins_to_bits(const int* spins, long n, int N, uint64_t* out, hipStream_t st);
 
 // ---- local energy (k_eloc.hip) -------------------------------------------
-// With a workspace of at least eloc_ws_bytes(m, h, B) bytes the term-major
-// kernels run (term tables, 64 samples per wave, fixed-order sums);
-// without one, the per-sample item-list kernel.
+// With a workspace of at least eloc_ws_bytes(m, h, B) bytes (real RBMs: and h's
+// term groups made) the term-major kernels run (term tables, 64 samples per
+// wave, fixed-order sums); without, the per-sample item-list kernel.
 // t and q: tanh(theta) and the small logistic member of every sample's
 // hidden inputs, as launch_forward writes them.
 template <typename R>

@@ -5,6 +5,7 @@ rescaling groups of 4, samples around one and two a lane, FP32.  The FP32
 bound is the oracle's own formula evaluated with 2^-24 in each of the M
 factors and in theta."""
 import ctypes
+import time
 
 import numpy as np
 import pytest
@@ -46,3 +47,28 @@ def test_real_local_energies(hip, orc, ham, Lx, Ly, per, M, B, scale, precision)
     assert not e[1].any()
     hip.nqs_ansatz_free(ah)
     orc.orc_ansatz_free(ao)
+
+
+@pytest.mark.parametrize("kind", [RBM, 6])
+def test_alternating_hamiltonians(hip, kind):
+    """Two Hamiltonians in turn cost a caller their upload (about 0.1 ms for 1024
+    pairs), not a millisecond of grouping terms on the host at every call."""
+    L, B = 16, 1
+    cfgs = [config_defaults(ansatz=kind, hamiltonian=J1J2, rbm_hidden_units=2, rbm_init_scale=0.1,
+                            j2_coupling=j2, rng_seed=3) for j2 in (0.4, 0.5)]
+    a = hip.nqs_ansatz_create(ctypes.byref(cfgs[0]), L * L)
+    s = scenarios.spins_random(B, L * L, 5, sz0=True)
+    e, opt = [np.zeros(B), np.zeros(B)], options_defaults(periodic=1)
+
+    def call(cfg):
+        t = time.perf_counter()
+        assert hip.nqs_hip_local_energy_batch_ex(ctypes.byref(cfg), L, L, ctypes.byref(opt), ptr(s), B,
+                                                 fnptr(hip, "nqs_ansatz_log_amp"), a, ptr(e[0]),
+                                                 ptr(e[1])) == 0
+        return time.perf_counter() - t
+
+    same = min(call(cfgs[0]) for _ in range(40))
+    turn = min(call(cfgs[i & 1]) for i in range(1, 41))
+    hip.nqs_ansatz_free(a)
+    print("same / in turn:", same, turn, flush=True)
+    assert turn - same < 2.5e-4, (same, turn)
