@@ -3974,19 +3974,28 @@ int seeded_lanczos(nqs_log_amp_fn_t fn, void* user, const EdHam& H, const EdProj
   return full_lanczos(q, out_vec, out_vals, out);
 }
 
-// One symmetry sector's orbits (k_edsym.hip)
+// One symmetry sector's orbits (k_edsym.hip) and the vectors of its recurrence
 struct EdSector {
   nqs::EdSym y;
-  ScopedBuf tab, chi, reps, code, len, ell, used, diag;
+  ScopedBuf tab, chi, reps, code, len, ell, used, diag, v[5], part, scal, big;
+  std::vector<unsigned> h_tab, h_count, h_first;   // copied from and to while the device works
   long R = 0;
+  size_t left = SIZE_MAX;   // device memory that may still be taken
+  int take(ScopedBuf& b, size_t bytes) {
+    if (bytes > left) return -1;
+    left -= bytes;
+    return b.b.ensure(bytes);
+  }
 };
 
 // Whether H and P are what the sector path needs: the operations are a group,
 // each as often as the others, its characters are +-1 and multiply with it, and
 // the bond list is the same after every one; the tables fit the LDS, and the
 // couplings (4 bytes an orbit, bond and flipped site) fit what the four
-// full-basis vectors of the general path would take.  Operations left once
-// each in perm / chi.
+// full-basis vectors of the general path would take.  With the codes (4 bytes a
+// state), the vectors and what an orbit has besides (44 bytes) the sector can
+// take half as much again at worst; where that cannot be had, ed_sector_setup
+// fails and the full basis serves.  Operations left once each in perm / chi.
 bool ed_sector_applies(const EdHam& H, const EdProj& P, int N, std::vector<std::vector<int>>& perm,
                        std::vector<double>& chi) {
   if (P.identity) return false;
@@ -4028,23 +4037,36 @@ bool ed_sector_applies(const EdHam& H, const EdProj& P, int N, std::vector<std::
   return true;
 }
 
-int ed_sector_build(const EdHam& H, const std::vector<std::vector<int>>& perm,
-                    const std::vector<double>& chi, int N, EdSector& S) {
+double ed_sector_start(EdSector& S, long dim, unsigned long long seed) {
+  if (ed_seed_vector(S.big.b.as<double>(), dim, seed) ||
+      nqs::launch_eds_restrict(S.y, S.reps.b.as<unsigned>(), S.R, S.big.b.as<double>(),
+                               S.len.b.as<double>(), S.v[0].b.as<double>(), S.part.b.as<double>(),
+                               S.scal.b.as<double>() + 1, g_stream))
+    return NAN;
+  return ed_read(S.scal.b.as<double>() + 1);
+}
+
+// Everything that sector_lanczos needs on the device: the orbits, the start
+// vector (n2 its squared norm; its full-basis form goes before the couplings
+// come, unless an eigenvector will want the room), the couplings
+int ed_sector_setup(const EdHam& H, const std::vector<std::vector<int>>& perm,
+                    const std::vector<double>& chi, int N, bool vec, EdSector& S, double& n2) {
   const int G = (int)perm.size();
   const long dim = 1L << N;
   // the longest runs of bits whose tables fit
   int bits = 6;
   while (bits > 3 && 4L * G * ((N + bits - 1) / bits) * (1L << bits) > nqs::kEdSymLds) bits--;
   const int nc = (N + bits - 1) / bits;
-  std::vector<unsigned> tab((size_t)G * nc << bits, 0u);
+  std::vector<unsigned>& tab = S.h_tab;
+  tab.assign((size_t)G * nc << bits, 0u);
   for (int g = 0; g < G; g++)
     for (int i = 0; i < N; i++) {   // bit perm[i] of s is bit i of T(g) s
       const int j = perm[g][i], c = j / bits, b = j % bits;
       for (int v = 0; v < 1 << bits; v++)
         if ((v >> b) & 1) tab[((size_t)(g * nc + c) << bits) + v] |= 1u << i;
     }
-  CKR(S.tab.b.ensure(sizeof(unsigned) * tab.size()));
-  CKR(S.chi.b.ensure(sizeof(double) * G));
+  CKR(S.take(S.tab, sizeof(unsigned) * tab.size()));
+  CKR(S.take(S.chi, sizeof(double) * G));
   CK(hipMemcpyAsync(S.tab.b.p, tab.data(), sizeof(unsigned) * tab.size(), hipMemcpyHostToDevice,
                     g_stream));
   CK(hipMemcpyAsync(S.chi.b.p, chi.data(), sizeof(double) * G, hipMemcpyHostToDevice, g_stream));
@@ -4054,61 +4076,65 @@ int ed_sector_build(const EdHam& H, const std::vector<std::vector<int>>& perm,
   S.y.bits = bits;
   S.y.nc = nc;
   const long nb = nqs::ed_state_blocks(dim);
-  ScopedBuf flags, counts, first;
-  CKR(flags.b.ensure(sizeof(unsigned long long) * 64 * nb));
-  CKR(counts.b.ensure(sizeof(unsigned) * 32 * nb));
-  CKR(first.b.ensure(sizeof(unsigned) * 32 * nb));
-  CKR(nqs::launch_eds_flags(S.y, dim, flags.b.as<unsigned long long>(), counts.b.as<unsigned>(), g_stream));
-  std::vector<unsigned> n(32 * nb), at(32 * nb);
-  CK(hipMemcpyAsync(n.data(), counts.b.p, sizeof(unsigned) * 32 * nb, hipMemcpyDeviceToHost, g_stream));
-  CK(hipStreamSynchronize(g_stream));
-  S.R = 0;
-  for (int p = 0; p < 32; p++)   // by set bits, then by block
-    for (long i = 0; i < nb; i++) {
-      at[32 * i + p] = (unsigned)S.R;
-      S.R += n[32 * i + p];
-    }
-  CK(hipMemcpyAsync(first.b.p, at.data(), sizeof(unsigned) * 32 * nb, hipMemcpyHostToDevice, g_stream));
+  {
+    ScopedBuf flags, counts, first;
+    CKR(S.take(flags, sizeof(unsigned long long) * 64 * nb));
+    CKR(S.take(counts, sizeof(unsigned) * 32 * nb));
+    CKR(S.take(first, sizeof(unsigned) * 32 * nb));
+    CKR(nqs::launch_eds_flags(S.y, dim, flags.b.as<unsigned long long>(), counts.b.as<unsigned>(),
+                              g_stream));
+    std::vector<unsigned>&n = S.h_count, &at = S.h_first;
+    n.resize(32 * nb);
+    at.resize(32 * nb);
+    CK(hipMemcpyAsync(n.data(), counts.b.p, sizeof(unsigned) * 32 * nb, hipMemcpyDeviceToHost, g_stream));
+    CK(hipStreamSynchronize(g_stream));
+    S.R = 0;
+    for (int p = 0; p < 32; p++)   // by set bits, then by block
+      for (long i = 0; i < nb; i++) {
+        at[32 * i + p] = (unsigned)S.R;
+        S.R += n[32 * i + p];
+      }
+    CK(hipMemcpyAsync(first.b.p, at.data(), sizeof(unsigned) * 32 * nb, hipMemcpyHostToDevice, g_stream));
+    CKR(S.take(S.reps, sizeof(unsigned) * S.R));
+    CKR(S.take(S.code, sizeof(unsigned) * dim));
+    CKR(S.take(S.len, sizeof(double) * S.R));
+    CKR(nqs::launch_eds_orbits(S.y, dim, flags.b.as<unsigned long long>(), first.b.as<unsigned>(),
+                               S.reps.b.as<unsigned>(), S.R, S.code.b.as<unsigned>(),
+                               S.len.b.as<double>(), g_stream));
+    CK(hipStreamSynchronize(g_stream));   // flags, counts and first end here
+    S.left += flags.b.bytes + counts.b.bytes + first.b.bytes;
+  }
+  const long R = S.R;
+  for (int i = 0; i < (vec ? 5 : 3); i++) CKR(S.take(S.v[i], sizeof(double) * (R + 1)));
+  CKR(S.take(S.part, sizeof(double) * nqs::ed_partials()));
+  CKR(S.take(S.scal, sizeof(double) * 8));
+  CKR(S.take(S.big, sizeof(double) * dim));
+  n2 = ed_sector_start(S, dim, 0xA5A5A5A5A5A5A5A5ULL);
+  if (!(sqrt(n2) >= 1e-14)) n2 = ed_sector_start(S, dim, 0xBEEFBABEULL);
+  if (!vec) {
+    S.left += S.big.b.bytes;
+    S.big.b.release();
+  }
   const size_t rows = (H.op.jo != 0.0 ? H.op.nb : 0) + (H.op.field != 0.0 ? N : 0);
-  CKR(S.reps.b.ensure(sizeof(unsigned) * S.R));
-  CKR(S.code.b.ensure(sizeof(unsigned) * dim));
-  CKR(S.len.b.ensure(sizeof(double) * S.R));
-  CKR(S.diag.b.ensure(sizeof(double) * S.R));
-  CKR(S.ell.b.ensure(sizeof(unsigned) * rows * S.R));
-  CKR(S.used.b.ensure(sizeof(int) * ((S.R + 255) / 256 * 4)));
-  CKR(nqs::launch_eds_orbits(S.y, dim, flags.b.as<unsigned long long>(), first.b.as<unsigned>(),
-                             S.reps.b.as<unsigned>(), S.R, S.code.b.as<unsigned>(),
-                             S.len.b.as<double>(), H.op, S.ell.b.as<unsigned>(), S.used.b.as<int>(),
-                             S.diag.b.as<double>(), g_stream));
-  CK(hipStreamSynchronize(g_stream));   // at, flags, counts and first end here
-  return 0;
+  CKR(S.take(S.diag, sizeof(double) * R));
+  CKR(S.take(S.ell, sizeof(unsigned) * rows * R));
+  CKR(S.take(S.used, sizeof(int) * ((R + 255) / 256 * 4)));
+  return nqs::launch_eds_couplings(H.op, S.reps.b.as<unsigned>(), R, S.code.b.as<unsigned>(),
+                                   S.ell.b.as<unsigned>(), S.used.b.as<int>(), S.diag.b.as<double>(),
+                                   g_stream);
 }
 
 // lean_lanczos on the sector's orbits.  The next product is under way while the
 // host takes a step's alpha, beta and Ritz value; past the last step it is not used.
-int sector_lanczos(const EdHam& H, const EdSector& S, int N, int max_iters, double tol,
+int sector_lanczos(const EdHam& H, const EdSector& S, double n2, int N, int max_iters, double tol,
                    double* out_val, double* out_vec, lanczos_result_t* out) {
   const long dim = 1L << N, R = S.R;
-  ScopedBuf vb[5], part, scal, big;
-  for (int i = 0; i < (out_vec ? 5 : 3); i++) CKR(vb[i].b.ensure(sizeof(double) * (R + 1)));
-  CKR(part.b.ensure(sizeof(double) * nqs::ed_partials()));
-  CKR(scal.b.ensure(sizeof(double) * 8));
-  CKR(big.b.ensure(sizeof(double) * dim));
-  double *vc = vb[0].b.as<double>(), *vp = vb[1].b.as<double>(), *w = vb[2].b.as<double>();
-  double *sc = scal.b.as<double>(), *pt = part.b.as<double>();
+  double *vc = S.v[0].b.as<double>(), *vp = S.v[1].b.as<double>(), *w = S.v[2].b.as<double>();
+  double *sc = S.scal.b.as<double>(), *pt = S.part.b.as<double>();
   const double* len = S.len.b.as<double>();
-  auto start = [&](unsigned long long seed) -> double {
-    if (ed_seed_vector(big.b.as<double>(), dim, seed) ||
-        nqs::launch_eds_restrict(S.y, S.reps.b.as<unsigned>(), R, big.b.as<double>(), len, vc, pt, sc + 1,
-                                 g_stream))
-      return NAN;
-    return ed_read(sc + 1);
-  };
-  double n2 = start(0xA5A5A5A5A5A5A5A5ULL);
-  if (!(sqrt(n2) >= 1e-14)) n2 = start(0xBEEFBABEULL);
   if (!std::isfinite(n2)) return -1;
   if (n2 > 0.0) CKR(nqs::launch_ed_scale(vc, vc, 1.0 / sqrt(n2), R, pt, nullptr, g_stream));
-  double* seed = out_vec ? vb[3].b.as<double>() : nullptr;
+  double* seed = out_vec ? S.v[3].b.as<double>() : nullptr;
   if (seed)
     CK(hipMemcpyAsync(seed, vc, sizeof(double) * (R + 1), hipMemcpyDeviceToDevice, g_stream));
   std::vector<double> alpha(max_iters), beta(max_iters + 1, 0.0), d(max_iters), e(max_iters);
@@ -4174,7 +4200,7 @@ int sector_lanczos(const EdHam& H, const EdSector& S, int N, int max_iters, doub
   lambda = tridiag_eig(d.data(), e.data(), K, 0);
   std::vector<double> z(K);
   tridiag_vec(d.data(), e.data(), K, lambda, z.data());
-  double* acc = vb[4].b.as<double>();
+  double* acc = S.v[4].b.as<double>();
   CK(hipMemcpyAsync(vc, seed, sizeof(double) * (R + 1), hipMemcpyDeviceToDevice, g_stream));
   CKR(nqs::launch_ed_scale(seed, acc, z[0], R + 1, pt, nullptr, g_stream));
   for (int j = 0; j + 1 < K; j++) {
@@ -4184,7 +4210,7 @@ int sector_lanczos(const EdHam& H, const EdSector& S, int N, int max_iters, doub
     CKR(nqs::launch_eds_unit(w, vc, sc + 1, R, g_stream));
     CKR(nqs::launch_ed_axpy2(acc, vc, -z[j + 1], nullptr, 0.0, R, pt, nullptr, g_stream));
   }
-  double* full = big.b.as<double>();
+  double* full = S.big.b.as<double>();
   CKR(nqs::launch_eds_expand(S.code.b.as<unsigned>(), acc, dim, 1.0, full, g_stream));
   const double a2 = ed_norm2(full, dim, pt, sc);
   if (!std::isfinite(a2)) return -1;
@@ -4217,9 +4243,15 @@ int lean_lanczos(const EdHam& H, const EdProj& P, int N, int max_iters, double t
   std::vector<std::vector<int>> perm;
   std::vector<double> chi;
   if (ed_sector_applies(H, P, N, perm, chi)) {
+    // NQS_HIP_ED_SECTOR_BYTES=n: the sector takes n bytes of device memory at most
+    const char* cap = getenv("NQS_HIP_ED_SECTOR_BYTES");
     EdSector S;
-    CKR(ed_sector_build(H, perm, chi, N, S));
-    return sector_lanczos(H, S, N, max_iters, tol, out_val, out_vec, out);
+    if (cap) S.left = strtoull(cap, nullptr, 10);
+    double n2 = 0.0;
+    if (ed_sector_setup(H, perm, chi, N, out_vec != nullptr, S, n2) == 0)
+      return sector_lanczos(H, S, n2, N, max_iters, tol, out_val, out_vec, out);
+    fprintf(stderr, "nqs_lanczos: no device memory for the symmetry sector; on the full basis\n");
+    CK(hipStreamSynchronize(g_stream));   // before its buffers go
   }
   const int nvec = out_vec ? 6 : 4;
   ScopedBuf vb[6], part, scal;

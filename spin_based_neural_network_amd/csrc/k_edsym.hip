@@ -334,15 +334,22 @@ int launch_eds_flags(const EdSym& y, long dim, unsigned long long* flags, unsign
 }
 
 int launch_eds_orbits(const EdSym& y, long dim, const unsigned long long* flags, const unsigned* first,
-                      unsigned* reps, long R, unsigned* code, double* len, const EdOp& op, unsigned* ell,
-                      int* used, double* diag, hipStream_t st) {
+                      unsigned* reps, long R, unsigned* code, double* len, hipStream_t st) {
   KScope ks("ed_orbits", st);
   hipLaunchKernelGGL(k_eds_list, dim3((unsigned)ed_state_blocks(dim)), dim3(64), 0, st, flags, first,
                      reps);
   hipLaunchKernelGGL(k_eds_orbit, dim3(blocks_of(R)), dim3(256), tab_bytes(y), st, y, reps, R, code, len);
+  count_launch(2);
+  NQS_HIP_CHECK(hipGetLastError());
+  return 0;
+}
+
+int launch_eds_couplings(const EdOp& op, const unsigned* reps, long R, const unsigned* code,
+                         unsigned* ell, int* used, double* diag, hipStream_t st) {
+  KScope ks("ed_orbits", st);
   hipLaunchKernelGGL(k_eds_ell, dim3(blocks_of(R)), dim3(256), 0, st, op, reps, R, code, ell, used,
                      diag);
-  for (int i = 0; i < 3; i++) count_launch();
+  count_launch();
   NQS_HIP_CHECK(hipGetLastError());
   return 0;
 }

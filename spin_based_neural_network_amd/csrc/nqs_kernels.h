@@ -366,11 +366,12 @@ long ed_state_blocks(long dim);
 int launch_eds_flags(const EdSym& y, long dim, unsigned long long* flags, unsigned* counts,
                      hipStream_t st);
 // representatives by set bits and block (first: sums of counts), codes of all
-// states, orbit lengths, couplings [bonds, sites][R], their bonds in use per 64
-// orbits, diagonal
+// states, orbit lengths
 int launch_eds_orbits(const EdSym& y, long dim, const unsigned long long* flags, const unsigned* first,
-                      unsigned* reps, long R, unsigned* code, double* len, const EdOp& op, unsigned* ell,
-                      int* used, double* diag, hipStream_t st);
+                      unsigned* reps, long R, unsigned* code, double* len, hipStream_t st);
+// couplings [bonds, sites][R], their bonds in use per 64 orbits, diagonal
+int launch_eds_couplings(const EdOp& op, const unsigned* reps, long R, const unsigned* code,
+                         unsigned* ell, int* used, double* diag, hipStream_t st);
 // vectors of R + 1 entries, the last 0
 int launch_eds_restrict(const EdSym& y, const unsigned* reps, long R, const double* v, const double* len,
                         double* x, double* part, double* norm2, hipStream_t st);

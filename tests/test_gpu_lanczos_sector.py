@@ -125,3 +125,27 @@ def test_sector_lanczos(hip, what, Lx, Ly, pbc, ops):
         # converged Ritz pair of the sector
         assert np.abs(_project(ops, N, vec) - vec).max() < 1e-12
         assert np.linalg.norm(_apply(bonds, N, vec) - val.value * vec) < 1e-5
+
+
+@pytest.mark.parametrize("cap", [0, 20000, 60000, 100000, 160000])
+def test_sector_without_memory(hip, monkeypatch, capfd, cap):
+    """A sector whose buffers cannot be had, from the first one (the tables) to
+    the last (the couplings): the full basis gives the value and the vector."""
+    Lx, Ly, ops = 2, 2, _translations(2, 2, -1, 1)
+    N, G, bonds = 12, 4, _bonds(2, 2, 1)
+    perm = np.ascontiguousarray([p for p, _ in ops], dtype=np.int32)
+    chi = np.array([c for _, c in ops])
+    want = _lean(bonds, ops, N, 12)
+    monkeypatch.setenv("NQS_HIP_ED_SECTOR_BYTES", str(cap))
+    val, res = ctypes.c_double(), LanczosResult()
+    assert hip.nqs_lanczos_e0_kagome_heisenberg_projected_lean(
+        Lx, Ly, 1.0, 1, ptr(perm), ptr(chi), G, 12, 0.0, ctypes.byref(val), ctypes.byref(res)) == 0
+    assert capfd.readouterr().err.count("full basis") == 1
+    assert abs(val.value - want) < 1e-12 * len(bonds)
+    vec = np.zeros(1 << N)
+    assert hip.nqs_lanczos_e0_kagome_heisenberg_projected_lean_eigvec(
+        Lx, Ly, 1.0, 1, ptr(perm), ptr(chi), G, 60, 1e-13, ctypes.byref(val), ptr(vec),
+        ctypes.byref(res)) == 0
+    assert capfd.readouterr().err.count("full basis") == 1
+    assert np.abs(_project(ops, N, vec) - vec).max() < 1e-12
+    assert np.linalg.norm(_apply(bonds, N, vec) - val.value * vec) < 1e-5
