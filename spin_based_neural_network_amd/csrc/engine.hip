@@ -1876,11 +1876,12 @@ struct StepTimer {
 };
 
 // CG solve of (A + eps I) x = F on the device; A applied through `apply`.
-// Eight iterations are queued at a time and the scalars of the eight before
-// are looked at meanwhile, so the queue never drains; iterations past the
-// end do nothing.
+// Eight iterations are queued at a time.  Where A's products look at `done`
+// themselves (`skips`), the scalars of the eight before are looked at meanwhile,
+// so the queue never drains, and iterations past the end do nothing; products
+// over stored rows would be made in full, and their eight are waited for.
 template <typename Apply>
-int cg_device(long P, const double* F, double* x, int max_iters, double tol, Apply apply,
+int cg_device(long P, const double* F, double* x, int max_iters, double tol, bool skips, Apply apply,
               int& iters, int& converged, int& breakdown, double& pAp_out, double& rs_ratio) {
   CKR(g_ws.cg.ensure(sizeof(nqs::CGScalars)));
   nqs::CGScalars* sc = g_ws.cg.as<nqs::CGScalars>();
@@ -1908,9 +1909,10 @@ int cg_device(long P, const double* F, double* x, int max_iters, double tol, App
       const int k = groups++ & 1;
       CK(hipMemcpyAsync(seen + k, sc, sizeof(*sc), hipMemcpyDeviceToHost, g_stream));
       CK(hipEventRecord(ev[k], g_stream));
-      if (groups > 1) {
-        CK(hipEventSynchronize(ev[k ^ 1]));
-        if (seen[k ^ 1].done) break;
+      if (!skips || groups > 1) {
+        const int look = skips ? k ^ 1 : k;
+        CK(hipEventSynchronize(ev[look]));
+        if (seen[look].done) break;
       }
     }
   }
@@ -2532,7 +2534,7 @@ int sr_step_impl(int method, const nqs_config_t* cfg, int Lx, int Ly, nqs_ansatz
     };
     int breakdown = 0;
     double pAp = 0.0, rr = 0.0;
-    CKR(cg_device(P, F, delta, cfg->sr_cg_max_iters, cfg->sr_cg_tol, apply, iters, converged,
+    CKR(cg_device(P, F, delta, cfg->sr_cg_max_iters, cfg->sr_cg_tol, frows, apply, iters, converged,
                   breakdown, pAp, rr));
     if (breakdown && !holo)
       fprintf(stderr, "nqs_sr cg_solve: Krylov breakdown at iter=%d, pAp=%.3e, residual/rhs=%.3e "

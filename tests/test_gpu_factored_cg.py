@@ -79,3 +79,37 @@ def test_factored_cg_single_precision_factors(hip, kind, holo):
     f64 = _steps(hip, kind, 12, 24, 480, 60, holo, 0, False, steps=1)[0]
     assert abs(f32[0]["mean_energy"] - f64[0]["mean_energy"]) < 1e-4 * abs(f64[0]["mean_energy"])
     assert np.abs(f32[1] - f64[1]).max() < 2e-3 * f64[0]["update_norm"] + 1e-6
+
+
+@pytest.mark.parametrize("holo", [True, False])
+def test_stored_rows_stop_with_their_eight(hip, holo):
+    """A solve that converges within eight iterations launches nothing past
+    them where its products read stored rows: as many launches as one that is
+    limited to eight."""
+    def launches(iters):
+        cfg = config_defaults(ansatz=CRBM, hamiltonian=TFIM, transverse_field=0.9, rbm_hidden_units=4,
+                              num_samples=256, num_thermalize=8, num_decorrelate=2, rng_seed=5,
+                              learning_rate=1e-2, sr_diag_shift=10.0, sr_cg_max_iters=iters,
+                              sr_cg_tol=1e-2)
+        r = scenarios.Runner(hip, "nqs_")
+        a, fn = r.ansatz(cfg, 6), fnptr(hip, "nqs_ansatz_log_amp")
+        opt = options_defaults(num_chains=32, periodic=1)
+        s = hip.nqs_hip_sampler_create_ex(6, ctypes.byref(cfg), ctypes.byref(opt), fn, a)
+        assert s
+        hip.nqs_sampler_thermalize(s)
+        cb = (HOLO_CB(lambda u, x, sp, n, re, im:
+                      hip.nqs_ansatz_logpsi_gradient_complex(x, sp, n, re, im)) if holo else
+              REAL_CB(lambda u, x, sp, n, g: hip.nqs_ansatz_logpsi_gradient(x, sp, n, g)))
+        step = hip.nqs_sr_step_holomorphic_full if holo else hip.nqs_sr_step_custom_full
+        info, before = SrInfo(), hip.nqs_hip_device_launches()
+        assert step(ctypes.byref(cfg), 6, 1, a, s, fn, a, ctypes.cast(cb, ctypes.c_void_p), None,
+                    ctypes.byref(info)) == 0
+        n = hip.nqs_hip_device_launches() - before
+        hip.nqs_sampler_free(s)
+        hip.nqs_ansatz_free(a)
+        return n, info.cg_iterations, info.converged
+
+    launches(8)   # buffers and tables once
+    few, many = launches(8), launches(100)
+    assert many[2] == 1 and many[1] <= 8
+    assert few == many
