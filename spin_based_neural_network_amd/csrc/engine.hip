@@ -1898,7 +1898,7 @@ int cg_device(long P, const double* F, double* x, int max_iters, double tol, boo
   int groups = 0;
   for (int it = 0; it < max_iters; it++) {
     CKR(apply(p, Ap, &sc->done));
-    if (P <= nqs::kCgOneBlock) {
+    if (P <= (skips ? nqs::kCgOneBlock : nqs::kCgOneBlock / 2)) {
       CKR(nqs::launch_cg_rest(sc, x, r, p, Ap, P, tol, g_stream));
     } else {
       CKR(nqs::launch_cg_alpha(sc, p, Ap, P, g_stream));
@@ -2365,9 +2365,10 @@ int sr_step_impl(int method, const nqs_config_t* cfg, int Lx, int Ly, nqs_ansatz
   const bool fdual = method == SR_MINSR && dual && prec == NQS_HIP_MIXED && rbm_like && !holo &&
                      factored_dual_on(a);
   // CG-SR with an RBM's own gradient takes its products with O from the
-  // factors (k_frows.hip: the bits that the stored rows give); gradient
-  // callbacks and mean-field go through O
-  const bool frows = method != SR_MINSR && rbm_like && !hfn && a->M >= 1;
+  // factors (k_frows.hip: the bits that the stored rows give) where that is
+  // faster; gradient callbacks and mean-field go through O
+  const bool frows = method != SR_MINSR && rbm_like && !hfn && a->M >= 1 &&
+                     nqs::frows_pays(N, a->M, P, B, a->kind == NQS_ANSATZ_COMPLEX_RBM, holo);
   nqs::FactorRows fr;
   // ---- 3. O matrix -----------------------------------------------------------
   const size_t ob = sizeof(double) * (size_t)B * (size_t)P;

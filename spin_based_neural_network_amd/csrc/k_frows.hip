@@ -579,8 +579,12 @@ __global__ __launch_bounds__(256) void k_fr_finish(FactorRows f, const double* _
 }
 
 // One CG iteration after A p, on one workgroup: alpha, x, r, the stopping
-// rule, p (k_sum's order of sums).  For P up to kCgOneBlock; at P = 4848 it
-// takes the place of seven dependent launches of 4 to 6 us.
+// rule, p (k_sum's order of sums).  In place of seven dependent launches an
+// iteration over stored rows takes 34 us at P = 2208 (40 with them), 49 at 4848
+// (50), 65 at 7928 (65), 86 at 11828 (83), 106 at 15728 (98): half of kCgOneBlock
+// there.  With the factored products, whose iterations past the end are queued
+// and do nothing, seven launches fewer in each of those are worth more: up to
+// kCgOneBlock (P = 15728, 32 samples: 2.58 ms a step, 2.76 with the launches).
 __global__ __launch_bounds__(1024) void k_cg_rest(CGScalars* sc, double* __restrict__ x,
                                                   double* __restrict__ r, double* __restrict__ p,
                                                   const double* __restrict__ Ap, long P, double tol) {
@@ -705,6 +709,28 @@ int rowdot(const FactorRows& f, const Shape& s, const double* v, double* u1, dou
 }
 
 }  // namespace
+
+// A row product is one workgroup's pass over the P entries for every 64 rows,
+// as long for 64 rows as for 16384; stored rows cost what they weigh, and up to
+// 256 MB of them stay in the memory-side cache.  Where N is a multiple of 64 and
+// the weights do not begin at a multiple of 8, one wave has all the groups that
+// reach into the next hidden unit, and twice the others' steps.  us of a CG
+// iteration, factored / stored:
+//   R alone    N 16, P 2208, B 80: 39 / 37, 160: 40 / 42
+//              N 24, P 4848, B 320: 65 / 57, 1280: 64 / 65, 2560: 65 / 71
+//              N 64, P 7928, B 1024: 100 / 83, 2048: 101 / 92, 4096: 102 / 130
+//              N 100, P 30500, B 1024: 276 / 224, 2048: 282 / 366
+//              N 100, P 81000, B 256: 677 / 483, 512: 688 / 688
+// and of a holomorphic step (R and I), where the stored rows' two planes are
+// also made first:
+//   N 24, P 4848, B 16: 1210 / 1280;  N 36, P 7472, B 16: 1330 / 1500
+//   N 64, P 11828, B 16: 1700 / 1340, 64: 2940 / 2800, 80: 3310 / 3340
+//   N 64, P 15728, B 16: 1640 / 1540, 32: 2560 / 2640
+bool frows_pays(int N, int M, long P, int B, bool cplx, bool holo) {
+  const bool uneven = N % 64 == 0 && (N + M) % 8 != 0;
+  if (holo) return !cplx || P < 7680 || P > 16384 || B > (uneven && P <= 12288 ? 64 : 16);
+  return B > (uneven ? 2560 : 1280) || 2L * B > P - 2048 || 8L * B * P > (256L << 20);
+}
 
 size_t frows_work_elems(const FactorRows& f) {
   const Shape s = shape_of(f);

@@ -503,6 +503,9 @@ struct FactorRows {
   double* work = nullptr;                   // frows_work_elems
   int Bp = 0;                               // set by launch_frows_prep
 };
+// whether the products from the factors take less than stored rows (cplx, holo:
+// kind 2)
+bool frows_pays(int N, int M, long P, int B, bool cplx, bool holo);
 int frows_hidden(int M);
 size_t frows_bits_elems(int B, int N);
 size_t frows_lane_elems(int B, int N);

@@ -113,3 +113,31 @@ def test_stored_rows_stop_with_their_eight(hip, holo):
     few, many = launches(8), launches(100)
     assert many[2] == 1 and many[1] <= 8
     assert few == many
+
+
+@pytest.mark.parametrize("kind,holo,N,M,B,factored", [
+    (CRBM, False, 9, 100, 16, True), (CRBM, False, 16, 64, 80, False), (CRBM, False, 16, 64, 81, True),
+    (CRBM, False, 64, 20, 340, False), (CRBM, False, 64, 20, 341, True),
+    (CRBM, False, 24, 96, 1280, False), (CRBM, False, 24, 96, 1281, True),
+    (CRBM, True, 36, 100, 16, True), (CRBM, True, 64, 120, 16, False), (CRBM, True, 64, 120, 17, True),
+    (CRBM, True, 64, 90, 64, False), (CRBM, True, 64, 90, 65, True), (CRBM, True, 64, 130, 16, True),
+    (RBM, True, 36, 100, 16, True),
+])
+def test_few_rows_are_stored(hip, kind, holo, N, M, B, factored):
+    """Few samples of many parameters go through stored rows, which take less
+    there, on either side of the lines; with the same bits.  (From 512 samples
+    on theta comes from a product of its own, which a callback's rows do not
+    see: the route alone.)"""
+    print("route:", kind, holo, N, M, B, flush=True)
+    c, ms = ctypes.c_longlong(), ctypes.c_double()
+    hip.nqs_hip_kernel_timing(b"frows_rowdot")
+    got = _steps(hip, kind, N, M, B, 16, holo, 0, False)
+    on = hip.nqs_hip_kernel_stats(b"frows_rowdot", ctypes.byref(c), ctypes.byref(ms)) == 0 and c.value > 0
+    hip.nqs_hip_kernel_timing(None)
+    assert on == factored
+    if B >= 512:
+        return
+    ref = _steps(hip, kind, N, M, B, 16, holo, 0, True)
+    for (gi, gp), (ri, rp) in zip(got, ref):
+        assert gi == ri
+        assert np.array_equal(gp, rp)
