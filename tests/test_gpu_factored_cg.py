@@ -15,7 +15,8 @@ import numpy as np
 import pytest
 
 import scenarios
-from spin_based_neural_network_amd.abi import SrInfo, config_defaults, fnptr, options_defaults
+from spin_based_neural_network_amd.abi import (MarshallWrapper, SrInfo, config_defaults, fnptr,
+                                               options_defaults)
 
 pytestmark = pytest.mark.gpu
 
@@ -26,16 +27,19 @@ HOLO_CB = ctypes.CFUNCTYPE(ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctype
                            ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p)
 
 
-def _steps(hip, kind, N, M, B, chains, holo, precision, rows, steps=2):
+def _steps(hip, kind, N, M, B, chains, holo, precision, rows, steps=2, marshall=False):
     cfg = config_defaults(ansatz=kind, hamiltonian=TFIM, transverse_field=0.9, rbm_hidden_units=M,
                           rbm_init_scale=0.4, num_samples=B, num_thermalize=2 * N,
                           num_decorrelate=N, rng_seed=31 + N + M, learning_rate=1e-2,
                           sr_diag_shift=1e-3, sr_cg_max_iters=40, sr_cg_tol=1e-6)
     r = scenarios.Runner(hip, "nqs_")
     a = r.ansatz(cfg, N)
-    fn = fnptr(hip, "nqs_ansatz_log_amp")
+    fn, user = fnptr(hip, "nqs_ansatz_log_amp"), a
+    if marshall:
+        wrap = MarshallWrapper(fn, a, N, 1)
+        fn, user = fnptr(hip, "nqs_marshall_log_amp"), ctypes.addressof(wrap)
     opt = options_defaults(num_chains=chains, periodic=1, precision=precision)
-    s = hip.nqs_hip_sampler_create_ex(N, ctypes.byref(cfg), ctypes.byref(opt), fn, a)
+    s = hip.nqs_hip_sampler_create_ex(N, ctypes.byref(cfg), ctypes.byref(opt), fn, user)
     assert s
     hip.nqs_sampler_thermalize(s)
     cb = None
@@ -47,7 +51,7 @@ def _steps(hip, kind, N, M, B, chains, holo, precision, rows, steps=2):
     out = []
     for _ in range(steps):
         info = SrInfo()
-        assert step(ctypes.byref(cfg), N, 1, a, s, fn, a, ctypes.cast(cb, ctypes.c_void_p), None,
+        assert step(ctypes.byref(cfg), N, 1, a, s, fn, user, ctypes.cast(cb, ctypes.c_void_p), None,
                     ctypes.byref(info)) == 0
         out.append((info.as_dict(), r.params(a)))
     hip.nqs_sampler_free(s)
@@ -65,6 +69,31 @@ def test_factored_cg_equals_stored_rows(hip, kind, holo, N, M, B, chains):
     print("factored CG:", kind, holo, N, M, B, flush=True)
     got = _steps(hip, kind, N, M, B, chains, holo, 0, False)
     ref = _steps(hip, kind, N, M, B, chains, holo, 0, True)
+    for (gi, gp), (ri, rp) in zip(got, ref):
+        assert gi == ri
+        assert np.array_equal(gp, rp)
+
+
+# more than 64 sites, hidden units past one staging with enough rows for the
+# factored route; the real-projected step of a real RBM (with a sign rule on its
+# amplitude, which keeps it out of the batched path)
+@pytest.mark.parametrize("kind,holo,N,M,B,chains", [
+    (CRBM, True, 65, 16, 70, 14), (CRBM, True, 81, 20, 100, 50), (CRBM, True, 100, 33, 129, 43),
+    (CRBM, True, 128, 31, 191, 30), (CRBM, True, 256, 3, 64, 16), (CRBM, False, 65, 15, 257, 64),
+    (CRBM, False, 127, 8, 128, 32), (CRBM, False, 200, 5, 300, 60), (CRBM, False, 5, 150, 200, 40),
+    (RBM, False, 15, 31, 63, 21), (RBM, False, 16, 32, 64, 32), (RBM, False, 17, 33, 65, 13),
+    (RBM, False, 31, 16, 127, 127), (RBM, False, 33, 15, 129, 43), (RBM, False, 64, 20, 128, 64),
+    (RBM, False, 100, 17, 300, 60), (RBM, False, 3, 1, 40, 8),
+])
+def test_factored_cg_equals_stored_rows_wide(hip, kind, holo, N, M, B, chains):
+    print("factored CG:", kind, holo, N, M, B, flush=True)
+    marshall = kind == RBM
+    c, ms = ctypes.c_longlong(), ctypes.c_double()
+    hip.nqs_hip_kernel_timing(b"frows_rowdot")
+    got = _steps(hip, kind, N, M, B, chains, holo, 0, False, marshall=marshall)
+    assert hip.nqs_hip_kernel_stats(b"frows_rowdot", ctypes.byref(c), ctypes.byref(ms)) == 0 and c.value > 0
+    hip.nqs_hip_kernel_timing(None)
+    ref = _steps(hip, kind, N, M, B, chains, holo, 0, True, marshall=marshall)
     for (gi, gp), (ri, rp) in zip(got, ref):
         assert gi == ri
         assert np.array_equal(gp, rp)

@@ -9,7 +9,8 @@
   sample, more samples in a workgroup than it has in hand.
 * The cooperative launch against the launch sequence, bit for bit, for
   batches with fewer workgroups than the vectors want (vectors in memory) and
-  with more problems than CUs (no cooperative launch).
+  with more problems than CUs (no cooperative launch; its problems in smaller
+  batches have it).
 """
 import ctypes
 
@@ -71,27 +72,40 @@ def test_one_problem_equals_stored_rows(hip, N, M, B, chains):
     assert np.abs(got - ref).max() <= tol, (np.abs(got - ref).max(), tol)
 
 
-@pytest.mark.parametrize("n,N,M,B", [(160, 64, 64, 48), (300, 6, 8, 64), (40, 20, 90, 520)])
-def test_cooperative_launch_equals_launch_sequence(hip, n, N, M, B):
-    print("cooperative launch:", n, N, M, B, flush=True)
+@pytest.mark.parametrize("split", [8, 256])
+@pytest.mark.parametrize("n,N,M,B,group", [(160, 64, 64, 48, 160), (300, 6, 8, 64, 100),
+                                           (40, 20, 90, 520, 40)])
+def test_cooperative_launch_equals_launch_sequence(hip, monkeypatch, n, N, M, B, group, split):
+    """One batch as a launch sequence, and `group` problems at a time in the
+    cooperative launch, both at the same split target (4 and 8 slots for the
+    520 samples; timed targets may differ from batch to batch)."""
+    print("cooperative launch:", n, N, M, B, split, flush=True)
+    monkeypatch.setenv("NQS_HIP_MULTI_SPLIT", str(split))
     r = scenarios.Runner(hip, "nqs_")
     params = []
     for on in (0, 1):
         probs = [_problem(hip, r, N + i % 2, M + i % 3, B, 16, 12, 5 + i) for i in range(n)]
-        cfgs = (type(probs[0]["cfg"]) * n)(*[p["cfg"] for p in probs])
-        lx = (ctypes.c_int * n)(*[p["N"] for p in probs])
-        ly = (ctypes.c_int * n)(*[1] * n)
-        av = (ctypes.c_void_p * n)(*[p["a"] for p in probs])
-        sv = (ctypes.c_void_p * n)(*[p["s"] for p in probs])
-        m = hip.nqs_hip_multi_create(n, cfgs, lx, ly, av, sv)
-        assert m
-        assert hip.nqs_hip_multi_use_persistent(m, on) == 0
-        info = (SrInfo * n)()
-        for _ in range(2):
-            assert hip.nqs_hip_multi_step(m, info) == 0
-        assert hip.nqs_hip_multi_sync(m) == 0
+        for k in range(0, n, group if on else n):
+            part = probs[k:k + (group if on else n)]
+            g = len(part)
+            cfgs = (type(part[0]["cfg"]) * g)(*[p["cfg"] for p in part])
+            m = hip.nqs_hip_multi_create(g, cfgs, (ctypes.c_int * g)(*[p["N"] for p in part]),
+                                         (ctypes.c_int * g)(*[1] * g),
+                                         (ctypes.c_void_p * g)(*[p["a"] for p in part]),
+                                         (ctypes.c_void_p * g)(*[p["s"] for p in part]))
+            assert m
+            assert hip.nqs_hip_multi_use_persistent(m, on) == 0
+            info = (SrInfo * g)()
+            count, ms = ctypes.c_longlong(), ctypes.c_double()
+            hip.nqs_hip_kernel_timing(b"multi_cg")
+            for _ in range(2):
+                assert hip.nqs_hip_multi_step(m, info) == 0
+            assert hip.nqs_hip_kernel_stats(b"multi_cg", ctypes.byref(count), ctypes.byref(ms)) == 0
+            hip.nqs_hip_kernel_timing(None)
+            assert count.value == (2 if on else 0)
+            assert hip.nqs_hip_multi_sync(m) == 0
+            hip.nqs_hip_multi_free(m)
         params.append([r.params(p["a"]) for p in probs])
-        hip.nqs_hip_multi_free(m)
         _free(hip, probs)
     for p, q in zip(*params):
         assert np.array_equal(p, q)
