@@ -5363,7 +5363,7 @@ nqs_hip_multi* multi_new(int n, const nqs_config_t* cfgs, const int* size_x, con
     nqs::multi_shape(mp, 1);
     const size_t L = (size_t)M1 * N1, B = (size_t)q.B, d = sizeof(double);
     if (q.t.ensure(d * 2 * B * M) || q.tT.ensure(d * B * M) || q.E.ensure(d * 2 * B) ||
-        q.bits.ensure(sizeof(unsigned) * B * nqs::multi_words(N)) || q.U.ensure(d * B) ||
+        q.bits.ensure(sizeof(unsigned) * B * nqs::multi_words(N)) || q.U.ensure(d * B * nqs::multi_parts(M)) ||
         q.tA.ensure(d * nqs::multi_ta_elems(q.B, M)) || q.vec.ensure(d * 6 * L) ||
         q.part.ensure(d * 4 * nqs::kMultiMaxPart) || q.ticket.ensure(512) || q.sc.ensure(sizeof(nqs::CGScalars)) || q.stats.ensure(d * 8) ||
         s->d_samples.ensure(sizeof(int) * B * N))

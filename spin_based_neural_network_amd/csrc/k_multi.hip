@@ -15,7 +15,8 @@
 //
 // A CG iteration of a problem is five phases, and the workgroups of the
 // problem meet after each:
-//   Z     u = O p, split over samples
+//   Z     u = O p, split over samples, and over 64-row tiles of p where the
+//         workgroups outnumber the 16-sample tiles
 //   G     O^T u, split over tiles of 16 hidden units; in a workgroup the waves
 //         take slots of the samples (nsplit, in order) and sum them in LDS
 //   A p   and partial p.Ap, split over 256-element slices
@@ -52,7 +53,7 @@ typedef double v4d __attribute__((ext_vector_type(4)));
 constexpr int CT = 512;              // threads of the CG kernels
 constexpr int CW = CT / 64;
 constexpr int kZs = 512;             // samples of a workgroup in hand in Z
-constexpr int kZb = 128;             // samples of a workgroup of the launch of Z
+constexpr int kZb = 128;             // samples of a workgroup of the launch of Z, at most
 constexpr int kTiles = 4;            // most site tiles of a wave in G
 constexpr int kPairs = 4;            // pairs of slices of a workgroup in hand
 
@@ -112,7 +113,7 @@ struct Lds {
 __device__ __host__ inline size_t lds_head(int nw) {
   return kPairs * CT + kMultiMaxPart + 2 * kZs + (size_t)kZs * nw / 2;
 }
-__device__ inline Lds carve(const MultiProb& q, double* base) {
+__device__ inline Lds carve(const MultiProb& q, int hct, double* base) {
   Lds l;
   l.red = base;
   l.part = l.red + kPairs * CT;
@@ -120,7 +121,7 @@ __device__ inline Lds carve(const MultiProb& q, double* base) {
   l.cur = l.u + kZs;
   l.bits = (unsigned*)(l.cur + kZs);
   l.v = base + lds_head(q.nw);
-  l.up = l.v + q.hct * 16 * q.si;
+  l.up = l.v + hct * 16 * q.si;
   l.tile = l.v;
   l.wu = l.tile + CW * kTiles * 256;
   l.wbits = (unsigned*)(l.wu + CW * 64);
@@ -142,13 +143,25 @@ __device__ __forceinline__ void row_steps(const double* pa, const double* pb, un
   }
 }
 
-// ---- Z: row weights u = O p of the samples of 16-sample tiles t0 .. t1 - 1 -----
+__device__ __host__ inline int tiles64(int M) { return (M + 64) / 64; }
+
+// ---- Z: row weights u = O p of the samples of 16-sample tiles t0 .. t1 - 1, of
+// share `part` of the 64-row tiles ------------------------------------------------
 // own: p is l.red.  held: the samples' words are in l.bits from the call before.
-__device__ void cg_rows(const MultiProb& q, const Lds& l, int t0, int t1, bool own, bool held) {
+// SHARED false: rw.parts is 1 (the code without the shares: 1 % of an iteration).
+template <bool SHARED>
+__device__ void cg_rows(const MultiProb& q, const Lds& l, const MultiRows& rw, int part, int t0, int t1,
+                        bool own, bool held) {
   const int tid = threadIdx.x, wave = wave_of(), lane = tid & 63;
   const int lr = lane & 15, lk = lane >> 4;
   const int M = q.M, N1 = q.N + 1, M1 = M + 1, nw = q.nw, si = q.si;
   const int HT = (M1 + 15) >> 4, KK = (N1 + 3) >> 2;
+  int c0 = 0, c1 = HT;   // 16-row tiles c0 .. c1 - 1
+  if (SHARED) {
+    c0 = tiles64(M) * part / rw.parts * 4;
+    c1 = tiles64(M) * (part + 1) / rw.parts * 4;
+    if (c1 > HT) c1 = HT;
+  }
   const unsigned magic = 0xFFFFFFFFu / (unsigned)N1 + 1;   // f / N1 for f < 2^17
   const int end = t1 * 16 < q.B ? t1 * 16 : q.B;
   for (int g0 = t0 * 16; g0 < end; g0 += kZs) {
@@ -157,10 +170,10 @@ __device__ void cg_rows(const MultiProb& q, const Lds& l, int t0, int t1, bool o
       __syncthreads();
       for (int e = tid; e < ns * nw; e += CT) l.bits[e] = q.bits[(long)g0 * nw + e];
     }
-    for (int c = 0; c < HT; c += q.hct) {
-      const int nh = HT - c < q.hct ? HT - c : q.hct, pairs = (nh + 1) >> 1;
+    for (int c = c0; c < c1; c += rw.hct) {
+      const int nh = c1 - c < rw.hct ? c1 - c : rw.hct, pairs = (nh + 1) >> 1;
       __syncthreads();
-      if (q.hct < HT || g0 == t0 * 16) {
+      if (rw.hct < c1 - c0 || g0 == t0 * 16) {
         // rows past M and columns past N are zero
         const int r1 = M1 - c * 16 < pairs * 32 ? M1 - c * 16 : pairs * 32;
         for (int e = tid; e < r1 * (si - N1); e += CT) {
@@ -186,8 +199,8 @@ __device__ void cg_rows(const MultiProb& q, const Lds& l, int t0, int t1, bool o
           }
         }
       }
-      for (int b0 = 0; b0 < ns; b0 += q.zb) {
-        const int nb = ns - b0 < q.zb ? ns - b0 : q.zb, nst = (nb + 15) >> 4;
+      for (int b0 = 0; b0 < ns; b0 += rw.zb) {
+        const int nb = ns - b0 < rw.zb ? ns - b0 : rw.zb, nst = (nb + 15) >> 4;
         // an item: 32 rows x 16 samples, two tiles of Z = V S1^T (rows hidden
         // units), weighted by t in a chain of eight as they leave the
         // accumulators; the next item's t is under way meanwhile
@@ -235,7 +248,7 @@ __device__ void cg_rows(const MultiProb& q, const Lds& l, int t0, int t1, bool o
           for (int r = 0; r < 4; r++) x = fma(z0[r], w[r], x);
 #pragma unroll
           for (int r = 0; r < 4; r++) x = fma(z1[r], w[4 + r], x);
-          l.up[(p * 4 + lk) * q.zb + s] = x;
+          l.up[(p * 4 + lk) * rw.zb + s] = x;
         }
         __syncthreads();
         // the eight chains of a tile of 64 rows (two pairs) in order, then the tiles
@@ -246,12 +259,15 @@ __device__ void cg_rows(const MultiProb& q, const Lds& l, int t0, int t1, bool o
             const int g = c / 2 + p;
             if (!(g & 1)) cur = 0.0;
 #pragma unroll
-            for (int k = 0; k < 4; k++) cur += l.up[(p * 4 + k) * q.zb + tid];
-            if ((g & 1) || 2 * g + 2 >= HT) u = g < 2 ? cur : u + cur;
+            for (int k = 0; k < 4; k++) cur += l.up[(p * 4 + k) * rw.zb + tid];
+            if ((g & 1) || 2 * g + 2 >= HT) {
+              u = g < 2 ? cur : u + cur;
+              if (SHARED && rw.parts > 1) st_x(q.u + (long)(g >> 1) * q.B + g0 + s, cur);
+            }
           }
           l.cur[s] = cur;
           l.u[s] = u;
-          if (c + nh >= HT) st_x(q.u + g0 + s, u);
+          if ((!SHARED || rw.parts == 1) && c + nh >= HT) st_x(q.u + g0 + s, u);
         }
       }
     }
@@ -298,7 +314,9 @@ __device__ __forceinline__ void chain64(double* x, const double* wu, const unsig
 // site tiles for each of CW / ws groups of waves, the waves of a group on ws
 // slots at a time.  A lane fetches its sample's weight and words for the wave;
 // the next 64 samples (slot, unit) are under way while these are used.
-__device__ void cg_tiles(const MultiProb& q, const Lds& l, int u0, int us, int units, int mode,
+// parts: of the row weights (SHARED false: 1)
+template <bool SHARED>
+__device__ void cg_tiles(const MultiProb& q, const Lds& l, int u0, int us, int units, int mode, int parts,
                          double* out) {
   const int tid = threadIdx.x, wave = wave_of(), lane = tid & 63;
   const int N1 = q.N + 1, M1 = q.M + 1, sts = (N1 + 15) >> 4, nw = q.nw;
@@ -316,7 +334,19 @@ __device__ void cg_tiles(const MultiProb& q, const Lds& l, int u0, int us, int u
     const int b0 = (k0 + sl) * q.chunk + sub, end = (k0 + sl + 1) * q.chunk;
     const int b1 = end < q.B ? end : q.B;
     const int s = b0 + lane, sc = s < q.B ? s : q.B - 1;
-    const double w = mode == PH_G1 ? 1.0 : mode == PH_GE ? q.E[sc] : ld_x(q.u + sc);
+    double w = mode == PH_G1 ? 1.0 : mode == PH_GE ? q.E[sc] : ld_x(q.u + sc);
+    if (SHARED && mode == PH_G && parts > 1) {
+      // the 64-row tiles in order, four under way
+      const int T = tiles64(q.M);
+      for (int k = 1; k < T; k += 4) {
+        double y[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) y[j] = ld_x(q.u + (long)(k + j < T ? k + j : T - 1) * q.B + sc);
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+          if (k + j < T) w += y[j];
+      }
+    }
     u = s < b1 ? w : 0.0;
     const int w0 = first_tile(unit) >> 1;
     const unsigned* bw = q.bits + (long)sc * nw;
@@ -556,9 +586,9 @@ __global__ __launch_bounds__(CT) void k_mb_phase(MultiBatch mb, int phase, int i
   const MultiProb& q = mb.probs[phase == PH_Z ? find_prob<F_Z>(mb, blk)
                                 : phase <= PH_GE || phase == PH_G ? find_prob<F_G>(mb, blk)
                                                                   : find_prob<F_VEC>(mb, blk)];
-  const Lds l = carve(q, lds);
+  const Lds l = carve(q, q.solo.hct, lds);
   if (phase <= PH_GE) {
-    cg_tiles(q, l, blk - q.blk_g, 1, blk - q.blk_g + 1, phase, phase == PH_G1 ? q.g : q.Ap);
+    cg_tiles<false>(q, l, blk - q.blk_g, 1, blk - q.blk_g + 1, phase, 1, phase == PH_G1 ? q.g : q.Ap);
     return;
   }
   const long L = vec_len(q);
@@ -596,12 +626,14 @@ __global__ __launch_bounds__(CT) void k_mb_phase(MultiBatch mb, int phase, int i
   __syncthreads();
   if (done) return;
   if (phase == PH_Z) {
-    const int t0 = (blk - q.blk_z) * (kZb / 16), nT = (q.B + 15) / 16;
-    cg_rows(q, l, t0, t0 + kZb / 16 < nT ? t0 + kZb / 16 : nT, false, false);
+    const MultiRows& rw = q.solo;
+    const int at = (blk - q.blk_z) / rw.parts, nT = (q.B + 15) / 16, per = rw.samples / 16;
+    cg_rows<true>(q, l, rw, blk - q.blk_z - at * rw.parts, at * per, at * per + per < nT ? at * per + per : nT,
+            false, false);
     return;
   }
   if (phase == PH_G) {
-    cg_tiles(q, l, blk - q.blk_g, 1, blk - q.blk_g + 1, PH_G, q.g);
+    cg_tiles<true>(q, l, blk - q.blk_g, 1, blk - q.blk_g + 1, PH_G, q.solo.parts, q.g);
     return;
   }
   Elem st[kPairs];
@@ -680,16 +712,23 @@ __device__ inline bool meet(const MultiProb& q, unsigned& n, int polls) {
 // which changes nothing that the CG start has set).  Consecutive workgroups of
 // a problem sit on one XCD (block b runs on XCD b % 8), where its t stays in
 // that XCD's L2.
+// SHARED: a problem of the batch has its rows of p in shares.
+template <bool SHARED>
 __global__ __launch_bounds__(CT) void k_mb_cg(MultiBatch mb, int iters, int matvec_only) {
   extern __shared__ double lds[];
   const int lb = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
   if (lb >= mb.nblk_cg) return;
   const MultiProb& q = mb.probs[find_prob<F_CG>(mb, lb)];
   if (q.max_it <= 0) return;   // nothing to do, and no meeting to pass
-  const Lds l = carve(q, lds);
+  const MultiRows& rw = q.coop;
+  const Lds l = carve(q, rw.hct, lds);
   double* red = l.red;
   const int b = lb - q.blk_cg, nb = q.nb, J = (q.nvec + 1) >> 1, tid = threadIdx.x;
-  const int nT = (q.B + 15) / 16, t0 = (int)((long)nT * b / nb), t1 = (int)((long)nT * (b + 1) / nb);
+  // row weights: share b % parts of the rows of p for the samples of share
+  // b / parts (the last workgroups may have neither)
+  const int nT = (q.B + 15) / 16, parts = SHARED ? rw.parts : 1, shares = nb / parts, at = b / parts;
+  const int t0 = at < shares ? (int)((long)nT * at / shares) : nT;
+  const int t1 = at < shares ? (int)((long)nT * (at + 1) / shares) : nT;
   const int units = tile_units(q, q.nt);
   const long L = vec_len(q);
   // every workgroup has the whole vectors, or every js-th pair of slices; in
@@ -722,9 +761,9 @@ __global__ __launch_bounds__(CT) void k_mb_cg(MultiBatch mb, int iters, int matv
   };
   const int cap = matvec_only ? 1 : iters < q.max_it ? iters : q.max_it;
   while (it < cap) {
-    cg_rows(q, l, t0, t1, own, it > 0 && (t1 - t0) * 16 <= kZs);
+    cg_rows<SHARED>(q, l, rw, b % parts, t0, t1, own, it > 0 && (t1 - t0) * 16 <= kZs);
     if (!(live = meet(q, n, mb.polls))) break;
-    cg_tiles(q, l, b, nb, units, PH_G, q.g);
+    cg_tiles<SHARED>(q, l, b, nb, units, PH_G, parts, q.g);
     if (matvec_only) break;
     if (!(live = meet(q, n, mb.polls))) break;
     for (int g = 0; g < groups; g++) {
@@ -889,12 +928,30 @@ size_t lds_bytes(const MultiProb& q, int hct, int zb) {
   return sizeof(double) * (lds_head(q.nw) + (z > g ? z : g));
 }
 
+// Shares of the rows of p on nb workgroups, more than one where these outnumber
+// the 16-sample tiles: by samples alone every workgroup reads all of p for 16
+// samples that keep one wave in eight busy.  One problem, 50 iterations, by
+// samples / shared, ms: N 256, M 256 (66049 parameters), 512 samples 6.4 / 3.5,
+// 2048 7.3 / 5.8; N 128, M 128 (16641), 512 2.35 / 2.14, 1024 2.51 / 2.51, 2048
+// 2.81 / 3.21; N 64, M 64 (4225), 256 1.63 / 1.78.  So for many parameters, 16
+// and more to a sample.
+int row_parts(const MultiProb& q, int nb) {
+  const int nT = (q.B + 15) / 16, T = tiles64(q.M);
+  const long L = (q.M + 1L) * (q.N + 1);
+  if (L < 16384 || L < 16L * q.B) return 1;
+  const int p = nb / nT;
+  return p < 1 ? 1 : p < T ? p : T;
+}
+static_assert(16384 > kPairs * CT, "a problem that is whole in every workgroup (own) has one part");
+
 // Cycles of a CG iteration of q on nb workgroups of a CU each (FP64 16x16x4
 // MFMAs take a SIMD 64): Z by 16-sample tiles, G by units (the site tiles of a
 // wave, nt, for the fewest), the meetings and the vector work.
 double iter_cost(const MultiProb& q, int nb, int& nt) {
   const int HT = (q.M + 16) / 16, KK = (q.N + 4) / 4, nT = (q.B + 15) / 16;
-  const double z = 16.0 * ((nT + nb - 1) / nb) * HT * (KK + 4) + (q.M + 1.0) * (q.N + 1.0) / 8;
+  const int parts = row_parts(q, nb), per = nb / parts, hp = (tiles64(q.M) + parts - 1) / parts * 4;
+  const double z = 16.0 * ((nT + per - 1) / per) * (hp < HT ? hp : HT) * (KK + 4) +
+                   (q.M + 1.0) * (q.N + 1.0) / (8 * parts);
   const int ws = q.nsplit < CW ? q.nsplit : CW, rounds = q.nsplit / ws;
   double g = 0.0;
   for (int t = 1; t <= kTiles && t <= kTiles * 2 * ws / CW + 1; t++) {
@@ -914,6 +971,7 @@ double iter_cost(const MultiProb& q, int nb, int& nt) {
 }  // namespace
 
 int multi_words(int N) { return (N + 1 + 31) / 32; }
+int multi_parts(int M) { return tiles64(M); }
 size_t multi_ta_elems(int B, int M) { return (size_t)((M + 16) / 16) * ((B + 15) / 16 * 4) * 64; }
 
 // nsplit slots of equal runs of samples (multiples of 16)
@@ -927,16 +985,17 @@ void multi_shape(MultiProb& q, int nsplit) {
 }
 
 // Hidden tiles of a chunk of p and samples of a pass over it in Z, by what the
-// LDS holds for a workgroup's share of the samples
-void shape_rows(MultiProb& q) {
-  const int HT = (q.M + 16) / 16, nT = (q.B + 15) / 16;
-  q.zb = (nT + q.nb - 1) / q.nb * 16;
-  if (q.zb > kZs) q.zb = kZs;
-  q.hct = (HT + 1) / 2 * 2;
-  while (q.zb > kZb && lds_bytes(q, q.hct < 8 ? q.hct : 8, q.zb) > kCgLds) q.zb -= 16;
-  while (q.hct > 2 && lds_bytes(q, q.hct, q.zb) > kCgLds) q.hct -= 2;
-  const int nc = (HT + q.hct - 1) / q.hct;   // equal chunks
-  q.hct = ((HT + nc - 1) / nc + 1) / 2 * 2;
+// LDS holds for a workgroup's share of the rows (parts) and samples
+void shape_rows(const MultiProb& q, MultiRows& w) {
+  int HT = (tiles64(q.M) + w.parts - 1) / w.parts * 4;
+  if (HT > (q.M + 16) / 16) HT = (q.M + 16) / 16;
+  w.zb = w.samples;
+  if (w.zb > kZs) w.zb = kZs;
+  w.hct = (HT + 1) / 2 * 2;
+  while (w.zb > kZb && lds_bytes(q, w.hct < 8 ? w.hct : 8, w.zb) > kCgLds) w.zb -= 16;
+  while (w.hct > 2 && lds_bytes(q, w.hct, w.zb) > kCgLds) w.hct -= 2;
+  const int nc = (HT + w.hct - 1) / w.hct;   // equal chunks
+  w.hct = ((HT + nc - 1) / nc + 1) / 2 * 2;
 }
 
 // First blocks of every launch, and the workgroups of the cooperative one:
@@ -969,12 +1028,29 @@ void multi_layout(MultiProb* probs, int n, MultiBatch& mb) {
     q.nt = nt;
     cost[at] = c;
   }
+  // the launch of the row weights: 128 samples a workgroup, where that leaves
+  // CUs without one shares of the rows, then fewer samples
+  long items = 0;
+  for (int i = 0; i < n; i++) items += (probs[i].B + kZb - 1) / kZb;
+  const int want = items < cus ? (int)((cus + items - 1) / items) : 1;
   int prep = 0, z = 0, g = 0, vec = 0, apply = 0, cg = 0;
+  mb.shared = 0;
   for (int i = 0; i < n; i++) {
     MultiProb& q = probs[i];
-    shape_rows(q);
-    const size_t b = lds_bytes(q, q.hct, q.zb);
-    if (b > lds) lds = b;
+    const int T = tiles64(q.M);
+    q.coop.parts = row_parts(q, q.nb);
+    if (q.coop.parts > 1) mb.shared = 1;
+    const int shares = q.nb / q.coop.parts;
+    q.coop.samples = ((q.B + 15) / 16 + shares - 1) / shares * 16;
+    q.solo.parts = want < T ? want : T;
+    q.solo.samples = kZb;
+    while (q.solo.samples > 32 && q.solo.parts * kZb < want * q.solo.samples) q.solo.samples /= 2;
+    shape_rows(q, q.coop);
+    shape_rows(q, q.solo);
+    for (const MultiRows* w : {&q.coop, &q.solo}) {
+      const size_t b = lds_bytes(q, w->hct, w->zb);
+      if (b > lds) lds = b;
+    }
     q.blk_prep = prep;
     q.blk_z = z;
     q.blk_g = g;
@@ -982,7 +1058,7 @@ void multi_layout(MultiProb* probs, int n, MultiBatch& mb) {
     q.blk_apply = apply;
     q.blk_cg = cg;
     prep += (q.B + 63) / 64;
-    z += (q.B + kZb - 1) / kZb;
+    z += (q.B + q.solo.samples - 1) / q.solo.samples * q.solo.parts;
     g += tile_units(q, q.nt);
     vec += ((q.nvec + 1) / 2 + kPairs - 1) / kPairs;
     apply += q.nvec;
@@ -1051,19 +1127,20 @@ int launch_multi_cg_persist(const MultiBatch& mb, int iters, hipStream_t st, int
     fprintf(stderr, "nqs_hip: more problems than CUs for the persistent CG launch\n");
     return -1;
   }
-  static bool set = false;
-  if (!set) {
-    NQS_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k_mb_cg),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)kCgLds));
-    set = true;
+  const void* kernel = mb.shared ? reinterpret_cast<const void*>(k_mb_cg<true>)
+                                 : reinterpret_cast<const void*>(k_mb_cg<false>);
+  static bool set[2] = {false, false};
+  if (!set[mb.shared ? 1 : 0]) {
+    NQS_HIP_CHECK(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kCgLds));
+    set[mb.shared ? 1 : 0] = true;
   }
   MultiBatch a = mb;
   void* args[] = {&a, &iters, &matvec_only};
   KScope ks("multi_cg", st);
   // a grid of whole XCD rounds; the workgroups past the last problem return
   const unsigned grid = (unsigned)(mb.nblk_cg + 7) / 8 * 8;
-  const hipError_t e = hipLaunchCooperativeKernel(reinterpret_cast<const void*>(k_mb_cg), dim3(grid),
-                                                  dim3(CT), args, (unsigned)mb.lds, st);
+  const hipError_t e = hipLaunchCooperativeKernel(kernel, dim3(grid), dim3(CT), args,
+                                                  (unsigned)mb.lds, st);
   count_launch();
   if (e != hipSuccess) {
     (void)hipGetLastError();

@@ -536,6 +536,12 @@ int launch_cg_rest(CGScalars* sc, double* x, double* r, double* p, const double*
 // two small GEMMs through the spins and t instead of two passes over O.
 constexpr int kMultiVecBlock = 256;      // elements of a slice of the vectors
 constexpr int kMultiMaxPart = 512;       // slices per problem
+// Row weights: shares of the 64-row tiles of p (parts: past 1 a tile's weights
+// are kept apart and added where they are read), samples of a workgroup (of the
+// launch), 16-row tiles of a chunk of p, samples of a pass over it
+struct MultiRows {
+  int parts = 1, samples = 16, hct = 2, zb = 16;
+};
 struct MultiProb {
   int B = 0, N = 0, M = 0, nsplit = 1, max_it = 0, C = 0;
   double eps = 0.0, tol = 0.0, lr = 0.0;
@@ -547,7 +553,7 @@ struct MultiProb {
   unsigned* bits = nullptr;      // [B][multi_words(N)] spin words (bit set: s = -1)
   double* tT = nullptr;          // [M][B]
   double* tA = nullptr;          // multi_ta_elems: [t, 1] by MFMA operands
-  double* u = nullptr;           // [B] row weights O p
+  double* u = nullptr;           // [multi_parts(M)][B] row weights O p (parts 1: the first)
   double *g = nullptr;           // O^T u, padded vector
   double *x = nullptr, *r = nullptr, *p = nullptr, *Ap = nullptr, *Om = nullptr;  // padded vectors
   double* part = nullptr;        // [4][kMultiMaxPart] partial sums of the slices
@@ -560,9 +566,11 @@ struct MultiProb {
   const int* range_flag = nullptr;  // the ansatz tables' range verdict (nonzero: refused)
   // set by multi_shape: samples per slot, spin words, LDS row stride, slices
   int chunk = 16, nw = 1, si = 2, nvec = 1;
-  // set by multi_layout: workgroups in the cooperative launch, site tiles of
-  // a wave in O^T u, hidden tiles of a chunk of p, samples of a pass over it
-  int nb = 1, nt = 1, hct = 2, zb = 16;
+  // set by multi_layout: workgroups in the cooperative launch, site tiles of a
+  // wave in O^T u; the row weights' work in the cooperative launch and in a
+  // launch of its own
+  int nb = 1, nt = 1;
+  MultiRows coop, solo;
   // first block of this problem in each launch
   int blk_prep = 0, blk_z = 0, blk_g = 0, blk_vec = 0, blk_apply = 0, blk_cg = 0;
 };
@@ -570,10 +578,12 @@ struct MultiBatch {
   int n = 0;
   const MultiProb* probs = nullptr;   // device copy
   int nblk_prep = 0, nblk_z = 0, nblk_g = 0, nblk_vec = 0, nblk_apply = 0, nblk_cg = 0;
+  int shared = 0;                     // a problem's coop.parts is past 1
   int polls = 1 << 24;                // looks at a meeting's counter before it is given up
   size_t lds = 0;
 };
 int multi_words(int N);
+int multi_parts(int M);   // 64-row tiles
 size_t multi_ta_elems(int B, int M);
 void multi_shape(MultiProb& q, int nsplit);   // B, N, M set
 // fills the problems' first-block offsets of every launch and the totals

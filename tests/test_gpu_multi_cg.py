@@ -145,3 +145,66 @@ def test_workgroups_that_do_not_meet(hip, monkeypatch, capfd):
     for (gi, gp), (ri, rp) in zip(*out):
         assert gi == ri
         assert all(np.array_equal(g, q) for g, q in zip(gp, rp))
+
+
+@pytest.mark.parametrize("N,M,B", [(130, 130, 33), (64, 260, 500), (255, 65, 129), (20, 1000, 64), (128, 512, 16),
+                                   (200, 100, 1300)])
+def test_shared_rows_equal_one_share(hip, monkeypatch, N, M, B):
+    """Few samples of many parameters share the rows of p over workgroups, in the
+    cooperative launch and in the launch sequence: the bits of a batch that leaves
+    each problem too few workgroups for that (256 problems; others beside it)."""
+    print("shared rows:", N, M, B, flush=True)
+    monkeypatch.setenv("NQS_HIP_MULTI_SPLIT", "64")
+    r = scenarios.Runner(hip, "nqs_")
+    out = []
+    for on, beside in ((1, 0), (0, 0), (0, 300)):
+        probs = [_problem(hip, r, N, M, B, 16, 6, 9)]
+        probs += [_problem(hip, r, 4, 3, 128, 16, 6, 20 + i) for i in range(beside)]
+        n = len(probs)
+        cfgs = (type(probs[0]["cfg"]) * n)(*[p["cfg"] for p in probs])
+        m = hip.nqs_hip_multi_create(n, cfgs, (ctypes.c_int * n)(*[p["N"] for p in probs]),
+                                     (ctypes.c_int * n)(*[1] * n),
+                                     (ctypes.c_void_p * n)(*[p["a"] for p in probs]),
+                                     (ctypes.c_void_p * n)(*[p["s"] for p in probs]))
+        assert m
+        assert hip.nqs_hip_multi_use_persistent(m, on) == 0
+        info = (SrInfo * n)()
+        for _ in range(2):
+            assert hip.nqs_hip_multi_step(m, info) == 0
+        assert hip.nqs_hip_multi_sync(m) == 0
+        out.append((info[0].as_dict(), r.params(probs[0]["a"])))
+        hip.nqs_hip_multi_free(m)
+        _free(hip, probs)
+    for i, p in out[1:]:
+        assert i == out[0][0]
+        assert np.array_equal(p, out[0][1])
+
+
+@pytest.mark.parametrize("on,tag,part", [(1, b"multi_cg", 0.47), (0, b"multi_gemm_z", 0.75)])
+def test_few_samples_take_less(hip, monkeypatch, on, tag, part):
+    """66049 parameters, an eighth of the samples: a third of an iteration's time
+    in the cooperative launch, half of the row weights' as a launch (0.61 and
+    0.98 where every workgroup went over all parameters for 16 samples)."""
+    monkeypatch.setenv("NQS_HIP_MULTI_SPLIT", "64")
+    r, us = scenarios.Runner(hip, "nqs_"), []
+    for B in (512, 4096):
+        p = _problem(hip, r, 256, 256, B, 256, 20, 3)
+        p["cfg"].sr_cg_tol = 0.0
+        m = hip.nqs_hip_multi_create(1, ctypes.byref(p["cfg"]), (ctypes.c_int * 1)(256), (ctypes.c_int * 1)(1),
+                                     (ctypes.c_void_p * 1)(p["a"]), (ctypes.c_void_p * 1)(p["s"]))
+        assert m
+        assert hip.nqs_hip_multi_use_persistent(m, on) == 0
+        hip.nqs_hip_multi_use_graph(m, 0)
+        info, best = (SrInfo * 1)(), 1e9
+        for _ in range(4):
+            count, ms = ctypes.c_longlong(), ctypes.c_double()
+            hip.nqs_hip_kernel_timing(tag)
+            assert hip.nqs_hip_multi_step(m, info) == 0
+            assert hip.nqs_hip_kernel_stats(tag, ctypes.byref(count), ctypes.byref(ms)) == 0
+            hip.nqs_hip_kernel_timing(None)
+            best = min(best, 1e3 * ms.value / info[0].cg_iterations)
+        us.append(best)
+        hip.nqs_hip_multi_free(m)
+        _free(hip, [p])
+    print("us an iteration:", us, flush=True)
+    assert us[0] < part * us[1], us
