@@ -3567,8 +3567,23 @@ void tridiag_vec(const double* d, const double* e, int K, double lam, double* z)
 
 // the reference's deterministic start vector (src/mps/lanczos.c:160-176):
 // xorshift64 from seed ^ dim, element i = (x_i >> 11) / 2^53 - 1/2; made on
-// the device in runs, each from its own power of the generator's matrix
+// the device in runs, each from its own power of the generator's matrix, and on
+// the host up to 4096 elements, which is less than making the powers (8 states:
+// 9 us of a call of 195)
 int ed_seed_vector(double* d_v, long dim, unsigned long long seed) {
+  if (dim <= 4096) {
+    double h[4096];
+    unsigned long long x = seed ^ (unsigned long long)dim;
+    for (long i = 0; i < dim; i++) {
+      x ^= x << 13;
+      x ^= x >> 7;
+      x ^= x << 17;
+      h[i] = (double)(x >> 11) / 9007199254740992.0 - 0.5;
+    }
+    CK(hipMemcpyAsync(d_v, h, sizeof(double) * dim, hipMemcpyHostToDevice, g_stream));
+    CK(hipStreamSynchronize(g_stream));
+    return 0;
+  }
   std::vector<unsigned long long> jump;
   int nj = 0;
   for (; nj < 32 && (1L << nj) < dim; nj++) {
@@ -4245,7 +4260,12 @@ int lean_lanczos(const EdHam& H, const EdProj& P, int N, int max_iters, double t
   if (max_iters > dim) max_iters = (int)dim;
   std::vector<std::vector<int>> perm;
   std::vector<double> chi;
-  if (ed_sector_applies(H, P, N, perm, chi)) {
+  // the sector's set-up takes as long as a few steps on the full basis: us of a
+  // call in the sector / on the full basis, 12 sites 4 steps 349 / 346, 5 steps
+  // 366 / 405; 18 sites 551 / 519, 523 / 593; 21 sites 8 steps 2000 / 1770, 10 steps
+  // 2130 / 2140; 24 sites 1 step 3410 / 4740
+  const int few = N <= 18 ? 4 : N <= 21 ? 9 : 0;
+  if (max_iters > few && ed_sector_applies(H, P, N, perm, chi)) {
     // NQS_HIP_ED_SECTOR_BYTES=n: the sector takes n bytes of device memory at most
     const char* cap = getenv("NQS_HIP_ED_SECTOR_BYTES");
     EdSector S;

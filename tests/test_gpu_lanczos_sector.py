@@ -149,3 +149,24 @@ def test_sector_without_memory(hip, monkeypatch, capfd, cap):
     assert capfd.readouterr().err.count("full basis") == 1
     assert np.abs(_project(ops, N, vec) - vec).max() < 1e-12
     assert np.linalg.norm(_apply(bonds, N, vec) - val.value * vec) < 1e-5
+
+
+@pytest.mark.parametrize("Lx,Ly,iters,sector", [(2, 1, 4, False), (2, 1, 5, True), (2, 3, 4, False),
+                                                (2, 3, 5, True), (7, 1, 9, False), (7, 1, 10, True),
+                                                (4, 2, 1, True)])
+def test_few_steps_on_the_full_basis(hip, Lx, Ly, iters, sector):
+    """Steps that take less than setting the sector up (the orbits) stay on the
+    full basis."""
+    ops = _translations(Lx, Ly, 1, 1)
+    perm = np.ascontiguousarray([p for p, _ in ops], dtype=np.int32)
+    chi = np.array([c for _, c in ops])
+    val, res = ctypes.c_double(), LanczosResult()
+    count, ms = ctypes.c_longlong(), ctypes.c_double()
+    hip.nqs_hip_kernel_timing(b"ed_orbits")
+    assert hip.nqs_lanczos_e0_kagome_heisenberg_projected_lean(
+        Lx, Ly, 1.0, 1, ptr(perm), ptr(chi), len(ops), iters, 0.0, ctypes.byref(val), ctypes.byref(res)) == 0
+    assert hip.nqs_hip_kernel_stats(b"ed_orbits", ctypes.byref(count), ctypes.byref(ms)) == 0
+    hip.nqs_hip_kernel_timing(None)
+    assert (count.value > 0) == sector
+    if 3 * Lx * Ly <= 12:
+        assert abs(val.value - _lean(_bonds(Lx, Ly, 1), ops, 3 * Lx * Ly, iters)) < 1e-11
