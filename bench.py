@@ -195,27 +195,33 @@ def optimise(lib, w, st, budget):
     return out
 
 
-# kernel symbol (as rocprofv3 names it) behind each timing tag
+# kernel symbol (as rocprofv3 names it) behind each timing tag; the batched CG's
+# tags are phases of one kernel, whose counters are averages over unlike launches
 SYMBOL = {"gemm_potrf": "nqs::k_gemm_big<1>", "gemm_chain": "nqs::k_gemm_lat",
-          "multi_gemm_g": "nqs::(anonymous namespace)::k_mb_phase",
-          "multi_gemm_z": "nqs::(anonymous namespace)::k_mb_phase",
-          "multi_vec": "nqs::(anonymous namespace)::k_mb_phase",
+          "multi_gemm_g": "nqs::(anonymous namespace)::k_mb_phase, phase G",
+          "multi_gemm_z": "nqs::(anonymous namespace)::k_mb_phase, phase Z",
+          "multi_vec": "nqs::(anonymous namespace)::k_mb_phase, vector phases",
           "gemm": "nqs::k_gemm_big<0>",
-          "potrf_panel": "nqs::k_panel2",
-          "eloc": "nqs::k_eloc_terms<double>", "gen_O": "nqs::k_gen_O<double>",
+          "potrf_panel": "nqs::k_panel2", "gen_O": "nqs::k_gen_O<double>",
           "colsum": "nqs::k_colsum_partial", "mh": "nqs::k_mh<double, true, 64, 4>",
           "trsv": "nqs::k_sbsv_fwd", "gram_x3": "nqs::k_gemm_x3"}
 
 
-def traffic_bytes(workload, tag):
-    """HBM bytes per dispatch of the kernel behind `tag`, from the committed
+def symbol(tag, w, precision):
+    if tag != "eloc":
+        return SYMBOL.get(tag)
+    kernel = "k_eloc_terms" if w["kind"] == 6 else "k_eloc_slots"
+    return f"nqs::{kernel}<{'double' if precision == 'fp64' else 'float'}>"
+
+
+def traffic_bytes(workload, sym):
+    """HBM bytes per dispatch of the kernel `sym`, from the committed
     rocprofv3 --pmc summary of this workload (counter values scaled by the
     copy-probe calibration), or None."""
     path = os.path.join(ROOT, "profiles", f"{workload}_hbm_traffic.json")
     if not os.path.exists(path):
         return None
-    d = json.load(open(path)).get("bytes_per_dispatch", {})
-    v = d.get(SYMBOL.get(tag, ""))
+    v = json.load(open(path)).get("bytes_per_dispatch", {}).get(sym or "")
     return None if v is None else v["fetch"] + v["write"]
 
 
@@ -410,6 +416,7 @@ def gpu_run(args, w, move=None, budget=0):
         achieved, peak, runit = work / (avg_ms * 1e-3) / 1e12, pk / 1e12, "TFLOP/s"
     else:
         achieved, peak, runit = work / (avg_ms * 1e-3) / 1e9, PEAK_HBM / 1e9, "GB/s"
+    sym = symbol(dom, w, args.precision)
     res = dict(
         move=mname, ess_per_s=ess / sample_s if sample_s else ess / elapsed,
         ess_per_s_iteration=ess / elapsed,
@@ -418,8 +425,8 @@ def gpu_run(args, w, move=None, budget=0):
         samples_per_chain=int(series.shape[1]),
         energies=energies, acceptance=infos[-1]["acceptance_ratio"],
         stage_ms=np.mean(stages, axis=0).tolist() if stages else None,
-        roofline=dict(kernel=dom, symbol=SYMBOL.get(dom), bound=bound, achieved=achieved, peak=peak,
-                      unit=runit, frac=achieved / peak, traffic=traffic_bytes(args.workload, dom),
+        roofline=dict(kernel=dom, symbol=sym, bound=bound, achieved=achieved, peak=peak,
+                      unit=runit, frac=achieved / peak, traffic=traffic_bytes(args.workload, sym),
                       launches=c.value, avg_ms=avg_ms,
                       work_per_launch=work, work_unit=unit,
                       **({"mfma_products_per_flop": 3, "mfma_util": 3 * achieved / peak}
@@ -946,7 +953,7 @@ def main_multi(args, w):
         "data": "synthetic (random-init parameters N(0,0.01), chains started at random states)",
         "config": {"workload": args.workload + ": " + w["desc"], "instances": len(gpu["inst"]),
                    "samples_per_instance": w["chains"] * w["per_chain"], "method": "cg",
-                   "split_target": gpu["chosen"], "cg_launch": "launch sequence in the graph"},
+                   "split_target": gpu["chosen"], "cg_launch": "one cooperative launch"},
         "sr_iter_ms": gpu["ms_per_step"],
         "sample_ms": gpu["sample_ms"],
         "ess_per_s_iteration": gpu["ess_per_s_iteration"],
