@@ -202,7 +202,8 @@ int nqs_hip_sampler_learned_stats(const nqs_sampler_t *s, double *acceptance,
  * or one launch per phase and iteration (off); same results bit for bit.
  * Without this call or NQS_HIP_MULTI_PERSIST=0/1 at creation the cooperative
  * launch runs (up to one problem per CU).  A device that refuses the
- * cooperative launch gets the launch sequence.
+ * cooperative launch gets the launch sequence, and so does a batch whose
+ * workgroups did not meet in it (that step's CG is made again).
  * last_energies: the local energies of problem i's last batch, sample
  * r*C + c in slot r*C + c (chain c, round r); returns the count. */
 typedef struct nqs_hip_multi nqs_hip_multi_t;

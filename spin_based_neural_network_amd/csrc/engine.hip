@@ -4055,6 +4055,7 @@ bool ed_sector_applies(const EdHam& H, const EdProj& P, int N, std::vector<std::
   return true;
 }
 
+// the start vector's projection at the representatives; its squared norm
 double ed_sector_start(EdSector& S, long dim, unsigned long long seed) {
   if (ed_seed_vector(S.big.b.as<double>(), dim, seed) ||
       nqs::launch_eds_restrict(S.y, S.reps.b.as<unsigned>(), S.R, S.big.b.as<double>(),
@@ -4987,9 +4988,9 @@ struct nqs_hip_multi {
   long long steps_done = 0;
   int tuned = 0, use_graph = 1;
   // the CG iterations in one cooperative launch, the captured graph then
-  // holding the step up to the CG start: chosen by the first step's
-  // autotuning against the launch sequence, unless NQS_HIP_MULTI_PERSIST at
-  // creation or nqs_hip_multi_use_persistent chose (persist_set)
+  // holding the step up to the CG start: the default where the batch has a CU
+  // for every problem, unless NQS_HIP_MULTI_PERSIST at creation or
+  // nqs_hip_multi_use_persistent chose (persist_set)
   int persist = 0, persist_set = 0;
   // Metropolis jobs of all problems, grouped by kernel variant:
   // (variant, first job, jobs, blocks)

@@ -530,7 +530,7 @@ __global__ __launch_bounds__(256) void k_eloc_terms(ModelView<R> m, HamDev H,
 // weights once or twice.
 // What bounds it: vector issue, two FP64 instructions a factor and 4 / GS
 // selects of 32 bits (73 % of the issue cycles).  100 sites, 400 pairs, 800
-// hidden units, 16384 samples: 823 us, 1945 as k_eloc_terms had them (12
+// hidden units, 16384 samples: 853 us (815 to 882), 1945 as k_eloc_terms had them (12
 // instructions a factor).
 // ---------------------------------------------------------------------------
 template <typename R>
@@ -807,8 +807,8 @@ static void slots_go(const ModelView<R>& m, const HamDev& h, const int* spins, i
 }
 
 // Two samples a lane where that leaves two workgroups for every CU (100 sites,
-// 16384 samples: 823 us; four samples with half the waves 1010, workgroups of
-// eight waves 870)
+// 16384 samples, one run of each: 823 us; four samples with half the waves 1010,
+// workgroups of eight waves 870)
 template <typename R>
 static void slots_any(const ModelView<R>& m, const HamDev& h, const int* spins, int B, const R* t_re,
                       const R* q_re, const R* E, const double* bound, const double* cst, double* res_r,

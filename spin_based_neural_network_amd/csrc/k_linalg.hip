@@ -1845,8 +1845,6 @@ constexpr int SB = 256;
 static size_t sb_count(int n) { return (size_t)((n + SB - 1) / SB); }
 size_t potrf_linv_elems(int n) { return l21_offset(n) + l21_elems(n) + 4 * sb_count(n) * SB * SB; }
 
-// acc (+)= sign * A B over 64 x 64 LDS tiles; the thread owns rows
-// rb .. rb + 3 and columns cb .. cb + 3
 // acc (16 rows of this wave x 64 columns) += sign A B, both 64 x 64 in LDS:
 // each element one chain over k, as MFMA accumulates it
 __device__ inline void tile_mfma(v4d (&acc)[4], const double (*A)[LD], const double (*Bm)[LD],
