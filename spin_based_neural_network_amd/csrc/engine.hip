@@ -482,13 +482,14 @@ int ham_upload(const nqs::HamHost& H, const AmpSource& src, DBuf& store, DBuf& s
 // grouped: with the terms' groups (the local energies of real RBMs)
 int ham_device(const nqs_config_t* cfg, int Lx, int Ly, int per, const AmpSource& src,
                nqs::HamDev& out, bool grouped = false) {
-  if (same_ham(cfg, Lx, Ly, per, src) &&
-      (!grouped || g_ham.dev.n_oct || g_ham.dev.n_flip + g_ham.dev.n_pair == 0)) {
+  const bool same = same_ham(cfg, Lx, Ly, per, src);
+  if (same && (!grouped || g_ham.dev.n_oct || g_ham.dev.n_flip + g_ham.dev.n_pair == 0)) {
     out = g_ham.dev;
     return 0;
   }
   g_ham.valid = 0;
-  if (nqs::build_hamiltonian(cfg, Lx, Ly, per, g_ham.host) != 0) {
+  // (same: only the groups are missing, the host's terms stay)
+  if (!same && nqs::build_hamiltonian(cfg, Lx, Ly, per, g_ham.host) != 0) {
     fprintf(stderr, "nqs_hip: Hamiltonian kind %d is not provided by this library\n",
             (int)cfg->hamiltonian);
     return -1;
