@@ -555,6 +555,7 @@ __global__ __launch_bounds__(512) void k_slot_tables(ModelView<R> m, HamDev H, i
   __shared__ double part[8][8];
   __shared__ int pex[8][8];
   const int o = blockIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63, M = m.M;
+  const int nt = blockDim.x;
   double c[8];
   int ce[8];
 #pragma unroll
@@ -562,7 +563,7 @@ __global__ __launch_bounds__(512) void k_slot_tables(ModelView<R> m, HamDev H, i
     c[j] = 1.0;
     ce[j] = 0;
   }
-  for (int h = threadIdx.x; h < ((Mp + 511) & ~511); h += 512) {
+  for (int h = threadIdx.x; h < (Mp + nt - 1) / nt * nt; h += nt) {
     double big = 0.0, d[8];
 #pragma unroll
     for (int j = 0; j < 8; j++) {
@@ -600,7 +601,7 @@ __global__ __launch_bounds__(512) void k_slot_tables(ModelView<R> m, HamDev H, i
   if (threadIdx.x < 8) {
     double v = 1.0;
     int e = 0, e2;
-    for (int w = 0; w < 8; w++) {
+    for (int w = 0; w < nt >> 6; w++) {
       v *= part[threadIdx.x][w];
       e += pex[threadIdx.x][w];
     }
@@ -740,6 +741,12 @@ __global__ __launch_bounds__(64 * kSlotWaves) void k_eloc_slots(
   }
 }
 
+// Terms and diagonal parts up to which a thread's own loads take less than 128
+// fetched together: us at 64 / 16384 samples, real RBM, 8 of them 2.2 / 4.3 (7.6 /
+// 9.2 together), 36 5.2 / 9.6 (7.1 / 8.8), 64 9.2 / 18 (12.6 / 12.0), 80 12.6 / 18
+// (8.2 / 9.1); complex, 36 6.6 / 9.4 (9.7 / 9.5)
+constexpr int kFewTerms = 36;
+
 // E_loc(b) = diagonal part + sum over terms in order of res[t][b] (res_i null:
 // real amplitudes).  Four waves fetch 128 terms of 64 samples at a time, the
 // first adds them: one wave's own loads took 269 us for 400 terms and 16384
@@ -783,6 +790,29 @@ __global__ __launch_bounds__(256) void k_eloc_terms_sum(HamDev H, const int* __r
     return H.diag_c[d] * (double)(sp[H.diag_a[d]] * sp[H.diag_b[d]]);
   });
   if (wave != 0 || b >= B) return;
+  e_re[b] = diag + orr;
+  if (e_im) e_im[b] = oi;
+}
+
+// the same for few terms: a thread's own loads
+__global__ __launch_bounds__(256) void k_eloc_terms_sum_few(HamDev H, const int* __restrict__ spins,
+                                                            int B, int N,
+                                                            const double* __restrict__ res_r,
+                                                            const double* __restrict__ res_i,
+                                                            double* __restrict__ e_re,
+                                                            double* __restrict__ e_im) {
+  const int b = blockIdx.x * blockDim.x + threadIdx.x;
+  if (b >= B) return;
+  const int* s = spins + (size_t)b * N;
+  double diag = 0.0;
+  for (int d = 0; d < H.n_diag; d++)
+    diag += H.diag_c[d] * (double)(s[H.diag_a[d]] * s[H.diag_b[d]]);
+  const int T = H.n_flip + H.n_pair;
+  double orr = 0.0, oi = 0.0;
+  for (int t = 0; t < T; t++) {
+    orr += res_r[(size_t)t * B + b];
+    if (res_i) oi += res_i[(size_t)t * B + b];
+  }
   e_re[b] = diag + orr;
   if (e_im) e_im[b] = oi;
 }
@@ -864,7 +894,8 @@ static int eloc_terms_go(const ModelView<R>& m, const HamDev& h, const int* spin
     R* E = (R*)p;
     double* bound = (double*)(p + ((sizeof(R) * h.n_oct * Mp * 8 + 255) & ~(size_t)255));
     double* cst = bound + (size_t)h.n_oct * (Mp / SlotRange<R>::RG);
-    hipLaunchKernelGGL((k_slot_tables<R>), dim3(h.n_oct), dim3(512), 0, st, m, h, Mp, E, bound, cst);
+    const int nt = Mp < 64 ? 64 : Mp < 512 ? (Mp + 63) / 64 * 64 : 512;
+    hipLaunchKernelGGL((k_slot_tables<R>), dim3(h.n_oct), dim3(nt), 0, st, m, h, Mp, E, bound, cst);
     count_launch();
     slots_any<R>(m, h, spins, B, t_re, q_re, E, bound, cst, res_r, res_out ? res_i : nullptr, st);
     count_launch();
@@ -874,8 +905,12 @@ static int eloc_terms_go(const ModelView<R>& m, const HamDev& h, const int* spin
     res_out[1] = res_i;
   }
   if (e_re) {
-    hipLaunchKernelGGL(k_eloc_terms_sum, dim3((B + 63) / 64), dim3(256), 0, st, h, spins, B,
-                       m.N, res_r, CPLX ? res_i : nullptr, e_re, e_im);
+    if (T + h.n_diag <= kFewTerms)
+      hipLaunchKernelGGL(k_eloc_terms_sum_few, dim3((B + 255) / 256), dim3(256), 0, st, h, spins, B,
+                         m.N, res_r, CPLX ? res_i : nullptr, e_re, e_im);
+    else
+      hipLaunchKernelGGL(k_eloc_terms_sum, dim3((B + 63) / 64), dim3(256), 0, st, h, spins, B,
+                         m.N, res_r, CPLX ? res_i : nullptr, e_re, e_im);
     count_launch();
   }
   NQS_HIP_CHECK(hipGetLastError());
